@@ -33,7 +33,7 @@ HIP_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
-LIB_SOURCES = ["pfdtd_kernels.hip", "pfdtd_fused.hip", "pfdtd_capi.hip", "pfdtd_pool.hip",
+LIB_SOURCES = ["pfdtd_kernels.hip", "pfdtd_fused.hip", "pfdtd_sweep.hip", "pfdtd_capi.hip", "pfdtd_pool.hip",
                "pfdtd_voxel.hip", "pfdtd_probe.hip"]
 
 

@@ -79,6 +79,17 @@ struct pfdtd_ctx {
   uint32_t *d_air_rows3 = nullptr;   // the same for the three-level sweep's tiles
   bool air3_ok = false;              // d_air_rows3 built for the current domain (or no room)
   bool pm_ok = false;
+  // several-level sweep: entry plane and air bits of the current domain and plan, and the
+  // events (sources and receivers by wave tile and slice)
+  uint16_t *d_entry = nullptr;
+  size_t entry_cap = 0;
+  bool entry_ok = false;
+  uint64_t *d_row_bits = nullptr;
+  size_t air_cap = 0;
+  int32_t *d_ev_ptr = nullptr, *d_events = nullptr;
+  size_t ev_ptr_cap = 0, ev_cap = 0;
+  int sweep_key[4] = {0, 0, 0, 0};  // tile shape the air bits and events were built for
+  bool events_ok = false;
   int64_t dom_cap = 0;  // voxels the position/material buffers hold
   bool has_domain = false;
   DomainScan scan{};
@@ -371,6 +382,8 @@ int alloc_domain(pfdtd_ctx *c, int64_t X, int64_t Y, int64_t Z) {
   }
   c->pm_ok = false;
   c->air3_ok = false;
+  c->entry_ok = false;
+  c->events_ok = false;
   dfree(c->d_air_rows);  // sized by the grid's shape, not only its voxel count
   dfree(c->d_air_rows_p);
   dfree(c->d_air_rows3);
@@ -725,6 +738,175 @@ UpdateGeom plan_single(const pfdtd_ctx *c) {
   return plan_update_batch((int)c->X, (int)c->Y, (int)c->Z, ry, zc, lgB);
 }
 
+// ---- several-level sweep -------------------------------------------------------------------
+
+// Grows a device buffer to `need` elements.
+template <typename T>
+hipError_t grow(T *&p, size_t &cap, size_t need) {
+  if (need <= cap) return hipSuccess;
+  dfree(p);
+  cap = 0;
+  const hipError_t e = hipMalloc((void **)&p, sizeof(T) * need);
+  if (e == hipSuccess) cap = need;
+  return e;
+}
+
+// Sources and receivers of the sweep's wave tiles: a source belongs to every tile whose window
+// covers it (the levels below the last are computed there too), a receiver to the tile that owns
+// it; per tile by slice, the receivers of a slice before its sources, each in index order.
+int build_sweep_events(pfdtd_ctx *c, const SweepPlan &p) {
+  const int slots = batch_slots(c);
+  const int nty = p.nby * p.wy, ntile = nty * p.nbx;
+  struct Ev {
+    int tile, z, x, y, id;
+  };
+  std::vector<Ev> ev;
+  auto add = [&](const int32_t *q, int slot, int id, int bx, int by, int row) {
+    ev.push_back(Ev{slot * ntile + (by * p.wy + row / p.ty) * p.nbx + bx, q[2], q[0], q[1], id});
+  };
+  for (int r = 0; r < c->n_rec; ++r) {
+    const int32_t *q = &c->rec_xyz[3 * r];
+    if (lin_idx(c, q) < 0) continue;
+    const int bx = q[0] / p.ox, by = q[1] / p.oy;
+    add(q, c->rec_slot[r], (int)((uint32_t)r | 0x80000000u), bx, by, q[1] - by * p.oy + p.lm);
+  }
+  for (int s = 0; s < c->n_src; ++s) {
+    const int32_t *q = &c->src_xyz[3 * s];
+    if (lin_idx(c, q) < 0) continue;
+    for (int by = std::max(0, (q[1] - p.lm) / p.oy - 1); by < p.nby; ++by) {
+      const int row = q[1] - by * p.oy + p.lm;
+      if (row < 0) break;
+      if (row >= p.wy * p.ty) continue;
+      for (int bx = std::max(0, (q[0] - p.hx) / p.ox - 1); bx < p.nbx; ++bx) {
+        const int col = q[0] - bx * p.ox + p.hx;
+        if (col < 0) break;
+        if (col < p.w) add(q, c->src_slot[s], s, bx, by, row);
+      }
+    }
+  }
+  std::stable_sort(ev.begin(), ev.end(), [](const Ev &a, const Ev &b) {
+    return a.tile != b.tile ? a.tile < b.tile : a.z < b.z;
+  });
+  std::vector<int32_t> ptr((size_t)slots * ntile + 1, 0), data(4 * ev.size());
+  for (size_t i = 0; i < ev.size(); ++i) {
+    ++ptr[(size_t)ev[i].tile + 1];
+    data[4 * i] = ev[i].z;
+    data[4 * i + 1] = ev[i].x;
+    data[4 * i + 2] = ev[i].y;
+    data[4 * i + 3] = ev[i].id;
+  }
+  for (size_t i = 1; i < ptr.size(); ++i) ptr[i] += ptr[i - 1];
+  HIP_TRY(grow(c->d_ev_ptr, c->ev_ptr_cap, ptr.size()));
+  HIP_TRY(grow(c->d_events, c->ev_cap, std::max<size_t>(data.size(), 4)));
+  HIP_TRY(hipStreamSynchronize(c->stream));
+  HIP_TRY(hipMemcpy(c->d_ev_ptr, ptr.data(), sizeof(int32_t) * ptr.size(), hipMemcpyHostToDevice));
+  if (!data.empty())
+    HIP_TRY(hipMemcpy(c->d_events, data.data(), sizeof(int32_t) * data.size(), hipMemcpyHostToDevice));
+  return PFDTD_OK;
+}
+
+// Whether the sweep takes this context's runs: the forward scheme, FP32 or FP64 fields, slices
+// below 2^31 bytes and the automatic settings.
+bool sweep_eligible(const pfdtd_ctx *c) {
+  if (c->scheme != 0 || c->levels != 0 || c->fshape != PFDTD_SWEEP_AUTO) return false;
+  if (c->precision != PFDTD_F32 && c->precision != PFDTD_F64) return false;
+  const uint64_t esz = elem_size(c->precision);
+  return fused_eligible(c) && (uint64_t)c->X * (uint64_t)c->Y * esz < (1ull << 31);
+}
+
+// Entry plane, air bits and events for the sweep; *ok is cleared when there is no room for them.
+int ensure_sweep(pfdtd_ctx *c, const SweepPlan &p, bool *ok) {
+  const int ncol = coef_cols(c);
+  const int key[4] = {p.w, p.hx, p.oy, p.ty};
+  const bool same = std::equal(key, key + 4, c->sweep_key);
+  hipError_t e = hipSuccess;
+  if (!c->entry_ok) {
+    e = grow(c->d_entry, c->entry_cap, (size_t)p.pitch * c->Y * c->Z);
+    if (e == hipSuccess)
+      e = launch_pack_entry(c->d_pos, c->d_mat, c->d_entry, (int)c->X, (int)c->Y, (int)c->Z,
+                            p.pitch, ncol, c->stream);
+  }
+  if (e == hipSuccess && (!c->entry_ok || !same)) {
+    e = grow(c->d_row_bits, c->air_cap, 2 * (size_t)p.nbx * p.nby * p.wy * p.words);
+    if (e == hipSuccess)
+      e = launch_row_bits(p, c->d_entry, c->d_row_bits, (int)c->X, (int)c->Y, (int)c->Z, ncol,
+                          c->stream);
+  }
+  if (e == hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    c->entry_ok = false;
+    *ok = false;
+    return PFDTD_OK;
+  }
+  if (e != hipSuccess) return fail(PFDTD_E_HIP, "sweep planes: %s", hipGetErrorString(e));
+  c->entry_ok = true;
+  if (!c->events_ok || !same) {
+    const int rc = build_sweep_events(c, p);
+    if (rc) return rc;
+    c->events_ok = true;
+  }
+  std::copy(key, key + 4, c->sweep_key);
+  return PFDTD_OK;
+}
+
+template <typename S, typename CT, typename C>
+SweepArgs<S, CT, C> sweep_args(const pfdtd_ctx *c, const CT *coef, CT air, C lam2, const C *sig,
+                               int step, int inject_end) {
+  SweepArgs<S, CT, C> a{};
+  a.pm = c->d_entry;
+  a.row_bits = c->d_row_bits;
+  a.ev_ptr = c->d_ev_ptr;
+  a.events = c->d_events;
+  a.A = (const S *)c->d_P;
+  a.B = (const S *)c->d_Pp;
+  a.Cn = (S *)c->d_Pp2;
+  a.Dn = (S *)c->d_P2;
+  a.coef = coef;
+  a.ncol = coef_cols(c);
+  a.air = air;
+  a.air_mask = c->air_uniform && air.inv == 1 && air.omb == 1 ? 0xFFu : 0u;
+  a.air_pm = 6u * (uint32_t)a.ncol * 0x10001u;
+  a.lam2 = lam2;
+  a.src_kind = c->d_src_kind;
+  a.sig = sig;
+  a.n_samples = c->n_samples;
+  a.step = step;
+  a.inject_end = inject_end;
+  a.soft_overwrite = (c->flags & PFDTD_SOFT_OVERWRITE) ? 1 : 0;
+  a.scale = (C)std::ldexp(1.0, c->scale_exp);
+  a.inv_scale = std::ldexp(1.0, -c->scale_exp);
+  a.resp = c->d_resp;
+  a.resp_steps = c->resp_steps;
+  a.X = (int)c->X;
+  a.Y = (int)c->Y;
+  a.Z = (int)c->Z;
+  a.n_slots = batch_slots(c);
+  a.slot_elems = c->N;
+  return a;
+}
+
+// Steps `step` .. `step + levels - 1` in one sweep, gathers and injections included; the new
+// current and past fields are in d_P and d_Pp afterwards.
+hipError_t run_sweep(pfdtd_ctx *c, const SweepPlan &p, int step, int levels, int inject_end) {
+  hipError_t e;
+  if (c->precision == PFDTD_F64)
+    e = launch_sweep_f64(p, sweep_args<double>(c, c->d_coef_d, c->air_d, c->lam2_d, c->d_sig_d,
+                                               step, inject_end), levels, c->stream);
+  else
+    e = launch_sweep_f32(p, sweep_args<float>(c, c->d_coef_f, c->air_f, c->lam2_f, c->d_sig_f,
+                                              step, inject_end), levels, c->stream);
+  if (levels > 1) {
+    std::swap(c->d_P, c->d_P2);
+    std::swap(c->d_Pp, c->d_Pp2);
+  } else {  // one level writes P^{n+1} only: P^n becomes the past field
+    void *spare = c->d_Pp;
+    c->d_Pp = c->d_P;
+    c->d_P = c->d_P2;
+    c->d_P2 = spare;
+  }
+  return e;
+}
+
 int ensure_events(pfdtd_ctx *c, size_t n) {
   while (c->events.size() < n) {
     hipEvent_t e;
@@ -794,6 +976,10 @@ int pfdtd_ctx_destroy(pfdtd_ctx *c) {
   dfree(c->d_air_rows);
   dfree(c->d_air_rows_p);
   dfree(c->d_air_rows3);
+  dfree(c->d_entry);
+  dfree(c->d_row_bits);
+  dfree(c->d_ev_ptr);
+  dfree(c->d_events);
   dfree(c->d_scan);
   dfree(c->d_coef_f);
   dfree(c->d_coef_d);
@@ -1084,6 +1270,7 @@ int pfdtd_set_sources(pfdtd_ctx *c, int n_src, const int32_t *xyz, const int32_t
     if (kind[s] < PFDTD_SRC_HARD || kind[s] > PFDTD_SRC_TRANSPARENT)
       return fail(PFDTD_E_ARG, "source %d: unknown kind %d", s, kind[s]);
   HIP_TRY(hipStreamSynchronize(c->stream));
+  c->events_ok = false;
   dfree(c->d_src_idx);
   dfree(c->d_src_xyz);
   dfree(c->d_src_kind);
@@ -1135,6 +1322,7 @@ int pfdtd_set_receivers(pfdtd_ctx *c, int n_rec, const int32_t *xyz) {
   if (n_rec < 0) return fail(PFDTD_E_ARG, "negative receiver count");
   if (n_rec > 0 && !xyz) return fail(PFDTD_E_ARG, "null receiver array");
   HIP_TRY(hipStreamSynchronize(c->stream));
+  c->events_ok = false;
   dfree(c->d_rec_idx);
   dfree(c->d_rec_xyz);
   dfree(c->d_rec_slot);
@@ -1265,7 +1453,14 @@ int pfdtd_run(pfdtd_ctx *c, int precision, int n_steps, pfdtd_interrupt_cb inter
     HIP_TRY(launch_inject_gather(p_storage(c->precision), c->d_P, ia, c->stream));
   }
 
-  bool fused = fused_eligible(c);
+  bool sweep = !diff && sweep_eligible(c);
+  SweepPlan sp{};
+  if (sweep) {
+    sp = plan_sweep(c->precision, (int)c->X, (int)c->Y, (int)c->Z, c->fzc, batch_slots(c));
+    rc = ensure_sweep(c, sp, &sweep);
+    if (rc) return rc;
+  }
+  bool fused = !sweep && fused_eligible(c);
   rc = ensure_pm(c, &fused);
   if (rc) return rc;
   const FusedGeom fg = plan_fused((int)c->X, (int)c->Y, (int)c->Z, c->fzc, c->precision, false,
@@ -1290,6 +1485,16 @@ int pfdtd_run(pfdtd_ctx *c, int precision, int n_steps, pfdtd_interrupt_cb inter
     int nev = 0;
     for (int k = 0; k < nb;) {
       const int step = done + k;
+      if (sweep) {
+        const int lv = std::min(sp.lm, nb - k);
+        if (c->kernel_timing) HIP_TRY(hipEventRecord(c->events[2 * nev], c->stream));
+        HIP_TRY(run_sweep(c, sp, step, lv, n_steps));
+        if (c->kernel_timing) HIP_TRY(hipEventRecord(c->events[2 * nev + 1], c->stream));
+        ++nev;
+        k += lv;
+        c->upd_launches += lv;
+        continue;
+      }
       // four steps left take two two-level sweeps rather than three levels and a single step
       if (three && k + 3 <= nb && nb - k != 4) {
         if (c->kernel_timing) HIP_TRY(hipEventRecord(c->events[2 * nev], c->stream));
@@ -1428,7 +1633,14 @@ int pfdtd_steps(pfdtd_ctx *c, int first_step, int n_steps) {
     if (n_steps == 0) return PFDTD_OK;
   }
   const UpdateGeom g = plan_single(c);
-  bool fused = fused_eligible(c);
+  bool sweep = sweep_eligible(c);
+  SweepPlan sp{};
+  if (sweep) {
+    sp = plan_sweep(c->precision, (int)c->X, (int)c->Y, (int)c->Z, c->fzc, batch_slots(c));
+    rc = ensure_sweep(c, sp, &sweep);
+    if (rc) return rc;
+  }
+  bool fused = !sweep && fused_eligible(c);
   rc = ensure_pm(c, &fused);
   if (rc) return rc;
   const FusedGeom fg = plan_fused((int)c->X, (int)c->Y, (int)c->Z, c->fzc, c->precision, false,
@@ -1446,6 +1658,12 @@ int pfdtd_steps(pfdtd_ctx *c, int first_step, int n_steps) {
   HIP_TRY(launch_inject_gather(c->precision, c->d_P, inject_args(c, -1, first_step), c->stream));
   for (int k = 0; k < n_steps;) {
     const int step = first_step + k;
+    if (sweep) {
+      const int lv = std::min(sp.lm, n_steps - k);
+      HIP_TRY(run_sweep(c, sp, step, lv, first_step + n_steps));
+      k += lv;
+      continue;
+    }
     if (three && k + 3 <= n_steps && n_steps - k != 4) {
       HIP_TRY(launch_update3(c, fg3, step));
       const int next = k + 3 < n_steps ? step + 3 : -1;
@@ -1656,6 +1874,7 @@ int pfdtd_set_sweep_shape(pfdtd_ctx *c, int shape) {
 
 // Re-derives the device element indices of sources and receivers (grid, batch or slots changed).
 static int refresh_indices(pfdtd_ctx *c) {
+  c->events_ok = false;
   if (c->n_src) {
     std::vector<int64_t> idx(c->n_src);
     for (int s = 0; s < c->n_src; ++s) idx[s] = elem_idx(c, &c->src_xyz[3 * s], c->src_slot[s]);

@@ -240,6 +240,59 @@ hipError_t launch_update3_f16(const FusedGeom &g, const Fused2Args<h16, CoefF, f
 hipError_t launch_update3_bf16(const FusedGeom &g, const Fused2Args<b16, CoefF, float> &a,
                                hipStream_t stream);
 
+// Several-level sweep (pfdtd_sweep.hip): reads P^n (A) and P^{n-1} (B), writes P^{n+L-1} (Cn) and
+// P^{n+L} (Dn) with the sources of steps n+1 .. n+L injected and the receivers of steps
+// n .. n+L-1 gathered on the way.
+template <typename S, typename CT, typename C>
+struct SweepArgs {
+  const uint16_t *pm;  // coefficient entry per voxel, rows of `pitch` elements
+  int pitch;
+  const uint64_t *row_bits;  // per wave tile, two bytes per slice: its rows of plain air, solid rows
+  int air_words;             // words per wave tile
+  const int32_t *ev_ptr;     // per (slot, wave tile): first event, then one past the last
+  const int32_t *events;     // {z, x, y, source index or receiver index | 1 << 31}, by z
+  const S *A;
+  const S *B;
+  S *Cn;
+  S *Dn;
+  const CT *coef;
+  int ncol;
+  CT air;
+  uint32_t air_mask;  // 0xFF; 0 when the air entry needs the table (inv or omb not 1, not uniform)
+  uint32_t air_pm;  // packed entries of two plain air voxels
+  C lam2;
+  const int32_t *src_kind;
+  const C *sig;
+  int n_samples;
+  int step;        // n
+  int inject_end;  // sources are injected for time indices below this
+  int soft_overwrite;
+  C scale;
+  double inv_scale;
+  double *resp;
+  int resp_steps;
+  int X, Y, Z, zc;
+  int nbx, nby, band;
+  int n_slots;
+  int64_t slot_elems;
+};
+
+struct SweepPlan {
+  int nc, ty, wy, lm;    // columns per lane, rows per wave, waves per block, most levels
+  int w, hx, ox, oy;     // window columns, halo columns, owned columns and rows of a block
+  int nbx, nby, zc, band, words, pitch;
+  int64_t blocks;
+};
+SweepPlan plan_sweep(int precision, int X, int Y, int Z, int zc, int slots);
+hipError_t launch_pack_entry(const uint8_t *pos, const uint8_t *mat, uint16_t *pm, int X, int Y,
+                             int Z, int pitch, int ncol, hipStream_t stream);
+hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint64_t *out, int X, int Y,
+                           int Z, int ncol, hipStream_t stream);
+hipError_t launch_sweep_f32(const SweepPlan &p, SweepArgs<float, CoefF, float> a, int levels,
+                            hipStream_t stream);
+hipError_t launch_sweep_f64(const SweepPlan &p, SweepArgs<double, CoefD, double> a, int levels,
+                            hipStream_t stream);
+
 // Receiver gather of time index `gather_step` (skipped when < 0) followed by injection of
 // source samples of time index `inject_step` (skipped when < 0) into the same field.
 struct InjectArgs {

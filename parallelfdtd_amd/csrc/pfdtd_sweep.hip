@@ -1,0 +1,718 @@
+// pfdtd_sweep.hip -- several time levels of the forward update per sweep of the field.
+//
+// One launch reads P^n (A) and P^{n-1} (B) once and writes P^{n+L-1} (Cn) and P^{n+L} (Dn); the L-1
+// levels between never leave the chip. Sources are injected and receivers gathered at every level,
+// the last included, in the reference's order (a level's gather before the next step's injection),
+// and the node arithmetic, sum order and storage rounding are the single step's, so the results are
+// L single steps bit for bit.
+//
+// Tiling. A block of WY waves marches a z-chunk. A wave holds TY rows of a window of 64 NC columns,
+// two slices of every level's rows in registers: at iteration k the rows of level i advance to slice
+// k-i+1 from level i-1's slices k-i, k-i+1 and (just computed) k-i+2, row by row through all levels,
+// and each new row takes the place of the oldest one. x-neighbours come from the lane's other column
+// or a DPP shift; y-neighbours from the wave's other rows or, at its first and last row, from the
+// neighbouring wave's through LDS: every wave publishes the edge rows of its new slices, one barrier
+// per slice, double-buffered. So a block recomputes a halo only at its own border (L rows and HX
+// columns on either side), where a sweep of independent waves recomputes one around every wave: the
+// three-level sweep computes 1.8 nodes and loads 4.5 rows per node-update it keeps, this one 1.5 (L =
+// 5) and 2.2.
+//
+// What bounds it (2048x1536x768 FP32, L = 5): 2.25-2.40 ms per step against 3.73-3.83 for the
+// three-level sweep of independent waves. Its arithmetic alone (no loads, no stores, all air) takes
+// 1.20 ms, the table rows 0.4 more, the loads alone 1.41, the stores alone 1.66: it is bound by the
+// traffic, 19.4 GB written and 1.5 passes of the two fields read per launch. FP64 (L = 4):
+// 1024x768x384 0.70 ms against 1.03. Tiles measured (ms per step, 2048x1536x768 FP32, same box): L = 4
+// 8 rows 2.95, 6 rows 2.96; L = 5 6 rows 2.52, 7 rows (spills) 2.55; L = 6 does not fit LDS. Windows: stores of
+// whole 64-byte lines matter (112 owned columns 2.99, 120 columns 3.26 with L = 4), so HX is 8
+// although five columns would do; 16 (96 owned columns) 3.07.
+//
+// Rows of plain air at every level of an iteration take the air entry as an immediate (nine VALU
+// operations per node); rows with nothing to update at any level are zeros; the others gather
+// every node's table entry from LDS, the gathers of the next level in flight during the last. The
+// choice is made by two bits per row and slice built once per domain. Made once for all rows of an
+// iteration instead, it keeps both the old and the new queue entries live (75 registers more).
+//
+// Loads, stores and masks. Slices are accessed through buffer descriptors: rows and columns past
+// the grid read 0, stores that a lane or row does not own are given an offset past the slice and
+// dropped, so the body has no masked branches. The loads of the next slice are issued as soon as a
+// row has consumed its own, a whole iteration ahead of their use.
+#include "../../include/pfdtd.h"
+#include "pfdtd_device.h"
+
+#include <algorithm>
+#include <type_traits>
+
+namespace pfdtd {
+
+namespace {
+
+__device__ __forceinline__ float sw_next(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x130, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float sw_prev(float v) {
+  return __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), 0x138, 0xF, 0xF, true));
+}
+__device__ __forceinline__ double sw_next(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x130, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x130, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+__device__ __forceinline__ double sw_prev(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), 0x138, 0xF, 0xF, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), 0x138, 0xF, 0xF, true);
+  return __hiloint2double(hi, lo);
+}
+
+// Slice access through a buffer descriptor: out-of-range offsets read 0 and drop stores, so
+// rows and columns past the grid need no clamps and masked stores no branches.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t sw_rsrc(const void *p, uint32_t nbytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)nbytes,
+                                           0x00020000);
+}
+
+// Keeps a value's computation ahead of the select that masks it (a select between it and 0 would
+// otherwise become a lane-masked branch around the computation).
+__device__ __forceinline__ void sw_keep(float &v) { asm("" : "+v"(v)); }
+__device__ __forceinline__ void sw_keep(double &v) { asm("" : "+v"(v)); }
+
+// NC columns of one row held by a lane, and their raw form in the storage type.
+template <typename C, int NC>
+struct Cols {
+  C v[NC];
+};
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
+
+template <typename S, int NC>
+struct Raw;
+template <>
+struct Raw<float, 2> {
+  typedef u32x2 T;
+  static __device__ __forceinline__ T ld(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
+  }
+  static __device__ __forceinline__ Cols<float, 2> up(T t) {
+    return Cols<float, 2>{{__uint_as_float(t.x), __uint_as_float(t.y)}};
+  }
+  static __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, uint32_t off,
+                                            const Cols<float, 2> &c) {
+    u32x2 t;
+    t.x = __float_as_uint(c.v[0]);
+    t.y = __float_as_uint(c.v[1]);
+    __builtin_amdgcn_raw_buffer_store_b64(t, r, (int)off, 0, 0);
+  }
+  static __device__ __forceinline__ void st1(__amdgpu_buffer_rsrc_t r, uint32_t off, float v) {
+    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, (int)off, 0, 0);
+  }
+};
+template <>
+struct Raw<double, 1> {
+  typedef u32x2 T;
+  static __device__ __forceinline__ T ld(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_bit_cast(T, __builtin_amdgcn_raw_buffer_load_b64(r, (int)off, 0, 0));
+  }
+  static __device__ __forceinline__ Cols<double, 1> up(T t) {
+    return Cols<double, 1>{{__hiloint2double((int)t.y, (int)t.x)}};
+  }
+  static __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, uint32_t off,
+                                            const Cols<double, 1> &c) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, c.v[0]), r, (int)off, 0, 0);
+  }
+  static __device__ __forceinline__ void st1(__amdgpu_buffer_rsrc_t r, uint32_t off, double v) {
+    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int)off, 0, 0);
+  }
+};
+template <typename S>
+struct Raw<S, 2> {
+  static_assert(sizeof(S) == 2, "16-bit storage");
+  typedef uint32_t T;
+  static __device__ __forceinline__ T ld(__amdgpu_buffer_rsrc_t r, uint32_t off) {
+    return __builtin_amdgcn_raw_buffer_load_b32(r, (int)off, 0, 0);
+  }
+  static __device__ __forceinline__ Cols<float, 2> up(T t) {
+    return Cols<float, 2>{{Fmt<S>::val(S{(uint16_t)(t & 0xFFFFu)}), Fmt<S>::val(S{(uint16_t)(t >> 16)})}};
+  }
+  static __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, uint32_t off,
+                                            const Cols<float, 2> &c) {
+    const uint32_t t = (uint32_t)Fmt<S>::raw(c.v[0]).bits | ((uint32_t)Fmt<S>::raw(c.v[1]).bits << 16);
+    __builtin_amdgcn_raw_buffer_store_b32(t, r, (int)off, 0, 0);
+  }
+  static __device__ __forceinline__ void st1(__amdgpu_buffer_rsrc_t r, uint32_t off, float v) {
+    __builtin_amdgcn_raw_buffer_store_b16(Fmt<S>::raw(v).bits, r, (int)off, 0, 0);
+  }
+};
+
+// x+1 and x-1 neighbours of column c of a lane's NC columns.
+template <typename C, int NC>
+__device__ __forceinline__ C x_next(const Cols<C, NC> &q, int c) {
+  return c + 1 < NC ? q.v[c + 1 < NC ? c + 1 : 0] : sw_next(q.v[0]);
+}
+template <typename C, int NC>
+__device__ __forceinline__ C x_prev(const Cols<C, NC> &q, int c) {
+  return c > 0 ? q.v[c > 0 ? c - 1 : 0] : sw_prev(q.v[NC - 1]);
+}
+
+typedef const __attribute__((address_space(4))) int32_t *ConstI32;
+typedef const __attribute__((address_space(4))) uint64_t *ConstU64;
+
+// Slices of packed rows a wave keeps in LDS: the L - 1 slices above the first level's, rounded up
+// to a power of two.
+constexpr int sweep_ring(int L) { return L <= 2 ? 1 : L == 3 ? 2 : L <= 5 ? 4 : 8; }
+
+constexpr uint32_t kDrop = 0x80000000u;  // offset bit that puts a store out of range
+
+}  // namespace
+
+template <typename S, int L, int LM, int TY, int WY, int NC, int HX>
+__global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_kernel(
+    SweepArgs<S, typename CoefOf<typename Fmt<S>::C>::T, typename Fmt<S>::C> a) {
+#pragma clang fp contract(off)
+  typedef typename Fmt<S>::C C;
+  typedef typename CoefOf<C>::T CE;
+  typedef const __attribute__((address_space(4))) SweepArgs<S, CE, C> *ConstArgs;
+  typedef Cols<C, NC> V;
+  typedef Raw<S, NC> R;
+  typedef typename std::conditional<NC == 2, uint32_t, uint16_t>::type PM;
+  static_assert(TY >= 2 && TY <= 8 && L >= 1 && L <= LM && LM <= 8 && HX >= LM && HX % NC == 0, "");
+  constexpr int W = 64 * NC, OX = W - 2 * HX;
+  constexpr int H = WY * TY, OY = H - 2 * LM;
+  constexpr int RING = sweep_ring(L);
+  constexpr uint64_t kRowAir = L == 8 ? 0x0101010101010101ull : 0x0101010101010101ull & ((1ull << (8 * L % 64)) - 1ull);
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const int X = a.X, Y = a.Y, Z = a.Z;
+  const unsigned ncol = (unsigned)a.ncol;
+  // XCD-aware order: every XCD walks a contiguous run of tiles
+  const unsigned total = gridDim.x, lin = blockIdx.x, full = total & ~7u;
+  unsigned tile = lin < full ? (lin & 7u) * (full >> 3) + (lin >> 3) : lin;
+  const int slot = (int)(tile % (unsigned)a.n_slots);
+  tile /= (unsigned)a.n_slots;
+  const unsigned nxy = (unsigned)(a.nbx * a.nby);
+  const unsigned tl = tile % nxy;
+  const int bzi = (int)(tile / nxy);
+  const unsigned bg = (unsigned)a.band;
+  const unsigned band = tl / (bg * a.nbx), in_band = tl % (bg * a.nbx);
+  const unsigned band_rows = min(bg, (unsigned)a.nby - band * bg);
+  const int byi = (int)(band * bg + in_band % band_rows);
+  const int bxi = (int)(in_band / band_rows);
+  const int64_t soff = (int64_t)slot * a.slot_elems;
+  const S *__restrict__ gA = a.A + soff;
+  const S *__restrict__ gB = a.B + soff;
+  S *__restrict__ gC = a.Cn + soff;
+  S *__restrict__ gD = a.Dn + soff;
+
+  const int x0 = bxi * OX - HX + NC * lane;           // this lane's first column
+  const int yw = byi * OY - LM + wave * TY;           // this wave's first row
+  const int z0 = 1 + bzi * a.zc, z1 = min(z0 + a.zc, Z - 1);
+
+  // LDS: coefficient rows | halo rows [2][L][WY][2][64] | packed rows [WY][RING][TY][64]
+  extern __shared__ __align__(16) unsigned char s_dyn[];
+  CE *s_coef = reinterpret_cast<CE *>(s_dyn);
+  V *s_halo = reinterpret_cast<V *>(s_dyn + sizeof(CE) * (kStageRows * ncol + 1));
+  PM *s_pm = reinterpret_cast<PM *>(s_halo + 2 * L * WY * 2 * 64) + wave * (RING * TY * 64) + lane;
+  for (unsigned i = threadIdx.x; i < kStageRows * ncol; i += 64 * WY)
+    s_coef[i] = a.coef[(i / ncol) * 256u + i % ncol];
+  if (threadIdx.x == 0) {  // outside voxels: the result is 0
+    CE e = a.coef[0];
+    e.inv = 0;
+    s_coef[kStageRows * ncol] = e;
+  }
+
+  const size_t XY = (size_t)X * (size_t)Y;
+  const uint32_t sbytes = (uint32_t)(XY * sizeof(S));
+  const size_t XYP = (size_t)a.pitch * (size_t)Y;
+  const uint32_t vcol = (uint32_t)((yw * X + x0) * (int)sizeof(S));
+  const uint32_t pcol = (uint32_t)((yw * a.pitch + x0) * 2);
+  // owned columns of this lane, owned rows of this wave
+  const bool own_x = NC * lane >= HX && NC * lane < HX + OX && x0 < X;
+  const uint32_t vst = own_x ? vcol : kDrop;
+  uint32_t own_rows = 0;
+#pragma unroll
+  for (int r = 0; r < TY; ++r) {
+    const int br = wave * TY + r, y = yw + r;
+    if (br >= LM && br < LM + OY && y < Y) own_rows |= 1u << r;
+  }
+  bool col_ok[NC];
+#pragma unroll
+  for (int c = 0; c < NC; ++c) col_ok[c] = x0 + c > 0 && x0 + c < X - 1;
+  const bool x_odd = NC == 2 && (X & 1);
+  const C air_tk = a.air.tk, lam2 = a.lam2;
+  const uint32_t air_pm = a.air_pm, air_mask = a.air_mask, out_pm = kStageRows * ncol * 0x10001u;
+
+  // air and solid rows of this wave's tile (a byte each per slice, 8 slices per word), and its
+  // events by z
+  const int wt = (byi * WY + wave) * a.nbx + bxi;
+  const ConstU64 gair = (ConstU64)(a.row_bits + 2 * (size_t)wt * a.air_words);
+  int ev = 0, ev_end = 0;
+  {
+    const int et = slot * (a.nby * WY * a.nbx) + wt;
+    ev = ((ConstI32)a.ev_ptr)[et];
+    ev_end = ((ConstI32)a.ev_ptr)[et + 1];
+  }
+  auto ev_at = [&](int n, int i) -> int {
+    ConstArgs ka = (ConstArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(ka));
+    return ((ConstI32)ka->events)[4 * n + i];
+  };
+
+  V q[L][2][TY];  // level 0: P^n, level i: P^{n+i}; two slices each
+  typename R::T pl[TY], pq[TY];  // raw P^n[k+1] and P^{n-1}[k]
+  uint32_t pmr[TY];              // packed entries of slice k where it is not all air
+#pragma unroll
+  for (int i = 0; i < L; ++i)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < TY; ++r)
+#pragma unroll
+        for (int c = 0; c < NC; ++c) q[i][b][r].v[c] = (C)0;
+#pragma unroll
+  for (int r = 0; r < TY; ++r) pmr[r] = 0;
+
+  auto a_rsrc = [&](int k) {
+    const bool in = k >= 0 && k < Z;
+    return sw_rsrc(gA + (in ? (size_t)k * XY : 0), in ? sbytes : 0u);
+  };
+  auto b_rsrc = [&](int k) {
+    const bool in = k >= 1 && k < Z - 1;
+    return sw_rsrc(gB + (in ? (size_t)k * XY : 0), in ? sbytes : 0u);
+  };
+  auto load_pm = [&](int k) __attribute__((always_inline)) {
+    const bool in = k >= 1 && k < Z - 1;
+    const auto rp = sw_rsrc(a.pm + (in ? (size_t)k * XYP : 0), in ? (uint32_t)(XYP * 2) : 0u);
+    uint32_t off = pcol, step = (uint32_t)a.pitch * 2u;
+#pragma unroll
+    for (int r = 0; r < TY; ++r, off += step)
+      pmr[r] = NC == 2 ? __builtin_amdgcn_raw_buffer_load_b32(rp, (int)off, 0, 0)
+                       : (uint32_t)__builtin_amdgcn_raw_buffer_load_b16(rp, (int)off, 0, 0);
+  };
+  auto halo_at = [&](int buf, int lev, int w, int side) -> V * {
+    return s_halo + (((buf * L + lev) * WY + w) * 2 + side) * 64 + lane;
+  };
+  const int wu = wave > 0 ? wave - 1 : 0, wd = wave < WY - 1 ? wave + 1 : WY - 1;
+
+  // row bytes of the current and the next 8 slices: x plain air, y solid (or not updated); every
+  // row of a slice outside 1..Z-2 is solid
+  struct Rows {
+    uint64_t air, solid;
+  };
+  Rows bw, bn;
+  auto load_rows = [&](int w) -> Rows {
+    if (w >= a.air_words) return Rows{0, 0};
+    return Rows{gair[2 * w], gair[2 * w + 1]};
+  };
+  struct RowBits {
+    uint32_t air, solid;
+  };
+  auto row_bits = [&](int k, bool step) -> RowBits {
+    if (k < 1 || k > Z - 2) return RowBits{0u, 0xFFu};
+    if (step && (k & 7) == 0) {
+      bw = bn;
+      bn = load_rows((k >> 3) + 1);
+    }
+    const int sh = 8 * (k & 7);
+    return RowBits{(uint32_t)(bw.air >> sh) & air_mask, (uint32_t)(bw.solid >> sh) & 0xFFu};
+  };
+
+  const int kb = z0 - (L - 1), ke = z1 - 1 + (L - 1);
+  {
+    const uint32_t rstep = (uint32_t)X * (uint32_t)sizeof(S);
+    const auto r0 = a_rsrc(kb - 1), r1 = a_rsrc(kb), r2 = a_rsrc(kb + 1), rq = b_rsrc(kb);
+#pragma unroll
+    for (int r = 0; r < TY; ++r) {
+      q[0][0][r] = R::up(R::ld(r0, vcol + r * rstep));
+      q[0][1][r] = R::up(R::ld(r1, vcol + r * rstep));
+    }
+#pragma unroll
+    for (int r = 0; r < TY; ++r) {
+      pl[r] = R::ld(r2, vcol + r * rstep);
+      pq[r] = R::ld(rq, vcol + r * rstep);
+    }
+    *halo_at((kb - 1) & 1, 0, wave, 0) = q[0][1][0];
+    *halo_at((kb - 1) & 1, 0, wave, 1) = q[0][1][TY - 1];
+  }
+  // first event at or above the first slice of this chunk
+  for (int hi = ev_end; ev < hi;) {
+    const int mid = (ev + hi) >> 1;
+    if (ev_at(mid, 0) < kb)
+      ev = mid + 1;
+    else
+      hi = mid;
+  }
+  // row bytes of slices k, k-1, ...: those below the chunk count as air and solid (their levels
+  // are not used)
+  uint64_t hist = ~0ull, hist_s = ~0ull;
+  {
+    const int kf = kb < 1 ? 1 : kb;
+    bw = load_rows(kf >> 3);
+    bn = load_rows((kf >> 3) + 1);
+  }
+  RowBits rows_k = row_bits(kb, false);
+  if ((rows_k.air | rows_k.solid) != 0xFFu) load_pm(kb);
+  __syncthreads();
+
+  auto body = [&](auto cur_c, int k) __attribute__((always_inline)) {
+    constexpr int cur = decltype(cur_c)::value;
+    // slices prev = cur ^ 1 hold k-1 (level i: k-1-i), cur hold k (k-i)
+    hist = (hist << 8) | rows_k.air;
+    hist_s = (hist_s << 8) | rows_k.solid;
+    const int hb = (k - 1) & 1;
+    uint32_t ev_rows = 0;  // rows with an event on one of the slices k-L+1 .. k
+    if (ev < ev_end) {
+      while (ev < ev_end && ev_at(ev, 0) < k - (L - 1)) ++ev;
+      for (int n = ev; n < ev_end && ev_at(n, 0) <= k; ++n) ev_rows |= 1u << (ev_at(n, 2) - yw);
+    }
+    const RowBits rows_next = row_bits(k + 1, true);
+    const auto ra = a_rsrc(k + 2), rb = b_rsrc(k + 1);
+    const int sC = k - (L - 2), sD = k - (L - 1);
+    const bool inC = L >= 2 && sC >= z0 && sC < z1, inD = sD >= z0 && sD < z1;
+    const auto rC = sw_rsrc(gC + (inC ? (size_t)sC * XY : 0), inC ? sbytes : 0u);
+    const auto rD = sw_rsrc(gD + (inD ? (size_t)sD * XY : 0), inD ? sbytes : 0u);
+    // row offsets are formed where used: kept across the sweep they would hold 2 TY registers
+    uint32_t rstep = (uint32_t)X * (uint32_t)sizeof(S);
+    asm volatile("" : "+s"(rstep));
+    V hu[L], hd[L];
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+      hu[i] = *halo_at(hb, i, wu, 1);
+      hd[i] = *halo_at(hb, i, wd, 0);
+    }
+
+    // One row of every level. KIND 0: plain air at all of them; 1: the table; 2: the table and
+    // this row's events; 3: solid at all of them.
+    auto row = [&](auto kind, int r) __attribute__((always_inline)) {
+      constexpr int KIND = decltype(kind)::value;
+      constexpr bool TABLE = KIND == 1 || KIND == 2;
+      // every level's entries first: the gathers then overlap the arithmetic
+      uint32_t pm[L + 1];
+      CE e[2][NC];
+      V t[L + 1];
+      t[0] = R::up(pl[r]);
+      const V past0 = R::up(pq[r]);
+      auto gather = [&](int i) __attribute__((always_inline)) {
+        if ((hist >> (8 * (i - 1) + r)) & 1ull)
+          pm[i] = air_pm;
+        else if ((hist_s >> (8 * (i - 1) + r)) & 1ull)
+          pm[i] = out_pm;
+#pragma unroll
+        for (int c = 0; c < NC; ++c) e[i & 1][c] = s_coef[c == 0 ? pm[i] & 0xFFFFu : pm[i] >> 16];
+      };
+      if constexpr (TABLE) {
+#pragma unroll
+        for (int i = 2; i <= L; ++i)
+          pm[i] = (uint32_t)s_pm[(((k - (i - 1)) & (RING - 1)) * TY + r) * 64];
+        pm[1] = pmr[r];
+        gather(1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int i = 1; i <= L; ++i) {
+        const V zn = t[i - 1];
+        const V zp = q[i - 1][cur ^ 1][r];
+        const V ce = q[i - 1][cur][r];
+        const V yn = r + 1 < TY ? q[i - 1][cur][r + 1 < TY ? r + 1 : r] : hd[i - 1];
+        const V yp = r > 0 ? q[i - 1][cur][r > 0 ? r - 1 : r] : hu[i - 1];
+        const V past = i == 1 ? past0 : q[i >= 2 ? i - 2 : 0][cur ^ 1][r];
+        const int s = k - (i - 1);
+        if constexpr (TABLE) {
+          if (i < L) {  // the next level's entries are in flight during this level
+            gather(i + 1 <= L ? i + 1 : L);
+            __builtin_amdgcn_sched_barrier(0);
+          }
+        }
+        const bool row_ok = !((hist_s >> (8 * (i - 1) + r)) & 1ull);
+#pragma unroll
+        for (int c = 0; c < NC; ++c) {
+          if constexpr (KIND == 3) {
+            t[i].v[c] = (C)0;
+            continue;
+          }
+          C u = zn.v[c] + zp.v[c];
+          u = u + yn.v[c];
+          u = u + yp.v[c];
+          u = u + x_next(ce, c);
+          u = u + x_prev(ce, c);
+          if constexpr (KIND == 0) {
+            t[i].v[c] = Fmt<S>::round((air_tk * ce.v[c] + lam2 * u) - past.v[c]);
+          } else if constexpr (TABLE) {
+            const CE &n = e[i & 1][c];
+            C v = n.inv * ((n.tk * ce.v[c] + lam2 * u) - n.omb * past.v[c]);
+            sw_keep(v);
+            t[i].v[c] = Fmt<S>::round((row_ok && col_ok[c]) ? v : (C)0);
+          }
+        }
+        if constexpr (KIND == 2) {
+          // the event arguments are re-read here, so that they hold no scalar registers across
+          // the sweep
+          ConstArgs ka = (ConstArgs)__builtin_amdgcn_kernarg_segment_ptr();
+          asm volatile("" : "+s"(ka));
+          const ConstI32 gev = (ConstI32)ka->events;
+          for (int n = ev; n < ev_end && gev[4 * n] <= k; ++n) {
+            if (gev[4 * n] != s || gev[4 * n + 2] != yw + r) continue;
+            const int xe = gev[4 * n + 1], id = gev[4 * n + 3];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+              if (xe != x0 + c) continue;
+              if (id < 0) {  // receiver
+                if (own_x && ((own_rows >> r) & 1u) && s >= z0 && s < z1)
+                  ka->resp[(int64_t)(id & 0x7FFFFFFF) * ka->resp_steps + ka->step + i - 1] =
+                      (double)t[i].v[c] * ka->inv_scale;
+              } else if (ka->step + i < ka->inject_end) {
+                C smp = (C)0;
+                if (ka->step + i < ka->n_samples)
+                  smp = (C)ka->sig[(int64_t)id * ka->n_samples + ka->step + i];
+                smp = smp * ka->scale;
+                const bool hard = ka->src_kind[id] == 0 || ka->soft_overwrite;
+                t[i].v[c] = Fmt<S>::round(hard ? smp : t[i].v[c] + smp);
+              }
+            }
+          }
+        }
+        if (i >= L - 1 && i >= 1) {
+          const uint32_t off = (vst + r * rstep) | (((own_rows >> r) & 1u) ? 0u : kDrop);
+          const auto rs = i == L ? rD : rC;
+          if (KIND != 0 && x_odd) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+              R::st1(rs, (off | (x0 + c < X ? 0u : kDrop)) + c * (uint32_t)sizeof(S), t[i].v[c]);
+          } else {
+            R::st(rs, off, t[i]);
+          }
+        }
+      }
+      if constexpr (TABLE && L > 1) s_pm[((k & (RING - 1)) * TY + r) * 64] = (PM)pmr[r];
+#pragma unroll
+      for (int i = 0; i < L; ++i) q[i][cur ^ 1][r] = t[i];
+      __builtin_amdgcn_sched_barrier(0);
+      pl[r] = R::ld(ra, vcol + r * rstep);
+      pq[r] = R::ld(rb, vcol + r * rstep);
+    };
+    // the choice is made row by row: one choice for all rows would keep every queue entry of
+    // the iteration live beside its replacement
+    auto rows = [&](int r) __attribute__((always_inline)) {
+      if ((ev_rows >> r) & 1u)
+        row(std::integral_constant<int, 2>(), r);
+      else if (((hist >> r) & kRowAir) == kRowAir)
+        row(std::integral_constant<int, 0>(), r);
+      else if (((hist_s >> r) & kRowAir) == kRowAir)
+        row(std::integral_constant<int, 3>(), r);
+      else
+        row(std::integral_constant<int, 1>(), r);
+    };
+#pragma unroll
+    for (int r = 1; r < TY - 1; ++r) rows(r);
+    rows(0);
+    rows(TY - 1);
+    // publish the edge rows of the new slices
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+      *halo_at(hb ^ 1, i, wave, 0) = q[i][cur ^ 1][0];
+      *halo_at(hb ^ 1, i, wave, 1) = q[i][cur ^ 1][TY - 1];
+    }
+    rows_k = rows_next;
+    if ((rows_k.air | rows_k.solid) != 0xFFu) load_pm(k + 1);
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+  };
+  for (int k = kb;;) {
+    body(std::integral_constant<int, 1>(), k);
+    if (++k > ke) break;
+    body(std::integral_constant<int, 0>(), k);
+    if (++k > ke) break;
+  }
+}
+
+// Coefficient entry per voxel: row min(K, 6) of ncol material columns, or kStageRows * ncol outside.
+__global__ __launch_bounds__(256) void pack_entry_kernel(const uint8_t *__restrict__ pos,
+                                                         const uint8_t *__restrict__ mat,
+                                                         uint16_t *__restrict__ pm, int X,
+                                                         int pitch, int64_t rows, unsigned ncol) {
+  const int64_t n = rows * pitch;
+  for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
+    const int64_t row = i / pitch;
+    const int x = (int)(i - row * pitch);
+    unsigned v = kStageRows * ncol;
+    if (x < X) {
+      const unsigned p = pos[row * X + x], m = mat[row * X + x];
+      if (p & 0x80u) v = min(p & 0x7Fu, 6u) * ncol + min(m, ncol - 1);
+    }
+    pm[i] = (uint16_t)v;
+  }
+}
+
+hipError_t launch_pack_entry(const uint8_t *pos, const uint8_t *mat, uint16_t *pm, int X, int Y,
+                             int Z, int pitch, int ncol, hipStream_t stream) {
+  const int64_t rows = (int64_t)Y * Z, n = rows * pitch;
+  const unsigned grid = (unsigned)std::min<int64_t>((n + 255) / 256, 65536);
+  hipLaunchKernelGGL(pack_entry_kernel, dim3(grid), dim3(256), 0, stream, pos, mat, pm, X, pitch,
+                     rows, (unsigned)ncol);
+  return hipGetLastError();
+}
+
+// Two bytes per (wave tile, slice), 8 slices to a pair of words: bit r of the first is set when the
+// tile's row r is plain air over its whole window (and inside the grid), of the second when no
+// voxel of it is updated (outside voxels, or past the grid). Bits past the tile's rows are set in
+// both. A wave per tile and word.
+__global__ __launch_bounds__(64) void row_bits_kernel(const uint16_t *__restrict__ pm, int pitch,
+                                                      uint64_t *__restrict__ out, int X, int Y,
+                                                      int Z, int nbx, int ox, int hx, int w,
+                                                      int oy, int lm, int wy, int ty, int words,
+                                                      unsigned ncol) {
+  const int lane = threadIdx.x;
+  const int bx = blockIdx.x, tw = blockIdx.y;
+  const int xs = bx * ox - hx, ys = (tw / wy) * oy - lm + (tw % wy) * ty;
+  const bool x_in = xs >= 0 && xs + w <= X;
+  for (int word = blockIdx.z; word < words; word += gridDim.z) {
+    uint64_t air = 0, solid = 0;
+    for (int b = 0; b < 8; ++b) {
+      const int z = 8 * word + b;
+      uint32_t ma = (0xFFu << ty) & 0xFFu, ms = ma;
+      const uint16_t *slice = pm + (size_t)min(z, Z - 1) * (size_t)pitch * (size_t)Y;
+      for (int r = 0; r < ty; ++r) {
+        const int y = ys + r;
+        bool not_air = !x_in, not_solid = false;
+        if (y < 0 || y >= Y || z >= Z) {
+          not_air = true;
+        } else {
+          for (int c = lane; c < w; c += 64) {
+            if (xs + c < 0 || xs + c >= X) continue;
+            const unsigned v = slice[(size_t)y * pitch + xs + c];
+            not_air = not_air || v < 6u * ncol || v >= kStageRows * ncol;
+            not_solid = not_solid || v < kStageRows * ncol;
+          }
+        }
+        if (__ballot(not_air) == 0) ma |= 1u << r;
+        if (__ballot(not_solid) == 0) ms |= 1u << r;
+      }
+      air |= (uint64_t)ma << (8 * b);
+      solid |= (uint64_t)ms << (8 * b);
+    }
+    if (lane == 0) {
+      const size_t o = 2 * (((size_t)tw * nbx + bx) * words + word);
+      out[o] = air;
+      out[o + 1] = solid;
+    }
+  }
+}
+
+namespace {
+
+// Tile of the sweep per storage type: columns per lane, rows per wave, waves, most levels, halo
+// columns. Eight waves at 233 (FP32) and 227 (FP64) VGPRs, two waves per SIMD and one block per CU
+// (160 KB of LDS with 255 materials).
+template <typename S>
+struct SweepTile {
+  static constexpr int NC = 2, TY = 6, WY = 8, LM = 5, HX = 8;
+};
+template <>
+struct SweepTile<double> {
+  static constexpr int NC = 1, TY = 8, WY = 8, LM = 4, HX = 4;
+};
+
+template <typename S>
+SweepPlan plan_of(int X, int Y, int Z, int zc, int slots) {
+  typedef SweepTile<S> T;
+  SweepPlan p;
+  p.nc = T::NC;
+  p.ty = T::TY;
+  p.wy = T::WY;
+  p.lm = T::LM;
+  p.w = 64 * T::NC;
+  p.hx = T::HX;
+  p.ox = p.w - 2 * p.hx;
+  p.oy = T::TY * T::WY - 2 * T::LM;
+  p.nbx = (X + p.ox - 1) / p.ox;
+  p.nby = (Y + p.oy - 1) / p.oy;
+  p.words = (Z + 7) / 8;
+  p.pitch = X + (X & 1);
+  p.band = 2;
+  const int zi = Z - 2;
+  const int64_t bxy = (int64_t)p.nbx * p.nby * slots;
+  if (zc < 1) {
+    // One block per CU: a launch takes as many rounds as 256 goes into its blocks, and a round the
+    // chunk's slices plus the 2 (LM - 1) of its neighbours' and about two more to start. The chunk
+    // count with the least of both: on 256x256x256 FP32 24 slices (231 blocks) take 34 us per step,
+    // 16 slices (two rounds) 50 and 32 slices 42; on 1024x768x384 48-64 slices 345, 32 and 96
+    // slices 354 and 371.
+    double best = 0;
+    for (int nz = 1; nz <= zi; ++nz) {
+      const int c = (zi + nz - 1) / nz;
+      if (nz > 1 && c == (zi + nz - 2) / (nz - 1)) continue;
+      const int64_t blocks = bxy * ((zi + c - 1) / c);
+      const double full = (double)((blocks + 255) / 256);
+      const double rounds = blocks <= 1024 ? full : std::min(full, blocks / 256.0 + 0.4);
+      const double cost = rounds * (c + 2 * (T::LM - 1) + 2);
+      if (nz == 1 || cost < best) {
+        best = cost;
+        zc = c;
+      }
+    }
+  }
+  p.zc = std::min(zc, zi);
+  p.blocks = bxy * ((zi + p.zc - 1) / p.zc);
+  return p;
+}
+
+template <typename S, int L>
+hipError_t launch_levels(const SweepPlan &p, SweepArgs<S, typename CoefOf<typename Fmt<S>::C>::T, typename Fmt<S>::C> &a,
+                         hipStream_t stream) {
+  typedef SweepTile<S> T;
+  typedef typename Fmt<S>::C C;
+  typedef typename CoefOf<C>::T CE;
+  constexpr int RING = sweep_ring(L);
+  const size_t lds = sizeof(CE) * (kStageRows * (size_t)a.ncol + 1) +
+                     sizeof(Cols<C, T::NC>) * 2 * L * T::WY * 2 * 64 +
+                     2 * T::NC * (size_t)T::WY * RING * T::TY * 64;
+  hipLaunchKernelGGL((srl_sweep_kernel<S, L, T::LM, T::TY, T::WY, T::NC, T::HX>), dim3((unsigned)p.blocks),
+                     dim3(64 * T::WY), lds, stream, a);
+  return hipGetLastError();
+}
+
+template <typename S, typename A>
+hipError_t launch_any(const SweepPlan &p, A &a, int levels, hipStream_t stream) {
+  a.pitch = p.pitch;
+  a.air_words = p.words;
+  a.zc = p.zc;
+  a.nbx = p.nbx;
+  a.nby = p.nby;
+  a.band = p.band;
+  switch (levels) {
+  case 1: return launch_levels<S, 1>(p, a, stream);
+  case 2: return launch_levels<S, 2>(p, a, stream);
+  case 3: return launch_levels<S, 3>(p, a, stream);
+  case 4:
+    if constexpr (SweepTile<S>::LM >= 4) return launch_levels<S, 4>(p, a, stream);
+    break;
+  case 5:
+    if constexpr (SweepTile<S>::LM >= 5) return launch_levels<S, 5>(p, a, stream);
+    break;
+  case 6:
+    if constexpr (SweepTile<S>::LM >= 6) return launch_levels<S, 6>(p, a, stream);
+    break;
+  }
+  return hipErrorInvalidValue;
+}
+
+}  // namespace
+
+SweepPlan plan_sweep(int precision, int X, int Y, int Z, int zc, int slots) {
+  return precision == PFDTD_F64 ? plan_of<double>(X, Y, Z, zc, slots) : plan_of<float>(X, Y, Z, zc, slots);
+}
+
+hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint64_t *out, int X, int Y,
+                           int Z, int ncol, hipStream_t stream) {
+  const dim3 grid((unsigned)p.nbx, (unsigned)(p.nby * p.wy), (unsigned)std::min(p.words, 65535));
+  hipLaunchKernelGGL(row_bits_kernel, grid, dim3(64), 0, stream, pm, p.pitch, out, X, Y, Z, p.nbx,
+                     p.ox, p.hx, p.w, p.oy, p.lm, p.wy, p.ty, p.words, (unsigned)ncol);
+  return hipGetLastError();
+}
+
+hipError_t launch_sweep_f32(const SweepPlan &p, SweepArgs<float, CoefF, float> a, int levels,
+                            hipStream_t stream) {
+  return launch_any<float>(p, a, levels, stream);
+}
+hipError_t launch_sweep_f64(const SweepPlan &p, SweepArgs<double, CoefD, double> a, int levels,
+                            hipStream_t stream) {
+  return launch_any<double>(p, a, levels, stream);
+}
+}  // namespace pfdtd
