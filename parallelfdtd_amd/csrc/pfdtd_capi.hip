@@ -809,7 +809,7 @@ int build_sweep_events(pfdtd_ctx *c, const SweepPlan &p) {
 // below 2^31 bytes and the automatic settings.
 bool sweep_eligible(const pfdtd_ctx *c) {
   if (c->scheme != 0 || c->levels != 0 || c->fshape != PFDTD_SWEEP_AUTO) return false;
-  if (c->precision != PFDTD_F32 && c->precision != PFDTD_F64) return false;
+  if (c->precision == PFDTD_F16_DIFF) return false;
   const uint64_t esz = elem_size(c->precision);
   return fused_eligible(c) && (uint64_t)c->X * (uint64_t)c->Y * esz < (1ull << 31);
 }
@@ -889,12 +889,19 @@ SweepArgs<S, CT, C> sweep_args(const pfdtd_ctx *c, const CT *coef, CT air, C lam
 // current and past fields are in d_P and d_Pp afterwards.
 hipError_t run_sweep(pfdtd_ctx *c, const SweepPlan &p, int step, int levels, int inject_end) {
   hipError_t e;
-  if (c->precision == PFDTD_F64)
+  auto args = [&](auto tag) {
+    typedef decltype(tag) S;
+    return sweep_args<S>(c, c->d_coef_f, c->air_f, c->lam2_f, c->d_sig_f, step, inject_end);
+  };
+  switch (c->precision) {
+  case PFDTD_F64:
     e = launch_sweep_f64(p, sweep_args<double>(c, c->d_coef_d, c->air_d, c->lam2_d, c->d_sig_d,
                                                step, inject_end), levels, c->stream);
-  else
-    e = launch_sweep_f32(p, sweep_args<float>(c, c->d_coef_f, c->air_f, c->lam2_f, c->d_sig_f,
-                                              step, inject_end), levels, c->stream);
+    break;
+  case PFDTD_F16: e = launch_sweep_f16(p, args(h16{}), levels, c->stream); break;
+  case PFDTD_BF16: e = launch_sweep_bf16(p, args(b16{}), levels, c->stream); break;
+  default: e = launch_sweep_f32(p, args(float{}), levels, c->stream);
+  }
   if (levels > 1) {
     std::swap(c->d_P, c->d_P2);
     std::swap(c->d_Pp, c->d_Pp2);

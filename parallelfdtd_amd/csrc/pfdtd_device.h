@@ -45,6 +45,9 @@ struct Fmt<h16> {
     asm("" : "+v"(v));
     return __builtin_bit_cast(uint16_t, (_Float16)v);
   }
+  static __device__ __forceinline__ uint32_t bits2(float lo, float hi) {
+    return (uint32_t)bits(lo) | ((uint32_t)bits(hi) << 16);
+  }
   static __device__ __forceinline__ void st(h16 *p, int64_t i, float v) { p[i].bits = bits(v); }
   static __device__ __forceinline__ float val(h16 s) {
     return (float)__builtin_bit_cast(_Float16, s.bits);
@@ -62,11 +65,15 @@ struct Fmt<b16> {
     return __uint_as_float((uint32_t)p[i].bits << 16);
   }
   static __device__ __forceinline__ uint16_t bits(float v) {
-    const uint32_t x = __float_as_uint(v);
-    const uint32_t rne = (x + 0x7FFFu + ((x >> 16) & 1u)) >> 16;  // round to nearest even
-    const uint32_t qnan = (x >> 16) | 0x40u;                       // NaN stays a (quiet) NaN
-    // a select, not a branch: a lane-divergent branch here made every rounding a masked region
-    return (uint16_t)((x & 0x7FFFFFFFu) > 0x7F800000u ? qnan : rne);
+    // v_cvt_pk_bf16_f32: round to nearest even, NaN stays a (quiet) NaN -- for all 2^32 inputs the
+    // bits of (x + 0x7FFF + (x >> 16 & 1)) >> 16 and, for NaN, (x >> 16) | 0x40
+    return __builtin_bit_cast(uint16_t, (__bf16)v);
+  }
+  static __device__ __forceinline__ uint32_t bits2(float lo, float hi) {
+    typedef float f2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 b2 __attribute__((ext_vector_type(2)));
+    const f2 v = {lo, hi};
+    return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, b2));
   }
   static __device__ __forceinline__ void st(b16 *p, int64_t i, float v) { p[i].bits = bits(v); }
   static __device__ __forceinline__ float val(b16 s) { return __uint_as_float((uint32_t)s.bits << 16); }

@@ -290,6 +290,10 @@ hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint64_t *out
                            int Z, int ncol, hipStream_t stream);
 hipError_t launch_sweep_f32(const SweepPlan &p, SweepArgs<float, CoefF, float> a, int levels,
                             hipStream_t stream);
+hipError_t launch_sweep_f16(const SweepPlan &p, SweepArgs<h16, CoefF, float> a, int levels,
+                            hipStream_t stream);
+hipError_t launch_sweep_bf16(const SweepPlan &p, SweepArgs<b16, CoefF, float> a, int levels,
+                             hipStream_t stream);
 hipError_t launch_sweep_f64(const SweepPlan &p, SweepArgs<double, CoefD, double> a, int levels,
                             hipStream_t stream);
 

@@ -93,15 +93,17 @@ struct Raw<float, 2> {
   static __device__ __forceinline__ Cols<float, 2> up(T t) {
     return Cols<float, 2>{{__uint_as_float(t.x), __uint_as_float(t.y)}};
   }
-  static __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, uint32_t off,
-                                            const Cols<float, 2> &c) {
+  static __device__ __forceinline__ T pack(const Cols<float, 2> &c) {
     u32x2 t;
     t.x = __float_as_uint(c.v[0]);
     t.y = __float_as_uint(c.v[1]);
+    return t;
+  }
+  static __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, uint32_t off, T t) {
     __builtin_amdgcn_raw_buffer_store_b64(t, r, (int)off, 0, 0);
   }
-  static __device__ __forceinline__ void st1(__amdgpu_buffer_rsrc_t r, uint32_t off, float v) {
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(v), r, (int)off, 0, 0);
+  static __device__ __forceinline__ void st1(__amdgpu_buffer_rsrc_t r, uint32_t off, T t, int c) {
+    __builtin_amdgcn_raw_buffer_store_b32(c ? t.y : t.x, r, (int)off, 0, 0);
   }
 };
 template <>
@@ -113,12 +115,14 @@ struct Raw<double, 1> {
   static __device__ __forceinline__ Cols<double, 1> up(T t) {
     return Cols<double, 1>{{__hiloint2double((int)t.y, (int)t.x)}};
   }
-  static __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, uint32_t off,
-                                            const Cols<double, 1> &c) {
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, c.v[0]), r, (int)off, 0, 0);
+  static __device__ __forceinline__ T pack(const Cols<double, 1> &c) {
+    return __builtin_bit_cast(u32x2, c.v[0]);
   }
-  static __device__ __forceinline__ void st1(__amdgpu_buffer_rsrc_t r, uint32_t off, double v) {
-    __builtin_amdgcn_raw_buffer_store_b64(__builtin_bit_cast(u32x2, v), r, (int)off, 0, 0);
+  static __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, uint32_t off, T t) {
+    __builtin_amdgcn_raw_buffer_store_b64(t, r, (int)off, 0, 0);
+  }
+  static __device__ __forceinline__ void st1(__amdgpu_buffer_rsrc_t r, uint32_t off, T t, int) {
+    st(r, off, t);
   }
 };
 template <typename S>
@@ -131,13 +135,14 @@ struct Raw<S, 2> {
   static __device__ __forceinline__ Cols<float, 2> up(T t) {
     return Cols<float, 2>{{Fmt<S>::val(S{(uint16_t)(t & 0xFFFFu)}), Fmt<S>::val(S{(uint16_t)(t >> 16)})}};
   }
-  static __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, uint32_t off,
-                                            const Cols<float, 2> &c) {
-    const uint32_t t = (uint32_t)Fmt<S>::raw(c.v[0]).bits | ((uint32_t)Fmt<S>::raw(c.v[1]).bits << 16);
+  static __device__ __forceinline__ T pack(const Cols<float, 2> &c) {
+    return Fmt<S>::bits2(c.v[0], c.v[1]);
+  }
+  static __device__ __forceinline__ void st(__amdgpu_buffer_rsrc_t r, uint32_t off, T t) {
     __builtin_amdgcn_raw_buffer_store_b32(t, r, (int)off, 0, 0);
   }
-  static __device__ __forceinline__ void st1(__amdgpu_buffer_rsrc_t r, uint32_t off, float v) {
-    __builtin_amdgcn_raw_buffer_store_b16(Fmt<S>::raw(v).bits, r, (int)off, 0, 0);
+  static __device__ __forceinline__ void st1(__amdgpu_buffer_rsrc_t r, uint32_t off, T t, int c) {
+    __builtin_amdgcn_raw_buffer_store_b16((unsigned short)(c ? t >> 16 : t & 0xFFFFu), r, (int)off, 0, 0);
   }
 };
 
@@ -432,14 +437,17 @@ __global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_kernel(
           u = u + x_next(ce, c);
           u = u + x_prev(ce, c);
           if constexpr (KIND == 0) {
-            t[i].v[c] = Fmt<S>::round((air_tk * ce.v[c] + lam2 * u) - past.v[c]);
+            t[i].v[c] = (air_tk * ce.v[c] + lam2 * u) - past.v[c];
           } else if constexpr (TABLE) {
             const CE &n = e[i & 1][c];
             C v = n.inv * ((n.tk * ce.v[c] + lam2 * u) - n.omb * past.v[c]);
             sw_keep(v);
-            t[i].v[c] = Fmt<S>::round((row_ok && col_ok[c]) ? v : (C)0);
+            t[i].v[c] = (row_ok && col_ok[c]) ? v : (C)0;
           }
         }
+        // rounded to the storage type once: the stored bits and the value the next level reads
+        typename R::T raw = R::pack(t[i]);
+        if (i < L || KIND == 2) t[i] = R::up(raw);
         if constexpr (KIND == 2) {
           // the event arguments are re-read here, so that they hold no scalar registers across
           // the sweep
@@ -467,15 +475,16 @@ __global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_kernel(
             }
           }
         }
+        if constexpr (KIND == 2) raw = R::pack(t[i]);
         if (i >= L - 1 && i >= 1) {
           const uint32_t off = (vst + r * rstep) | (((own_rows >> r) & 1u) ? 0u : kDrop);
           const auto rs = i == L ? rD : rC;
           if (KIND != 0 && x_odd) {
 #pragma unroll
             for (int c = 0; c < NC; ++c)
-              R::st1(rs, (off | (x0 + c < X ? 0u : kDrop)) + c * (uint32_t)sizeof(S), t[i].v[c]);
+              R::st1(rs, (off | (x0 + c < X ? 0u : kDrop)) + c * (uint32_t)sizeof(S), raw, c);
           } else {
-            R::st(rs, off, t[i]);
+            R::st(rs, off, raw);
           }
         }
       }
@@ -609,6 +618,13 @@ struct SweepTile<double> {
   static constexpr int NC = 1, TY = 8, WY = 8, LM = 4, HX = 4;
 };
 
+template <>
+struct SweepTile<h16> {
+  static constexpr int NC = 2, TY = 6, WY = 8, LM = 5, HX = 8;
+};
+template <>
+struct SweepTile<b16> : SweepTile<h16> {};
+
 template <typename S>
 SweepPlan plan_of(int X, int Y, int Z, int zc, int slots) {
   typedef SweepTile<S> T;
@@ -696,7 +712,12 @@ hipError_t launch_any(const SweepPlan &p, A &a, int levels, hipStream_t stream) 
 }  // namespace
 
 SweepPlan plan_sweep(int precision, int X, int Y, int Z, int zc, int slots) {
-  return precision == PFDTD_F64 ? plan_of<double>(X, Y, Z, zc, slots) : plan_of<float>(X, Y, Z, zc, slots);
+  switch (precision) {
+  case PFDTD_F64: return plan_of<double>(X, Y, Z, zc, slots);
+  case PFDTD_F16: return plan_of<h16>(X, Y, Z, zc, slots);
+  case PFDTD_BF16: return plan_of<b16>(X, Y, Z, zc, slots);
+  default: return plan_of<float>(X, Y, Z, zc, slots);
+  }
 }
 
 hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint64_t *out, int X, int Y,
@@ -710,6 +731,14 @@ hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint64_t *out
 hipError_t launch_sweep_f32(const SweepPlan &p, SweepArgs<float, CoefF, float> a, int levels,
                             hipStream_t stream) {
   return launch_any<float>(p, a, levels, stream);
+}
+hipError_t launch_sweep_f16(const SweepPlan &p, SweepArgs<h16, CoefF, float> a, int levels,
+                            hipStream_t stream) {
+  return launch_any<h16>(p, a, levels, stream);
+}
+hipError_t launch_sweep_bf16(const SweepPlan &p, SweepArgs<b16, CoefF, float> a, int levels,
+                             hipStream_t stream) {
+  return launch_any<b16>(p, a, levels, stream);
 }
 hipError_t launch_sweep_f64(const SweepPlan &p, SweepArgs<double, CoefD, double> a, int levels,
                             hipStream_t stream) {

@@ -12,7 +12,7 @@ from test_gpu_fused import assert_same, run_both
 
 pytestmark = pytest.mark.gpu
 
-OWNED = {N.F32: (112, 38), N.F64: (56, 56)}  # owned columns and rows of a block
+OWNED = {N.F32: (112, 38), N.F64: (56, 56), N.F16: (112, 38), N.BF16: (112, 38)}  # owned columns and rows of a block
 
 
 def scene(seed, dims, n_steps, n_boxes=6, n_src=3, n_rec=8):
