@@ -133,6 +133,10 @@ struct pfdtd_ctx {
   // one after another; per-source/receiver slot
   int lgB = 0;
   int grouped = 0;
+  // an interleaved batch whose runs take the several-level sweep: its fields are held one slot
+  // after another all the same (four buffers) and interleaved when they are read out
+  bool planar = false;
+  size_t planar_nomem = 0;  // field size whose four buffers did not fit
   std::vector<int32_t> src_slot, rec_slot;
   int32_t *d_src_slot = nullptr, *d_rec_slot = nullptr;
   int64_t *d_rec_idx = nullptr;
@@ -290,13 +294,14 @@ int64_t lin_idx(const pfdtd_ctx *c, const int32_t *q) {
 }
 
 // Slots one two-level launch advances (grouped batch), 1 otherwise.
-int batch_slots(const pfdtd_ctx *c) { return c->grouped ? 1 << c->lgB : 1; }
+bool slot_major(const pfdtd_ctx *c) { return c->grouped || c->planar; }
+int batch_slots(const pfdtd_ctx *c) { return slot_major(c) ? 1 << c->lgB : 1; }
 
 // Element index of a source/receiver in the (possibly batched) field, -1 outside the grid.
 int64_t elem_idx(const pfdtd_ctx *c, const int32_t *q, int slot) {
   const int64_t v = lin_idx(c, q);
   if (v < 0) return -1;
-  return c->grouped ? (int64_t)slot * c->N + v : (v << c->lgB) + slot;
+  return slot_major(c) ? (int64_t)slot * c->N + v : (v << c->lgB) + slot;
 }
 
 // 1 when no two in-grid sources share a field element (injection order then cannot matter).
@@ -352,7 +357,7 @@ int scan_domain(pfdtd_ctx *c) {
 // per step on the large room).
 int levels_for(const pfdtd_ctx *c, int precision) {
   if (c->levels) return c->levels;
-  if ((precision == PFDTD_F32 || precision == PFDTD_F64) && (c->lgB == 0 || c->grouped))
+  if ((precision == PFDTD_F32 || precision == PFDTD_F64) && (c->lgB == 0 || slot_major(c)))
     return 3;
   return 2;
 }
@@ -389,6 +394,7 @@ int alloc_domain(pfdtd_ctx *c, int64_t X, int64_t Y, int64_t Z) {
   dfree(c->d_air_rows3);
   // fields sized for the previous grid are dropped
   free_fields(c);
+  c->planar_nomem = 0;
   if (!c->d_pos) {
     hipError_t e1 = hipMalloc((void **)&c->d_pos, (size_t)N);
     hipError_t e2 = e1 == hipSuccess ? hipMalloc((void **)&c->d_mat, (size_t)N) : e1;
@@ -469,7 +475,7 @@ int ensure_fields(pfdtd_ctx *c, int precision, int scale_exp) {
     return fail(PFDTD_E_ARG, "scale_exp applies to F16/BF16 storage only");
   if (scale_exp < -60 || scale_exp > 60) return fail(PFDTD_E_ARG, "scale_exp out of range");
   const size_t bytes = es * ((size_t)c->N << c->lgB);
-  const bool want4 = (c->lgB == 0 || c->grouped) && levels_for(c, precision) >= 2;
+  const bool want4 = (c->lgB == 0 || slot_major(c)) && levels_for(c, precision) >= 2;
   if (c->d_P && c->field_bytes == bytes && (!want4 || c->d_P2)) {
     c->precision = precision;
     c->scale_exp = scale_exp;
@@ -580,7 +586,7 @@ hipError_t launch_update_grouped(pfdtd_ctx *c, const UpdateGeom &g) {
 }
 
 hipError_t launch_update_any(pfdtd_ctx *c, const UpdateGeom &g) {
-  if (c->grouped && c->lgB > 0) return launch_update_grouped(c, g);
+  if (slot_major(c) && c->lgB > 0) return launch_update_grouped(c, g);
   const int ncol = coef_cols(c);
   switch (c->precision) {
   case PFDTD_F32:
@@ -604,19 +610,23 @@ hipError_t launch_update_any(pfdtd_ctx *c, const UpdateGeom &g) {
   }
 }
 
+bool boundary_source(const pfdtd_ctx *c) {
+  for (int s = 0; s < c->n_src; ++s) {
+    const int32_t *q = &c->src_xyz[3 * s];
+    if (lin_idx(c, q) >= 0 && (q[2] == 0 || q[2] == c->Z - 1)) return true;
+  }
+  return false;
+}
+
 // The two-level update needs the spare pair and no source on the never-updated slices
 // z = 0 and z = Z-1 (their values would have to be carried between the four buffers).
 bool fused_eligible(const pfdtd_ctx *c) {
-  if ((c->lgB > 0 && !c->grouped) || levels_for(c, c->precision) < 2 || !c->d_P2 || !c->d_Pp2)
+  if ((c->lgB > 0 && !slot_major(c)) || levels_for(c, c->precision) < 2 || !c->d_P2 || !c->d_Pp2)
     return false;
   // the two-level kernel addresses each z-slice through a buffer descriptor (32-bit range)
   const uint64_t esz = c->precision == PFDTD_F64 ? 8 : (c->precision == PFDTD_F32 ? 4 : 2);
   if ((uint64_t)c->X * (uint64_t)c->Y * esz >= (1ull << 32)) return false;
-  for (int s = 0; s < c->n_src; ++s) {
-    const int32_t *q = &c->src_xyz[3 * s];
-    if (lin_idx(c, q) >= 0 && (q[2] == 0 || q[2] == c->Z - 1)) return false;
-  }
-  return true;
+  return !boundary_source(c);
 }
 
 template <typename S, typename CT, typename C>
@@ -643,7 +653,7 @@ Fused2Args<S, CT, C> fused_args(const pfdtd_ctx *c, const CT *coef, CT air, C la
   a.inject_step = (c->n_src > 0 && step + 1 < c->resp_steps) ? step + 1 : -1;
   a.levels = 2;
   a.diff = c->precision == PFDTD_F16_DIFF ? 1 : 0;
-  if (c->grouped && c->lgB > 0) {
+  if (slot_major(c) && c->lgB > 0) {
     a.n_slots = 1 << c->lgB;
     a.slot_elems = c->N;
     a.src_slot = c->d_src_slot;
@@ -724,7 +734,7 @@ hipError_t launch_update3(pfdtd_ctx *c, const FusedGeom &g, int step) {
 // 8-64 slots on 512x384x256 run 13 % slower per source with 4 x 4 than with 2 x 8.
 UpdateGeom plan_single(const pfdtd_ctx *c) {
   int ry = c->ry, zc = c->zc;
-  const int lgB = c->grouped ? 0 : c->lgB;
+  const int lgB = slot_major(c) ? 0 : c->lgB;
   if (ry == 0) {
     ry = 2;
     zc = 8;
@@ -737,6 +747,10 @@ UpdateGeom plan_single(const pfdtd_ctx *c) {
   }
   return plan_update_batch((int)c->X, (int)c->Y, (int)c->Z, ry, zc, lgB);
 }
+
+}  // namespace
+static int refresh_indices(pfdtd_ctx *c);
+namespace {
 
 // ---- several-level sweep -------------------------------------------------------------------
 
@@ -805,13 +819,38 @@ int build_sweep_events(pfdtd_ctx *c, const SweepPlan &p) {
   return PFDTD_OK;
 }
 
-// Whether the sweep takes this context's runs: the forward scheme, FP32 or FP64 fields, slices
-// below 2^31 bytes and the automatic settings.
-bool sweep_eligible(const pfdtd_ctx *c) {
+// Whether the sweep can take runs of this precision: the forward scheme, slices below 2^31 bytes,
+// the automatic settings, and no source on the never-updated slices.
+bool sweep_takes(const pfdtd_ctx *c, int precision) {
   if (c->scheme != 0 || c->levels != 0 || c->fshape != PFDTD_SWEEP_AUTO) return false;
-  if (c->precision == PFDTD_F16_DIFF) return false;
-  const uint64_t esz = elem_size(c->precision);
-  return fused_eligible(c) && (uint64_t)c->X * (uint64_t)c->Y * esz < (1ull << 31);
+  if (precision == PFDTD_F16_DIFF || boundary_source(c)) return false;
+  return (uint64_t)c->X * (uint64_t)c->Y * elem_size(precision) < (1ull << 31);
+}
+bool sweep_eligible(const pfdtd_ctx *c) {
+  return sweep_takes(c, c->precision) && fused_eligible(c);
+}
+
+// Fields of a run (zeroed by the caller). An interleaved batch the sweep can take is held slot by
+// slot, if its four buffers fit: 32 sources on 512x384x256 take 1.9 ms per step that way against
+// 4.27 with the single-step kernel of the interleaved layout, which reads and writes every field
+// at every step.
+int ensure_run_fields(pfdtd_ctx *c, int precision, int scale_exp, bool may_planar) {
+  const size_t bytes = elem_size(precision) * ((size_t)c->N << c->lgB);
+  const bool want = may_planar && c->lgB > 0 && !c->grouped && sweep_takes(c, precision) &&
+                    (c->planar_nomem == 0 || bytes < c->planar_nomem);
+  const bool was = c->planar;
+  c->planar = want;
+  int rc = ensure_fields(c, precision, scale_exp);
+  if (rc == PFDTD_E_NOMEM && want) {
+    c->planar_nomem = bytes;
+    c->planar = false;
+    rc = ensure_fields(c, precision, scale_exp);
+  }
+  if (c->planar != was) {
+    const int rc2 = refresh_indices(c);
+    if (rc == PFDTD_OK) rc = rc2;
+  }
+  return rc;
 }
 
 // Entry plane, air bits and events for the sweep; *ok is cleared when there is no room for them.
@@ -1358,7 +1397,7 @@ int pfdtd_prepare_fields(pfdtd_ctx *c, int precision, int scale_exp) {
   int rc = check_ctx(c);
   if (rc) return rc;
   if (!c->has_domain) return fail(PFDTD_E_STATE, "no domain set");
-  rc = ensure_fields(c, precision, scale_exp);
+  rc = ensure_run_fields(c, precision, scale_exp, true);
   if (rc) return rc;
   if (precision == PFDTD_F16 || precision == PFDTD_BF16 || precision == PFDTD_F16_DIFF)
     c->scale_req = scale_exp;
@@ -1431,7 +1470,7 @@ int pfdtd_run(pfdtd_ctx *c, int precision, int n_steps, pfdtd_interrupt_cb inter
   if (rc) return rc;
   const int scale = (precision == PFDTD_F16 || precision == PFDTD_BF16 ||
                      precision == PFDTD_F16_DIFF) ? c->scale_req : 0;
-  rc = ensure_fields(c, precision, scale);
+  rc = ensure_run_fields(c, precision, scale, true);
   if (rc) return rc;
   const bool diff = precision == PFDTD_F16_DIFF;
   if (diff && (!fused_eligible(c) || c->scheme != 0 || c->X % 2 != 0 || c->lgB > 0 ||
@@ -1593,7 +1632,7 @@ int pfdtd_begin_steps(pfdtd_ctx *c, int precision, int n_steps) {
   rc = check_runnable(c);
   if (rc) return rc;
   const int scale = (precision == PFDTD_F16 || precision == PFDTD_BF16) ? c->scale_req : 0;
-  rc = ensure_fields(c, precision, scale);
+  rc = ensure_run_fields(c, precision, scale, false);
   if (rc) return rc;
   rc = zero_fields(c);
   if (rc) return rc;
@@ -1822,6 +1861,30 @@ int pfdtd_get_fields_raw(pfdtd_ctx *c, void *p_out, void *p_past_out, int64_t ca
   if (!c->d_P) return fail(PFDTD_E_STATE, "fields not prepared");
   if (capacity_bytes < (int64_t)c->field_bytes) return fail(PFDTD_E_ARG, "output buffer too small");
   HIP_TRY(hipStreamSynchronize(c->stream));
+  if (c->planar && c->lgB > 0) {
+    // [slot][voxel] to [voxel][slot], staged through a buffer of whole voxels
+    const size_t es = elem_size(c->precision), vox = es << c->lgB;
+    const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(c->N, (int64_t)((64u << 20) / vox)));
+    void *d_tmp = nullptr;
+    if (hipMalloc(&d_tmp, (size_t)chunk * vox) != hipSuccess) {
+      (void)hipGetLastError();
+      return fail(PFDTD_E_NOMEM, "no room to interleave the fields");
+    }
+    hipError_t e = hipSuccess;
+    for (int f = 0; f < 2; ++f) {
+      char *out = (char *)(f ? p_past_out : p_out);
+      const void *src = f ? c->d_Pp : c->d_P;
+      for (int64_t v = 0; out && v < c->N && e == hipSuccess; v += chunk) {
+        const int64_t n = std::min(chunk, c->N - v);
+        e = launch_interleave((int)es, src, c->N, v, n, 1 << c->lgB, d_tmp, c->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+        if (e == hipSuccess) e = hipMemcpy(out + (size_t)v * vox, d_tmp, (size_t)n * vox, hipMemcpyDeviceToHost);
+      }
+    }
+    (void)hipFree(d_tmp);
+    if (e != hipSuccess) return fail(PFDTD_E_HIP, "interleaved fields: %s", hipGetErrorString(e));
+    return PFDTD_OK;
+  }
   if (p_out) HIP_TRY(hipMemcpy(p_out, c->d_P, c->field_bytes, hipMemcpyDeviceToHost));
   if (p_past_out) HIP_TRY(hipMemcpy(p_past_out, c->d_Pp, c->field_bytes, hipMemcpyDeviceToHost));
   return PFDTD_OK;
@@ -1908,7 +1971,11 @@ int pfdtd_set_batch(pfdtd_ctx *c, int slots) {
   if (slots < 1 || slots > 256 || (1 << lg) != slots)
     return fail(PFDTD_E_ARG, "batch width %d is not a power of two in 1..256", slots);
   HIP_TRY(hipStreamSynchronize(c->stream));
-  if (lg != c->lgB) free_fields(c);
+  if (lg != c->lgB) {
+    free_fields(c);
+    c->planar = false;
+    c->planar_nomem = 0;
+  }
   c->lgB = lg;
   for (int32_t &s : c->src_slot) s = 0;
   for (int32_t &r : c->rec_slot) r = 0;
@@ -1921,7 +1988,10 @@ int pfdtd_set_batch_layout(pfdtd_ctx *c, int layout) {
   if (layout != PFDTD_BATCH_INTERLEAVED && layout != PFDTD_BATCH_GROUPED)
     return fail(PFDTD_E_ARG, "batch layout %d not INTERLEAVED (0) or GROUPED (1)", layout);
   HIP_TRY(hipStreamSynchronize(c->stream));
-  if (layout != c->grouped) free_fields(c);
+  if (layout != c->grouped) {
+    free_fields(c);
+    c->planar = false;
+  }
   c->grouped = layout;
   return refresh_indices(c);
 }

@@ -101,3 +101,35 @@ def test_changed_domain_sources_and_precision(gpu):
             s.set_receivers(sc.rec_xyz[::-1].copy())
             s.run(sc.n_steps, prec)
             assert np.array_equal(s.responses()[::-1], t.responses())
+
+
+@pytest.mark.parametrize("prec", list(OWNED))
+@pytest.mark.parametrize("B,dims", [(2, (121, 39, 11)), (16, (50, 44, 9))])
+def test_interleaved_batch_agrees_with_grouped_and_steps(gpu, prec, B, dims):
+    """The default (interleaved) layout, whose runs hold the slots one after another: responses,
+    interleaved raw fields, and step calls before and after a run."""
+    sc = scene(970, dims, 13, n_src=B, n_rec=2 * B)
+    raw = {N.F32: np.float32, N.F64: np.float64, N.F16: np.float16, N.BF16: np.uint16}[prec]
+    scale = 9 if prec in (N.F16, N.BF16) else 0
+    out = []
+    for layout in (N.BATCH_INTERLEAVED, N.BATCH_GROUPED):
+        with Solver() as s:
+            s.load_scene(sc)
+            s.set_batch_layout(layout)
+            s.set_batch(B)
+            s.set_source_slots(np.arange(B))
+            s.set_receiver_slots(np.arange(2 * B) % B)
+            s.prepare_fields(prec, scale)
+            for _ in range(2):
+                s.run(sc.n_steps, prec)
+                r, (P, Pp) = s.responses(), s.fields_raw(raw)
+                s.begin_steps(sc.n_steps, prec)
+                for k in range(sc.n_steps):
+                    s.step(k)
+                assert np.array_equal(s.responses(), r)
+            if layout == N.BATCH_INTERLEAVED:
+                P, Pp = np.moveaxis(P, -1, 0), np.moveaxis(Pp, -1, 0)
+            out.append((r, P, Pp))
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+    assert all(f.any() for f in out[0][1])  # every slot holds its own source
