@@ -765,51 +765,20 @@ hipError_t grow(T *&p, size_t &cap, size_t need) {
   return e;
 }
 
-// Sources and receivers of the sweep's wave tiles: a source belongs to every tile whose window
-// covers it (the levels below the last are computed there too), a receiver to the tile that owns
-// it; per tile by slice, the receivers of a slice before its sources, each in index order.
+// Sources and receivers of the sweep's wave tiles.
 int build_sweep_events(pfdtd_ctx *c, const SweepPlan &p) {
-  const int slots = batch_slots(c);
-  const int nty = p.nby * p.wy, ntile = nty * p.nbx;
-  struct Ev {
-    int tile, z, x, y, id;
-  };
-  std::vector<Ev> ev;
-  auto add = [&](const int32_t *q, int slot, int id, int bx, int by, int row) {
-    ev.push_back(Ev{slot * ntile + (by * p.wy + row / p.ty) * p.nbx + bx, q[2], q[0], q[1], id});
-  };
+  std::vector<SweepPoint> rec, src;
   for (int r = 0; r < c->n_rec; ++r) {
     const int32_t *q = &c->rec_xyz[3 * r];
-    if (lin_idx(c, q) < 0) continue;
-    const int bx = q[0] / p.ox, by = q[1] / p.oy;
-    add(q, c->rec_slot[r], (int)((uint32_t)r | 0x80000000u), bx, by, q[1] - by * p.oy + p.lm);
+    if (lin_idx(c, q) >= 0)
+      rec.push_back(SweepPoint{q[0], q[1], q[2], c->rec_slot[r], (int32_t)((uint32_t)r | 0x80000000u)});
   }
   for (int s = 0; s < c->n_src; ++s) {
     const int32_t *q = &c->src_xyz[3 * s];
-    if (lin_idx(c, q) < 0) continue;
-    for (int by = std::max(0, (q[1] - p.lm) / p.oy - 1); by < p.nby; ++by) {
-      const int row = q[1] - by * p.oy + p.lm;
-      if (row < 0) break;
-      if (row >= p.wy * p.ty) continue;
-      for (int bx = std::max(0, (q[0] - p.hx) / p.ox - 1); bx < p.nbx; ++bx) {
-        const int col = q[0] - bx * p.ox + p.hx;
-        if (col < 0) break;
-        if (col < p.w) add(q, c->src_slot[s], s, bx, by, row);
-      }
-    }
+    if (lin_idx(c, q) >= 0) src.push_back(SweepPoint{q[0], q[1], q[2], c->src_slot[s], s});
   }
-  std::stable_sort(ev.begin(), ev.end(), [](const Ev &a, const Ev &b) {
-    return a.tile != b.tile ? a.tile < b.tile : a.z < b.z;
-  });
-  std::vector<int32_t> ptr((size_t)slots * ntile + 1, 0), data(4 * ev.size());
-  for (size_t i = 0; i < ev.size(); ++i) {
-    ++ptr[(size_t)ev[i].tile + 1];
-    data[4 * i] = ev[i].z;
-    data[4 * i + 1] = ev[i].x;
-    data[4 * i + 2] = ev[i].y;
-    data[4 * i + 3] = ev[i].id;
-  }
-  for (size_t i = 1; i < ptr.size(); ++i) ptr[i] += ptr[i - 1];
+  std::vector<int32_t> ptr, data;
+  sweep_events(p, batch_slots(c), rec, src, ptr, data);
   HIP_TRY(grow(c->d_ev_ptr, c->ev_ptr_cap, ptr.size()));
   HIP_TRY(grow(c->d_events, c->ev_cap, std::max<size_t>(data.size(), 4)));
   HIP_TRY(hipStreamSynchronize(c->stream));
@@ -889,9 +858,10 @@ int ensure_sweep(pfdtd_ctx *c, const SweepPlan &p, bool *ok) {
 }
 
 template <typename S, typename CT, typename C>
-SweepArgs<S, CT, C> sweep_args(const pfdtd_ctx *c, const CT *coef, CT air, C lam2, const C *sig,
+SweepArgs<S, CT, C> sweep_args(const pfdtd_ctx *c, const SweepPlan &p, const CT *coef, CT air, C lam2, const C *sig,
                                int step, int inject_end) {
   SweepArgs<S, CT, C> a{};
+  sweep_geometry(p, a);
   a.pm = c->d_entry;
   a.row_bits = c->d_row_bits;
   a.ev_ptr = c->d_ev_ptr;
@@ -930,11 +900,11 @@ hipError_t run_sweep(pfdtd_ctx *c, const SweepPlan &p, int step, int levels, int
   hipError_t e;
   auto args = [&](auto tag) {
     typedef decltype(tag) S;
-    return sweep_args<S>(c, c->d_coef_f, c->air_f, c->lam2_f, c->d_sig_f, step, inject_end);
+    return sweep_args<S>(c, p, c->d_coef_f, c->air_f, c->lam2_f, c->d_sig_f, step, inject_end);
   };
   switch (c->precision) {
   case PFDTD_F64:
-    e = launch_sweep_f64(p, sweep_args<double>(c, c->d_coef_d, c->air_d, c->lam2_d, c->d_sig_d,
+    e = launch_sweep_f64(p, sweep_args<double>(c, p, c->d_coef_d, c->air_d, c->lam2_d, c->d_sig_d,
                                                step, inject_end), levels, c->stream);
     break;
   case PFDTD_F16: e = launch_sweep_f16(p, args(h16{}), levels, c->stream); break;
@@ -1509,7 +1479,7 @@ int pfdtd_run(pfdtd_ctx *c, int precision, int n_steps, pfdtd_interrupt_cb inter
   bool fused = !sweep && fused_eligible(c);
   rc = ensure_pm(c, &fused);
   if (rc) return rc;
-  const FusedGeom fg = plan_fused((int)c->X, (int)c->Y, (int)c->Z, c->fzc, c->precision, false,
+  const FusedGeom fg = plan_fused((int)c->X, (int)c->Y, (int)c->Z, c->fzc, c->precision,
                                   diff ? PFDTD_SWEEP_PAIR : c->fshape, c->scheme, batch_slots(c));
   if (diff && (!fused || !fg.pair))
     return fail(PFDTD_E_NOMEM, "no room for the packed plane the two-column sweep reads");
@@ -1689,7 +1659,7 @@ int pfdtd_steps(pfdtd_ctx *c, int first_step, int n_steps) {
   bool fused = !sweep && fused_eligible(c);
   rc = ensure_pm(c, &fused);
   if (rc) return rc;
-  const FusedGeom fg = plan_fused((int)c->X, (int)c->Y, (int)c->Z, c->fzc, c->precision, false,
+  const FusedGeom fg = plan_fused((int)c->X, (int)c->Y, (int)c->Z, c->fzc, c->precision,
                                   c->fshape, c->scheme, batch_slots(c));
   const bool three = fused && c->scheme == 0 && levels_for(c, c->precision) == 3;
   FusedGeom fg3;

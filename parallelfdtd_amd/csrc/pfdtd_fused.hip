@@ -22,9 +22,6 @@
 // P^{n+1} rows of a slice are all marked takes the air value instead of loading the packed
 // plane -- the value it would have loaded, so the results do not change.
 //
-// The same kernel serves two callers: a context's domain (POOL = false) and the two-level jobs
-// of one serving-pool launch (POOL = true: the block finds its job in the launch table and takes
-// its arguments from the job descriptor; a job with one step left runs only the first level).
 // SCHEME selects the boundary formulation of a context's domain: forward (Bilbao, update types
 // SRL_FORWARD and SHARED) or centred (Kowalczyk, update type SRL).
 //
@@ -166,8 +163,7 @@ static int fused_ty_host(int precision, int scheme) {
 // buffer set, five allocation offsets: FP64 forward 0.8-5.6 % faster, FP32 centred 0.8-6 %
 // faster (2 x 1 blocks: FP64 1.2-2.4 %); FP64 centred within 2 % either way. The 16-bit sweep is
 // not bound by HBM traffic: every wider block (2 x 2, 2 x 4, 4 x 2, 4 x 4) was 1-24 % slower
-// than the column, 6 % with the centred scheme. Serving-pool launches (small rooms) use the
-// column.
+// than the column, 6 % with the centred scheme.
 template <int SHAPE>
 struct FusedShape {
   static constexpr int WX = SHAPE == kWideBlocks ? 4 : SHAPE == kSquareBlocks ? 2 : 1;
@@ -178,19 +174,12 @@ constexpr int fused_waves() {
   return FusedShape<SHAPE>::WX * FusedShape<SHAPE>::WY;
 }
 
-// Kernel arguments: one context's domain, or the two-level jobs of one serving-pool launch.
+// Kernel arguments.
 template <typename S, typename CT, typename C>
 struct Fused2Ctx {
   Fused2Args<S, CT, C> a;
   int X, Y, Z, zc;
 };
-struct Fused2Pool {
-  const PoolJobDev *jobs;
-  const PoolState *state;
-  PoolLaunch L;
-  int zc;
-};
-
 // Four waves per SIMD (at most 128 VGPRs) for the forward update with FP32 and 16-bit storage;
 // FP64 and the centred update (six separate neighbours per node) need more registers.
 template <typename S, int SCHEME>
@@ -201,9 +190,9 @@ constexpr int fused_min_waves() {
 // SCHEME 0: forward (Bilbao) boundaries, update types SRL_FORWARD and SHARED; SCHEME 2: the
 // centred (Kowalczyk) boundaries of update type SRL, through the same `centred_node` as the
 // single-step kernel (the reference's operation order).
-template <typename S, typename CT, typename C, bool POOL, int SHAPE, int SCHEME>
+template <typename S, typename CT, typename C, int SHAPE, int SCHEME>
 __global__ __launch_bounds__((64 * fused_waves<SHAPE>()), (fused_min_waves<S, SCHEME>())) void srl_update2_kernel(
-    typename std::conditional<POOL, Fused2Pool, Fused2Ctx<S, CT, C>>::type p) {
+    Fused2Ctx<S, CT, C> p) {
 #pragma clang fp contract(off)
   constexpr int kFTY = fused_ty<S, SCHEME>();
   constexpr int WX = FusedShape<SHAPE>::WX, WY = FusedShape<SHAPE>::WY, kFWaves = WX * WY;
@@ -218,87 +207,25 @@ __global__ __launch_bounds__((64 * fused_waves<SHAPE>()), (fused_min_waves<S, SC
   // XCD-aware tile order: consecutive block ids are dealt round-robin to the 8 XCDs (each with
   // its own L2); remapping them so that every XCD walks a contiguous run of x-fastest tiles keeps
   // the halo columns and rows that neighbouring tiles share in one L2 while both are resident.
-  Fused2Args<S, CT, C> a;
-  int X, Y, Z, zc, bxi, byi, bzi;
-  bool two = true;  // second time level (a pool job with one step left takes only the first)
-  int slot = 0;
-  if constexpr (!POOL) {
-    a = p.a;
-    X = p.X;
-    Y = p.Y;
-    Z = p.Z;
-    zc = p.zc;
-    const unsigned nx = gridDim.x, ny = gridDim.y, total = nx * ny * gridDim.z;
-    const unsigned lin = blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z);
-    const unsigned full = total & ~7u;
-    unsigned tile = lin < full ? (lin & 7u) * (full >> 3) + (lin >> 3) : lin;
-    // grouped batch: the slots of one spatial tile are consecutive, so one XCD's L2 serves
-    // the tile's packed plane and air-row bits to all of them
-    slot = (int)(tile % (unsigned)a.n_slots);
-    tile /= (unsigned)a.n_slots;
-    bxi = (int)(tile % nx);
-    byi = (int)((tile / nx) % ny);
-    bzi = (int)(tile / (nx * ny));
-    if (slot) {
-      const int64_t off = (int64_t)slot * a.slot_elems;
-      a.A += off;
-      a.B += off;
-      a.Cn += off;
-      a.Dn += off;
-    }
-  } else {
-    // the flattened tiles of every job of the launch; the block finds its job by a binary
-    // search over the launch table's cumulative tile counts
-    const unsigned total = gridDim.x, lin = blockIdx.x, full = total & ~7u;
-    const int tile = (int)(lin < full ? (lin & 7u) * (full >> 3) + (lin >> 3) : lin);
-    int lo = 0, hi = p.L.n - 1;
-    while (lo < hi) {
-      const int mid = (lo + hi) >> 1;
-      if (p.L.tile_end[mid] > tile)
-        hi = mid;
-      else
-        lo = mid + 1;
-    }
-    const PoolJobDev &J = p.jobs[p.L.slot[lo]];
-    const PoolState st = p.state[p.L.slot[lo]];
-    const int remaining = J.n_steps - st.step;
-    if (remaining <= 0) return;  // the whole block: no barrier has been reached
-    two = remaining >= 2;
-    int o1, o2;
-    pool_spare(st.cur, st.past, o1, o2);
-    a.pm = J.pm;
-    a.air_rows = J.air_rows;
-    a.A = (const S *)J.F[st.cur];
-    a.B = (const S *)J.F[st.past];
-    a.Cn = (S *)J.F[o1];
-    a.Dn = (S *)J.F[o2];
-    a.coef = J.coef;
-    a.ncol = J.ncol;
-    a.air = J.air;
-    a.air_uniform = J.air_uniform;
-    a.lam2 = J.lam2;
-    a.src_xyz = J.src_xyz;
-    a.src_kind = J.src_kind;
-    a.n_src = J.n_src;
-    a.sig_f = J.sig;
-    a.sig_d = nullptr;
-    a.n_samples = J.n_samples;
-    a.inject_step = (J.n_src > 0 && st.step + 1 < J.n_steps) ? st.step + 1 : -1;
-    a.soft_overwrite = J.soft_overwrite;
-    a.scale_exp = J.scale_exp;
-    a.rec_xyz = J.rec_xyz;
-    a.n_rec = J.n_rec;
-    a.resp = J.resp;
-    a.resp_steps = J.n_steps;
-    a.gather_step = st.step;
-    X = J.X;
-    Y = J.Y;
-    Z = J.Z;
-    zc = p.zc;
-    const int t = tile - (lo ? p.L.tile_end[lo - 1] : 0);
-    bxi = t % J.fx;
-    byi = (t / J.fx) % J.fy;
-    bzi = t / (J.fx * J.fy);
+  Fused2Args<S, CT, C> a = p.a;
+  const int X = p.X, Y = p.Y, Z = p.Z, zc = p.zc;
+  const unsigned nx = gridDim.x, ny = gridDim.y, total = nx * ny * gridDim.z;
+  const unsigned lin = blockIdx.x + nx * (blockIdx.y + ny * blockIdx.z);
+  const unsigned full = total & ~7u;
+  unsigned tile = lin < full ? (lin & 7u) * (full >> 3) + (lin >> 3) : lin;
+  // grouped batch: the slots of one spatial tile are consecutive, so one XCD's L2 serves
+  // the tile's packed plane and air-row bits to all of them
+  const int slot = (int)(tile % (unsigned)a.n_slots);
+  tile /= (unsigned)a.n_slots;
+  const int bxi = (int)(tile % nx);
+  const int byi = (int)((tile / nx) % ny);
+  const int bzi = (int)(tile / (nx * ny));
+  if (slot) {
+    const int64_t off = (int64_t)slot * a.slot_elems;
+    a.A += off;
+    a.B += off;
+    a.Cn += off;
+    a.Dn += off;
   }
   const int xt = bxi * WX + wave % WX;  // this wave's x tile
   const int xb = xt * kFO;  // first owned column
@@ -550,7 +477,7 @@ __global__ __launch_bounds__((64 * fused_waves<SHAPE>()), (fused_min_waves<S, SC
     }
 
     // ---- second time level: P^{n+2}[k-1] on the owned rows
-    if (two && k - 1 >= z0) {
+    if (k - 1 >= z0) {
       const auto rD = slice_rsrc(gD + (size_t)(k - 1) * XY, sbytes);
       auto level2 = [&](auto table) {
 #pragma unroll
@@ -1878,7 +1805,7 @@ hipError_t launch_air_rows(const uint16_t *pm, uint32_t *rows, int X, int Y, int
   return hipGetLastError();
 }
 
-FusedGeom plan_fused(int X, int Y, int Z, int zc, int precision, bool pool, int shape,
+FusedGeom plan_fused(int X, int Y, int Z, int zc, int precision, int shape,
                      int scheme, int slots) {
   const int kFTY = fused_ty_host(precision, scheme);
   FusedGeom g;
@@ -1892,14 +1819,14 @@ FusedGeom plan_fused(int X, int Y, int Z, int zc, int precision, bool pool, int 
   // with the forward scheme and for FP32 with the centred one
   g.scheme = scheme;
   g.blocks = kColumnBlocks;
-  if (!pool && precision == 0 && scheme == 0 &&
+  if (precision == 0 && scheme == 0 &&
       (shape == PFDTD_SWEEP_WIDE || (shape == PFDTD_SWEEP_AUTO && ntx >= 16)))
     g.blocks = kWideBlocks;
-  else if (!pool && shape == PFDTD_SWEEP_AUTO && ntx >= 16 &&
+  else if (shape == PFDTD_SWEEP_AUTO && ntx >= 16 &&
            ((precision == 1 && scheme == 0) || (precision == 0 && scheme == 2)))
     g.blocks = kSquareBlocks;
   // 16-bit storage, forward scheme, X even, slices under 2^31 bytes: two columns per lane
-  g.pair = !pool && precision >= 2 && scheme == 0 && X % 2 == 0 &&
+  g.pair = precision >= 2 && scheme == 0 && X % 2 == 0 &&
            (int64_t)X * Y * 2 < (int64_t)kDropShift &&
            (shape == PFDTD_SWEEP_AUTO || shape == PFDTD_SWEEP_PAIR);
   if (g.pair) {
@@ -1965,56 +1892,31 @@ static hipError_t launch_fused(const FusedGeom &g, const Fused2Args<S, CT, C> &a
   if (g.scheme == 2) {
     if constexpr (std::is_same<S, float>::value) {
       if (g.blocks == kSquareBlocks) {
-        hipLaunchKernelGGL((srl_update2_kernel<S, CT, C, false, kSquareBlocks, 2>), g.grid,
+        hipLaunchKernelGGL((srl_update2_kernel<S, CT, C, kSquareBlocks, 2>), g.grid,
                            g.block, lds, stream, p);
         return hipGetLastError();
       }
     }
-    hipLaunchKernelGGL((srl_update2_kernel<S, CT, C, false, kColumnBlocks, 2>), g.grid, g.block,
+    hipLaunchKernelGGL((srl_update2_kernel<S, CT, C, kColumnBlocks, 2>), g.grid, g.block,
                        lds, stream, p);
     return hipGetLastError();
   }
   if constexpr (std::is_same<S, float>::value) {
     if (g.blocks == kWideBlocks) {
-      hipLaunchKernelGGL((srl_update2_kernel<S, CT, C, false, kWideBlocks, 0>), g.grid, g.block,
+      hipLaunchKernelGGL((srl_update2_kernel<S, CT, C, kWideBlocks, 0>), g.grid, g.block,
                          lds, stream, p);
       return hipGetLastError();
     }
   }
   if constexpr (std::is_same<S, double>::value) {
     if (g.blocks == kSquareBlocks) {
-      hipLaunchKernelGGL((srl_update2_kernel<S, CT, C, false, kSquareBlocks, 0>), g.grid,
+      hipLaunchKernelGGL((srl_update2_kernel<S, CT, C, kSquareBlocks, 0>), g.grid,
                          g.block, lds, stream, p);
       return hipGetLastError();
     }
   }
-  hipLaunchKernelGGL((srl_update2_kernel<S, CT, C, false, kColumnBlocks, 0>), g.grid, g.block,
+  hipLaunchKernelGGL((srl_update2_kernel<S, CT, C, kColumnBlocks, 0>), g.grid, g.block,
                      lds, stream, p);
-  return hipGetLastError();
-}
-
-hipError_t launch_pool_update2(int precision, int tiles, const PoolJobDev *jobs,
-                               const PoolState *st, const PoolLaunch &L, int zc,
-                               hipStream_t stream) {
-  const Fused2Pool p{jobs, st, L, zc};
-  const size_t lds = sizeof(CoefF) * kStageRows * (size_t)L.ncol_max;
-  const dim3 grid((unsigned)tiles);
-  switch (precision) {
-  case PFDTD_F32:
-    hipLaunchKernelGGL((srl_update2_kernel<float, CoefF, float, true, kColumnBlocks, 0>), grid,
-                       dim3(64 * fused_waves<kColumnBlocks>()), lds, stream, p);
-    break;
-  case PFDTD_F16:
-    hipLaunchKernelGGL((srl_update2_kernel<h16, CoefF, float, true, kColumnBlocks, 0>), grid,
-                       dim3(64 * fused_waves<kColumnBlocks>()), lds, stream, p);
-    break;
-  case PFDTD_BF16:
-    hipLaunchKernelGGL((srl_update2_kernel<b16, CoefF, float, true, kColumnBlocks, 0>), grid,
-                       dim3(64 * fused_waves<kColumnBlocks>()), lds, stream, p);
-    break;
-  default:
-    return hipErrorInvalidValue;
-  }
   return hipGetLastError();
 }
 

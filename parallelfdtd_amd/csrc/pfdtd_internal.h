@@ -74,16 +74,15 @@ struct UpdateArgs {
   int scheme;  // 0 forward (Bilbao) boundaries, 2 centred (Kowalczyk) boundaries
 };
 
-// ---- serving pool (pfdtd_pool.hip; the two-level pool launch lives in pfdtd_fused.hip)
+// ---- serving pool (pfdtd_pool.hip; the sweep over its jobs lives in pfdtd_sweep.hip)
 constexpr int kPoolMaxJobs = 64;
+constexpr int kPoolLevels = 5;  // steps per round: the levels of the sweep's FP32 and 16-bit tiles
 
 // One resident job. Field buffers F[0..3]: jobs advanced by single steps use F[0] and F[1];
-// jobs advanced by the two-level sweep (fused != 0) own all four.
+// jobs advanced by the several-level sweep own all four.
 struct PoolJobDev {
   const uint8_t *pos;
   const uint8_t *mat;
-  const uint16_t *pm;  // pos | mat << 8 (two-level jobs)
-  const uint32_t *air_rows;  // air-row bits of the two-level wave tiles (two-level jobs)
   void *F[4];
   const CoefF *coef;
   int ncol;  // material columns of the table the job's domain addresses (its n_mat)
@@ -92,13 +91,9 @@ struct PoolJobDev {
   float lam2;
   int X, Y, Z;
   int gx, gy;      // single-step tiles along x and y (z tiles follow from the tile count)
-  int fx, fy;      // two-level tiles along x and y
-  int fused;       // advanced by the two-level sweep
   const int64_t *rec_idx;
-  const int32_t *rec_xyz;
   double *resp;  // [n_rec][n_steps]
   const int64_t *src_idx;
-  const int32_t *src_xyz;
   const int32_t *src_kind;
   const float *sig;  // [n_src][n_samples]
   int n_rec, n_src, n_samples, n_steps;
@@ -133,14 +128,6 @@ struct PoolLaunch {
   int slot[kPoolMaxJobs];
   int tile_end[kPoolMaxJobs];
 };
-
-// Two-level sweep of every job of a launch (two steps, or one for a job with one step left),
-// then per job: gather/inject of the second step and the buffer rotation.
-hipError_t launch_pool_update2(int precision, int tiles, const PoolJobDev *jobs,
-                               const PoolState *st, const PoolLaunch &L, int zc,
-                               hipStream_t stream);
-hipError_t launch_pool_inject2(int precision, const PoolJobDev *jobs, PoolState *st,
-                               const PoolLaunch &L, hipStream_t stream);
 
 // Launchers (all asynchronous on `stream`; return the launch status).
 hipError_t launch_update_f32(const UpdateGeom &g, const UpdateArgs<float, CoefF, float> &a,
@@ -207,10 +194,10 @@ struct FusedGeom {
   int scheme;  // 0 forward boundaries, 2 centred
   dim3 grid, block;
 };
-// Grid of the two-level sweep; `pool`: serving-pool launches (1 x 4 blocks); `shape`: one of
-// PFDTD_SWEEP_AUTO / _COLUMN / _WIDE; `scheme`: 0 forward, 2 centred boundaries.
-FusedGeom plan_fused(int X, int Y, int Z, int zc, int precision, bool pool = false,
-                     int shape = 0, int scheme = 0, int slots = 1);
+// Grid of the two-level sweep; `shape`: one of PFDTD_SWEEP_AUTO / _COLUMN / _WIDE; `scheme`: 0
+// forward, 2 centred boundaries.
+FusedGeom plan_fused(int X, int Y, int Z, int zc, int precision, int shape = 0, int scheme = 0,
+                     int slots = 1);
 // Grid of the three-level sweep (forward scheme): 58-column, 4-row wave tiles in blocks of
 // 2 x 2 tiles, or (`shape` PFDTD_SWEEP_COLUMN) 1 x 4.
 FusedGeom plan_fused3(int X, int Y, int Z, int zc, int precision, int shape, int slots = 1);
@@ -284,17 +271,46 @@ struct SweepPlan {
   int64_t blocks;
 };
 SweepPlan plan_sweep(int precision, int X, int Y, int Z, int zc, int slots);
+// Fills the tile geometry of a sweep's arguments.
+template <typename A>
+void sweep_geometry(const SweepPlan &p, A &a) {
+  a.pitch = p.pitch;
+  a.air_words = p.words;
+  a.zc = p.zc;
+  a.nbx = p.nbx;
+  a.nby = p.nby;
+  a.band = p.band;
+}
+int sweep_zchunk(int n, const int64_t *bxy, const int *zi, int levels);
+// A source or receiver as the sweep's event lists take it.
+struct SweepPoint {
+  int32_t x, y, z, slot, id;  // id: source index, or receiver index | 1 << 31
+};
+// Events by wave tile (ptr: n_slots * nby * wy * nbx + 1 entries) and slice (data: four ints each):
+// a source belongs to every tile whose window covers it (the levels below the last are computed
+// there too), a receiver to the tile that owns it; per tile by slice, the receivers of a slice
+// before its sources, each in index order.
+void sweep_events(const SweepPlan &p, int slots, const std::vector<SweepPoint> &rec,
+                  const std::vector<SweepPoint> &src, std::vector<int32_t> &ptr,
+                  std::vector<int32_t> &data);
+// One round of a serving-pool bundle (SweepPlan::lm steps of every job), and the states' rotation
+// after its last one. args: SweepArgs of the storage type by job slot.
+hipError_t launch_sweep_pool(int precision, int tiles, const void *args, const PoolJobDev *jobs,
+                             const PoolState *st, const PoolLaunch &pl, int zc, int round,
+                             hipStream_t stream);
+hipError_t launch_pool_rotate(const PoolJobDev *jobs, PoolState *st, const PoolLaunch &pl,
+                              int rounds, int levels, hipStream_t stream);
 hipError_t launch_pack_entry(const uint8_t *pos, const uint8_t *mat, uint16_t *pm, int X, int Y,
                              int Z, int pitch, int ncol, hipStream_t stream);
 hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint64_t *out, int X, int Y,
                            int Z, int ncol, hipStream_t stream);
-hipError_t launch_sweep_f32(const SweepPlan &p, SweepArgs<float, CoefF, float> a, int levels,
+hipError_t launch_sweep_f32(const SweepPlan &p, const SweepArgs<float, CoefF, float> &a, int levels,
                             hipStream_t stream);
-hipError_t launch_sweep_f16(const SweepPlan &p, SweepArgs<h16, CoefF, float> a, int levels,
+hipError_t launch_sweep_f16(const SweepPlan &p, const SweepArgs<h16, CoefF, float> &a, int levels,
                             hipStream_t stream);
-hipError_t launch_sweep_bf16(const SweepPlan &p, SweepArgs<b16, CoefF, float> a, int levels,
+hipError_t launch_sweep_bf16(const SweepPlan &p, const SweepArgs<b16, CoefF, float> &a, int levels,
                              hipStream_t stream);
-hipError_t launch_sweep_f64(const SweepPlan &p, SweepArgs<double, CoefD, double> a, int levels,
+hipError_t launch_sweep_f64(const SweepPlan &p, const SweepArgs<double, CoefD, double> &a, int levels,
                             hipStream_t stream);
 
 // Voxels v0 .. v0 + n - 1 of a slot-major batch (element slot * N + voxel, elem_bytes each) to

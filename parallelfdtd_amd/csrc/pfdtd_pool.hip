@@ -1,20 +1,20 @@
 // pfdtd_pool.hip -- serving pool: many independent impulse-response jobs (rooms of different
 // sizes, FP32 / FP16 / BF16 storage) resident in one HBM arena and advanced together.
 //
-// Device side. Every resident job has a descriptor (PoolJobDev: its buffers, dimensions,
-// coefficients, sources and receivers) and a state (step, current buffer, past buffer) in device
-// memory, indexed by the job's slot. Jobs are advanced in rounds of two steps. A job whose
-// sources avoid the never-updated first and last z slices owns four field buffers and is
-// advanced by the two-level sweep (srl_update2_kernel in pool mode, pfdtd_fused.hip): ONE launch
-// per storage type enumerates the sweep tiles of every such job (a block finds its job by a
-// binary search over the launch table's tile prefix) and does two steps per job, or one for a
-// job with a single step left; pool_inject2_kernel (one block per job) then gathers and injects
-// the second step and rotates the buffer roles. Other jobs take two single steps per round:
-// pool_update_kernel (flattened single-step tiles) and pool_inject_kernel, which gathers,
-// injects the next samples and swaps current and past. Because the kernels read the state from
-// device memory, a bundle of rounds is replay-invariant: it is captured once into a hipGraph per
-// membership of the pool and replayed until a job joins or leaves. A job whose last step is
-// done is skipped by the kernels until the host drops it from the launch.
+// Device side. Every resident job has a descriptor (PoolJobDev: its buffers, sources and
+// receivers), a state (step, current buffer, past buffer) and, for the several-level sweep, the
+// sweep's arguments in device memory, indexed by the job's slot. Jobs are advanced in rounds of
+// kPoolLevels steps. A job whose sources avoid the never-updated first and last z slices owns four
+// field buffers and is advanced by the sweep (srl_sweep_pool_kernel, pfdtd_sweep.hip): ONE launch
+// per storage type and round enumerates the tiles of every such job (a block finds its job by a
+// binary search over the launch table's tile prefix), gathers and injections included; the steps
+// that do not fill a round are taken when the job is admitted. After the rounds of a bundle one
+// small kernel sets the jobs' steps and buffers. Other jobs take single steps: pool_update_kernel
+// (flattened single-step tiles) and pool_inject_kernel, which gathers, injects the next samples
+// and swaps current and past. Because the kernels read the state from device memory, a bundle is
+// replay-invariant: it is captured once into a hipGraph per membership of the pool and replayed
+// until a job joins or leaves. A job whose last step is done is skipped by the kernels until the
+// host drops it from the launch.
 //
 // Host side. Jobs are admitted (pfdtd_pool_submit) only when their buffers fit in the arena's
 // free space and a slot is free; the arena is one allocation made at pool creation, so
@@ -26,6 +26,7 @@
 #include "pfdtd_device.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
@@ -107,30 +108,6 @@ __global__ __launch_bounds__(256) void pool_inject_kernel(const PoolJobDev *__re
   if (threadIdx.x == 0) state[slot] = PoolState{st.step + 1, st.past, st.cur};
 }
 
-// After a two-level sweep (pool_update2 in pfdtd_fused.hip, which gathered step n and
-// injected step n+1 itself): with two steps done, gather step n+1 on P^{n+2} and inject step
-// n+2 into it; P^{n+2} and P^{n+1} (the spare buffers o2, o1) become current and past. With
-// one step done (the job's last), P^{n+1} in o1 becomes current.
-template <typename S>
-__global__ __launch_bounds__(256) void pool_inject2_kernel(const PoolJobDev *__restrict__ jobs,
-                                                           PoolState *__restrict__ state,
-                                                           PoolLaunch L) {
-  const int slot = L.slot[blockIdx.x];
-  const PoolJobDev &J = jobs[slot];
-  const PoolState st = state[slot];
-  const int remaining = J.n_steps - st.step;
-  if (remaining <= 0) return;
-  int o1, o2;
-  pool_spare(st.cur, st.past, o1, o2);
-  if (remaining >= 2) {
-    inject_gather_block<S>((S *)J.F[o2], pool_inject_args(J, st.step + 1, st.step + 2));
-    __syncthreads();
-    if (threadIdx.x == 0) state[slot] = PoolState{st.step + 2, o2, o1};
-  } else if (threadIdx.x == 0) {
-    state[slot] = PoolState{st.step + 1, o1, st.cur};
-  }
-}
-
 template <typename S>
 hipError_t launch_pool_update_t(int ry, int tiles, const PoolJobDev *jobs, const PoolState *st,
                                 const PoolLaunch &L, int zc, hipStream_t stream) {
@@ -160,18 +137,6 @@ hipError_t launch_pool_update(int precision, int ry, int tiles, const PoolJobDev
   case PFDTD_BF16: return launch_pool_update_t<b16>(ry, tiles, jobs, st, L, zc, stream);
   default: return hipErrorInvalidValue;
   }
-}
-
-hipError_t launch_pool_inject2(int precision, const PoolJobDev *jobs, PoolState *st,
-                               const PoolLaunch &L, hipStream_t stream) {
-  const dim3 grid(L.n), block(256);
-  switch (precision) {
-  case PFDTD_F32: hipLaunchKernelGGL(pool_inject2_kernel<float>, grid, block, 0, stream, jobs, st, L); break;
-  case PFDTD_F16: hipLaunchKernelGGL(pool_inject2_kernel<h16>, grid, block, 0, stream, jobs, st, L); break;
-  case PFDTD_BF16: hipLaunchKernelGGL(pool_inject2_kernel<b16>, grid, block, 0, stream, jobs, st, L); break;
-  default: return hipErrorInvalidValue;
-  }
-  return hipGetLastError();
 }
 
 hipError_t launch_pool_inject(int precision, const PoolJobDev *jobs, PoolState *st,
@@ -224,20 +189,18 @@ size_t storage_bytes(int precision) {
   }
 }
 
-// z-chunk of the two-level sweep in the pool: the C5 capacity probe (200 rooms of 64..512 per
-// side at once) sustains 479 Gvox/s with 16 slices, 480 with 8 and 460 with 32
-constexpr int kPoolFusedZc = 16;
-
-// Byte offsets of one job's buffers inside its arena block (a two-level job adds two field
-// buffers, the packed byte plane, its air-row bits and the source/receiver coordinates).
+// Byte offsets of one job's buffers inside its arena block (a job of the sweep adds two field
+// buffers, the entry plane, its row bits and its events).
 struct JobLayout {
-  size_t F[4], pos, mat, pm, air_rows, labels, coef, src_idx, src_xyz, src_kind, sig, rec_idx,
-      rec_xyz, resp, total;
+  size_t F[4], pos, mat, entry, row_bits, labels, coef, src_idx, ev_ptr, events, src_kind, sig,
+      rec_idx, resp, total;
 };
 
 JobLayout layout_job(int X, int Y, int Z, size_t es, int n_src, int n_samples, int n_rec,
-                     int n_steps, bool fused) {
+                     int n_steps, bool fused, int precision) {
   const int64_t N = (int64_t)X * Y * Z;
+  const SweepPlan sp = plan_sweep(precision, X, Y, Z, 1, 1);
+  const size_t wave_tiles = (size_t)sp.nbx * sp.nby * sp.wy;
   JobLayout L{};
   size_t o = 0;
   auto take = [&](size_t bytes) {
@@ -248,16 +211,17 @@ JobLayout layout_job(int X, int Y, int Z, size_t es, int n_src, int n_samples, i
   for (int b = 0; b < 4; ++b) L.F[b] = (b < 2 || fused) ? take(es * (size_t)N) : 0;
   L.pos = take((size_t)N);
   L.mat = take((size_t)N);
-  L.pm = fused ? take(sizeof(uint16_t) * (size_t)N) : 0;
-  L.air_rows = fused ? take(sizeof(uint32_t) * air_rows_words(X, Y, Z)) : 0;
+  L.entry = fused ? take(sizeof(uint16_t) * (size_t)sp.pitch * Y * Z) : 0;
+  L.row_bits = fused ? take(2 * sizeof(uint64_t) * wave_tiles * sp.words) : 0;
   L.labels = take((size_t)N);
   L.coef = take(sizeof(CoefF) * kCoefEntries);
   L.src_idx = take(sizeof(int64_t) * (size_t)n_src);
-  L.src_xyz = fused ? take(sizeof(int32_t) * 3 * (size_t)n_src) : 0;
+  // a source lies in the windows of at most two tiles along x and two along y
+  L.ev_ptr = fused ? take(sizeof(int32_t) * (wave_tiles + 1)) : 0;
+  L.events = fused ? take(4 * sizeof(int32_t) * ((size_t)n_rec + 4 * (size_t)n_src)) : 0;
   L.src_kind = take(sizeof(int32_t) * (size_t)n_src);
   L.sig = take(sizeof(float) * (size_t)n_src * (size_t)n_samples);
   L.rec_idx = take(sizeof(int64_t) * (size_t)n_rec);
-  L.rec_xyz = fused ? take(sizeof(int32_t) * 3 * (size_t)n_rec) : 0;
   L.resp = take(sizeof(double) * (size_t)n_rec * (size_t)n_steps);
   L.total = o;
   return L;
@@ -271,7 +235,9 @@ struct PoolJobHost {
   int precision = 0;
   int n_steps = 0, n_rec = 0;
   int64_t voxels = 0;
-  int tiles = 0;  // tiles of the job's update kernel (two-level or single-step)
+  int tiles = 0;  // tiles of the job's single-step kernel
+  int64_t bxy = 0;  // blocks of the sweep per z-chunk, and its slices
+  int zi = 0;
   bool fused = false;
   int ncol = 1;
   size_t off = 0, bytes = 0;
@@ -292,6 +258,7 @@ struct pfdtd_pool {
   std::map<size_t, size_t> free_blocks;  // offset -> size
   PoolJobDev *d_jobs = nullptr;
   PoolState *d_state = nullptr;
+  SweepArgs<float, CoefF, float> *d_args = nullptr;  // by slot; the fields come from the state
   std::vector<int64_t> slot_job;  // job id per slot, -1 free
   std::map<int64_t, PoolJobHost> jobs;
   int64_t next_id = 1;
@@ -308,8 +275,9 @@ struct pfdtd_pool {
   bool dirty = true;
   std::vector<int64_t> members;  // job ids in the current launch
   int prec_list[3] = {PFDTD_F32, PFDTD_F16, PFDTD_BF16};
-  PoolLaunch launch[3][2];  // [storage type][0 single-step jobs, 1 two-level jobs]
+  PoolLaunch launch[3][2];  // [storage type][0 single-step jobs, 1 jobs of the sweep]
   int tiles[3][2] = {{0, 0}, {0, 0}, {0, 0}};
+  int sweep_zc[3] = {1, 1, 1};
   hipGraphExec_t exec = nullptr;
   uint64_t exec_last_seq = 0;
   std::vector<std::pair<uint64_t, hipGraphExec_t>> retired;
@@ -411,30 +379,34 @@ int reap(pfdtd_pool *p, bool block) {
   return PFDTD_OK;
 }
 
-// A bundle is bundle/2 rounds; each round advances two-level jobs by one sweep (two steps, or
-// the last one) and single-step jobs by two steps.
+// Steps a bundle advances every unfinished job by.
+int bundle_steps(const pfdtd_pool *p) { return (p->bundle + kPoolLevels - 1) / kPoolLevels * kPoolLevels; }
+
+// A bundle: the rounds of the sweep (and the single steps of the other jobs), then the rotation. One
+// stream, so the captured graph is a chain: the storage types' launches follow each other.
 int enqueue_bundle_kernels(pfdtd_pool *p) {
-  for (int k = 0; k < p->bundle; k += 2) {
+  const int steps = bundle_steps(p), rounds = steps / kPoolLevels;
+  for (int k = 0; k < rounds; ++k)
     for (int q = 0; q < 3; ++q)
-      if (p->launch[q][1].n) {
-        POOL_TRY(launch_pool_update2(p->prec_list[q], p->tiles[q][1], p->d_jobs, p->d_state,
-                                     p->launch[q][1], kPoolFusedZc, p->run));
-        POOL_TRY(launch_pool_inject2(p->prec_list[q], p->d_jobs, p->d_state, p->launch[q][1],
-                                     p->run));
+      if (p->launch[q][1].n)
+        POOL_TRY(launch_sweep_pool(p->prec_list[q], p->tiles[q][1], p->d_args, p->d_jobs, p->d_state,
+                                   p->launch[q][1], p->sweep_zc[q], k, p->run));
+  for (int q = 0; q < 3; ++q)
+    if (p->launch[q][1].n)
+      POOL_TRY(launch_pool_rotate(p->d_jobs, p->d_state, p->launch[q][1], rounds, kPoolLevels, p->run));
+  for (int k = 0; k < steps; ++k)
+    for (int q = 0; q < 3; ++q)
+      if (p->launch[q][0].n) {
+        POOL_TRY(launch_pool_update(p->prec_list[q], p->ry, p->tiles[q][0], p->d_jobs, p->d_state,
+                                    p->launch[q][0], p->zc, p->run));
+        POOL_TRY(launch_pool_inject(p->prec_list[q], p->d_jobs, p->d_state, p->launch[q][0], p->run));
       }
-    for (int half = 0; half < 2; ++half)
-      for (int q = 0; q < 3; ++q)
-        if (p->launch[q][0].n) {
-          POOL_TRY(launch_pool_update(p->prec_list[q], p->ry, p->tiles[q][0], p->d_jobs,
-                                      p->d_state, p->launch[q][0], p->zc, p->run));
-          POOL_TRY(launch_pool_inject(p->prec_list[q], p->d_jobs, p->d_state, p->launch[q][0],
-                                      p->run));
-        }
-  }
   return PFDTD_OK;
 }
 
 int rebuild_membership(pfdtd_pool *p) {
+  int64_t bxy[3][kPoolMaxJobs];
+  int zi[3][kPoolMaxJobs];
   p->members.clear();
   for (int q = 0; q < 3; ++q)
     for (int f = 0; f < 2; ++f) {
@@ -450,10 +422,26 @@ int rebuild_membership(pfdtd_pool *p) {
     PoolLaunch &L = p->launch[q][f];
     L.slot[L.n] = j.slot;
     L.ncol_max = std::max(L.ncol_max, j.ncol);
-    p->tiles[q][f] += j.tiles;
-    L.tile_end[L.n] = p->tiles[q][f];
+    if (f == 0) {
+      p->tiles[q][0] += j.tiles;
+      L.tile_end[L.n] = p->tiles[q][0];
+    }
+    bxy[q][L.n] = j.bxy;
+    zi[q][L.n] = j.zi;
     ++L.n;
     p->members.push_back(j.id);
+  }
+  for (int q = 0; q < 3; ++q) {
+    PoolLaunch &L = p->launch[q][1];
+    if (!L.n) continue;
+    const int zc = p->sweep_zc[q] = sweep_zchunk(L.n, bxy[q], zi[q], kPoolLevels);
+    int64_t end = 0;
+    for (int i = 0; i < L.n; ++i) {
+      end += bxy[q][i] * ((zi[q][i] + zc - 1) / zc);
+      L.tile_end[i] = (int)end;
+    }
+    if (end > (int64_t)1 << 30) return pfail(PFDTD_E_ARG, "resident jobs too large for one launch");
+    p->tiles[q][1] = (int)end;
   }
   if (p->exec) {
     p->retired.emplace_back(p->exec_last_seq, p->exec);
@@ -521,18 +509,28 @@ int check_job(const pfdtd_job *j) {
   return PFDTD_OK;
 }
 
-// Whether a job is advanced by the two-level sweep: not when a source sits on the first or last
+// Whether a job is advanced by the several-level sweep: not when a source sits on the first or last
 // z slice (never updated, but read by its neighbours: the single-step order is needed there)
-// or when one z slice exceeds the sweep's 32-bit buffer range.
+// or when one z slice exceeds the sweep's buffer range.
 bool job_fused(const pfdtd_job *j) {
   const size_t es = storage_bytes(j->precision);
-  if ((uint64_t)j->X * (uint64_t)j->Y * es >= (1ull << 32)) return false;
+  if ((uint64_t)j->X * (uint64_t)j->Y * es >= (1ull << 31)) return false;
   for (int s = 0; s < j->n_src; ++s) {
     const int32_t *q = &j->src_xyz[3 * s];
     const bool in = q[0] >= 0 && q[1] >= 0 && q[2] >= 0 && q[0] < j->X && q[1] < j->Y && q[2] < j->Z;
     if (in && (q[2] == 0 || q[2] == j->Z - 1)) return false;
   }
   return true;
+}
+
+// The arguments of an FP32 sweep as those of another storage type (the types differ in what their
+// field pointers point to).
+template <typename S>
+SweepArgs<S, CoefF, float> args_as(const SweepArgs<float, CoefF, float> &a) {
+  SweepArgs<S, CoefF, float> b;
+  static_assert(sizeof(a) == sizeof(b), "");
+  std::memcpy((void *)&b, (const void *)&a, sizeof(b));
+  return b;
 }
 
 int64_t grid_index(const int32_t *q, int X, int Y, int Z) {
@@ -562,6 +560,7 @@ int pfdtd_pool_create(int device, int64_t arena_bytes, pfdtd_pool **out) {
   hipError_t e = hipMalloc((void **)&p->arena, want);
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_jobs, sizeof(PoolJobDev) * kPoolMaxJobs);
   if (e == hipSuccess) e = hipMalloc((void **)&p->d_state, sizeof(PoolState) * kPoolMaxJobs);
+  if (e == hipSuccess) e = hipMalloc((void **)&p->d_args, sizeof(*p->d_args) * kPoolMaxJobs);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&p->run, hipStreamNonBlocking);
   if (e == hipSuccess) e = hipStreamCreateWithFlags(&p->upload, hipStreamNonBlocking);
   if (e != hipSuccess) {
@@ -586,6 +585,7 @@ int pfdtd_pool_destroy(pfdtd_pool *p) {
   if (p->arena) (void)hipFree(p->arena);
   if (p->d_jobs) (void)hipFree(p->d_jobs);
   if (p->d_state) (void)hipFree(p->d_state);
+  if (p->d_args) (void)hipFree(p->d_args);
   if (p->run) (void)hipStreamDestroy(p->run);
   if (p->upload) (void)hipStreamDestroy(p->upload);
   delete p;
@@ -603,7 +603,7 @@ int pfdtd_pool_set_options(pfdtd_pool *p, int bundle_steps, int use_graph, int r
   // tile geometry of resident jobs depends on rows / zchunk: change only on an empty pool
   if ((rows != p->ry || zchunk != p->zc) && !p->jobs.empty())
     return pfail(PFDTD_E_STATE, "tiling can change only while the pool is empty");
-  p->bundle = bundle_steps + (bundle_steps & 1);  // whole rounds of two steps
+  p->bundle = bundle_steps;  // taken as whole rounds of kPoolLevels steps
   p->use_graph = use_graph ? 1 : 0;
   p->ry = rows;
   p->zc = zchunk;
@@ -618,7 +618,7 @@ int pfdtd_pool_job_bytes(const pfdtd_job *j, int64_t *bytes) {
   if (!es || j->X < 1 || j->Y < 1 || j->Z < 1 || j->n_steps < 0 || j->n_src < 0 || j->n_rec < 0)
     return pfail(PFDTD_E_ARG, "bad job dimensions or precision");
   *bytes = (int64_t)layout_job(j->X, j->Y, j->Z, es, j->n_src, j->n_samples, j->n_rec, j->n_steps,
-                              j->n_src == 0 || j->src_xyz ? job_fused(j) : false)
+                              j->n_src == 0 || j->src_xyz ? job_fused(j) : false, j->precision)
                .total;
   return PFDTD_OK;
 }
@@ -652,7 +652,8 @@ int pfdtd_pool_submit(pfdtd_pool *p, const pfdtd_job *j, int64_t *job_id) {
   const int64_t N = (int64_t)X * Y * Z;
   const size_t es = storage_bytes(j->precision);
   const bool fused = job_fused(j);
-  const JobLayout L = layout_job(X, Y, Z, es, j->n_src, j->n_samples, j->n_rec, j->n_steps, fused);
+  const JobLayout L = layout_job(X, Y, Z, es, j->n_src, j->n_samples, j->n_rec, j->n_steps, fused,
+                                 j->precision);
   size_t off = 0;
   if (!arena_alloc(p, L.total, &off)) {
     size_t big = 0;
@@ -679,8 +680,6 @@ int pfdtd_pool_submit(pfdtd_pool *p, const pfdtd_job *j, int64_t *job_id) {
   PoolJobDev d{};
   d.pos = (const uint8_t *)(base + L.pos);
   d.mat = (const uint8_t *)(base + L.mat);
-  d.pm = fused ? (const uint16_t *)(base + L.pm) : nullptr;
-  d.air_rows = fused ? (const uint32_t *)(base + L.air_rows) : nullptr;
   for (int b = 0; b < 4; ++b) d.F[b] = (b < 2 || fused) ? base + L.F[b] : nullptr;
   d.coef = (const CoefF *)(base + L.coef);
   d.ncol = j->n_mat;  // labels were checked to name materials 0..n_mat-1 only
@@ -694,21 +693,15 @@ int pfdtd_pool_submit(pfdtd_pool *p, const pfdtd_job *j, int64_t *job_id) {
   d.gx = (X + kPoolTW - 1) / kPoolTW;
   d.gy = (Y + rows_per_tile - 1) / rows_per_tile;
   const int gz = (Z - 2 + p->zc - 1) / p->zc;
-  const FusedGeom fg = plan_fused(X, Y, Z, kPoolFusedZc, j->precision == PFDTD_F32 ? 0 : 2, true);
-  d.fx = (int)fg.grid.x;
-  d.fy = (int)fg.grid.y;
-  d.fused = fused ? 1 : 0;
-  const int64_t tiles = fused ? (int64_t)fg.grid.x * fg.grid.y * fg.grid.z
-                              : (int64_t)d.gx * d.gy * gz;
+  const SweepPlan sp = plan_sweep(j->precision, X, Y, Z, 0, 1);
+  const int64_t tiles = fused ? (int64_t)sp.nbx * sp.nby * (Z - 2) : (int64_t)d.gx * d.gy * gz;
   if (tiles > (int64_t)1 << 30) {
     arena_free(p, off, L.total);
     return pfail(PFDTD_E_ARG, "job grid too large for one launch");
   }
   d.rec_idx = (const int64_t *)(base + L.rec_idx);
-  d.rec_xyz = fused ? (const int32_t *)(base + L.rec_xyz) : nullptr;
   d.resp = (double *)(base + L.resp);
   d.src_idx = (const int64_t *)(base + L.src_idx);
-  d.src_xyz = fused ? (const int32_t *)(base + L.src_xyz) : nullptr;
   d.src_kind = (const int32_t *)(base + L.src_kind);
   d.sig = (const float *)(base + L.sig);
   d.n_rec = j->n_rec;
@@ -724,7 +717,53 @@ int pfdtd_pool_submit(pfdtd_pool *p, const pfdtd_job *j, int64_t *job_id) {
     std::sort(v.begin(), v.end());
     d.distinct = std::adjacent_find(v.begin(), v.end()) == v.end() ? 1 : 0;
   }
-  const PoolState st0{0, 0, 1};
+  // the steps that do not fill a round are taken here
+  const int lead = fused ? j->n_steps % kPoolLevels : 0;
+  const PoolState st0 = lead == 0 ? PoolState{0, 0, 1}
+                        : lead == 1 ? PoolState{1, 3, 0} : PoolState{lead, 3, 2};
+  std::vector<int32_t> ev_ptr, ev_data;
+  SweepArgs<float, CoefF, float> a{};
+  if (fused) {
+    std::vector<SweepPoint> rec, src;
+    for (int r = 0; r < j->n_rec; ++r)
+      if (ridx[r] >= 0)
+        rec.push_back(SweepPoint{j->rec_xyz[3 * r], j->rec_xyz[3 * r + 1], j->rec_xyz[3 * r + 2], 0,
+                                 (int32_t)((uint32_t)r | 0x80000000u)});
+    for (int s = 0; s < j->n_src; ++s)
+      if (sidx[s] >= 0)
+        src.push_back(SweepPoint{j->src_xyz[3 * s], j->src_xyz[3 * s + 1], j->src_xyz[3 * s + 2], 0, s});
+    sweep_events(sp, 1, rec, src, ev_ptr, ev_data);
+    sweep_geometry(sp, a);
+    a.pm = (const uint16_t *)(base + L.entry);
+    a.row_bits = (const uint64_t *)(base + L.row_bits);
+    a.ev_ptr = (const int32_t *)(base + L.ev_ptr);
+    a.events = (const int32_t *)(base + L.events);
+    a.A = (const float *)d.F[0];
+    a.B = (const float *)d.F[1];
+    a.Cn = (float *)d.F[2];
+    a.Dn = (float *)d.F[3];
+    a.coef = d.coef;
+    a.ncol = d.ncol;
+    a.air = d.air;
+    a.air_mask = air_uniform && d.air.inv == 1.f && d.air.omb == 1.f ? 0xFFu : 0u;
+    a.air_pm = 6u * (uint32_t)d.ncol * 0x10001u;
+    a.lam2 = d.lam2;
+    a.src_kind = (const int32_t *)(base + L.src_kind);
+    a.sig = (const float *)(base + L.sig);
+    a.n_samples = j->n_samples;
+    a.step = 0;
+    a.inject_end = j->n_steps;
+    a.soft_overwrite = (j->flags & PFDTD_SOFT_OVERWRITE) ? 1 : 0;
+    a.scale = std::ldexp(1.f, j->scale_exp);
+    a.inv_scale = std::ldexp(1.0, -j->scale_exp);
+    a.resp = (double *)(base + L.resp);
+    a.resp_steps = j->n_steps;
+    a.X = X;
+    a.Y = Y;
+    a.Z = Z;
+    a.n_slots = 1;
+    a.slot_elems = N;
+  }
 
   // set-up on the upload stream, concurrent with the resident jobs' steps
   hipStream_t u = p->upload;
@@ -735,13 +774,13 @@ int pfdtd_pool_submit(pfdtd_pool *p, const pfdtd_job *j, int64_t *job_id) {
   for (int b = 0; b < 4 && e == hipSuccess; ++b)
     if (d.F[b]) e = hipMemsetAsync(d.F[b], 0, es * (size_t)N, u);
   if (e == hipSuccess && fused)
-    e = launch_pack_pm(d.pos, d.mat, (uint16_t *)(base + L.pm), N, u);
+    e = launch_pack_entry(d.pos, d.mat, (uint16_t *)(base + L.entry), X, Y, Z, sp.pitch, d.ncol, u);
   if (e == hipSuccess && fused)
-    e = launch_air_rows(d.pm, (uint32_t *)(base + L.air_rows), X, Y, Z, 0, false, u);
-  if (e == hipSuccess && fused && j->n_src)
-    e = hipMemcpyAsync(base + L.src_xyz, j->src_xyz, sizeof(int32_t) * 3 * j->n_src, hipMemcpyHostToDevice, u);
-  if (e == hipSuccess && fused && j->n_rec)
-    e = hipMemcpyAsync(base + L.rec_xyz, j->rec_xyz, sizeof(int32_t) * 3 * j->n_rec, hipMemcpyHostToDevice, u);
+    e = launch_row_bits(sp, a.pm, (uint64_t *)(base + L.row_bits), X, Y, Z, d.ncol, u);
+  if (e == hipSuccess && fused)
+    e = hipMemcpyAsync(base + L.ev_ptr, ev_ptr.data(), sizeof(int32_t) * ev_ptr.size(), hipMemcpyHostToDevice, u);
+  if (e == hipSuccess && !ev_data.empty())
+    e = hipMemcpyAsync(base + L.events, ev_data.data(), sizeof(int32_t) * ev_data.size(), hipMemcpyHostToDevice, u);
   if (e == hipSuccess && j->n_rec)
     e = hipMemsetAsync(base + L.resp, 0, sizeof(double) * (size_t)j->n_rec * j->n_steps, u);
   if (e == hipSuccess) e = hipMemcpyAsync(base + L.coef, cf.data(), sizeof(CoefF) * kCoefEntries, hipMemcpyHostToDevice, u);
@@ -757,24 +796,33 @@ int pfdtd_pool_submit(pfdtd_pool *p, const pfdtd_job *j, int64_t *job_id) {
     e = hipMemcpyAsync(base + L.rec_idx, ridx.data(), sizeof(int64_t) * j->n_rec, hipMemcpyHostToDevice, u);
   if (e == hipSuccess && j->n_src) {
     // step 0's samples go into the (zero) current field before the first update
-    InjectArgs a{};
-    a.rec_idx = d.rec_idx;
-    a.n_rec = 0;
-    a.resp = d.resp;
-    a.resp_steps = j->n_steps;
-    a.gather_step = -1;
-    a.src_idx = d.src_idx;
-    a.src_kind = d.src_kind;
-    a.n_src = j->n_src;
-    a.sig_f = d.sig;
-    a.sig_d = nullptr;
-    a.n_samples = j->n_samples;
-    a.inject_step = 0;
-    a.soft_overwrite = d.soft_overwrite;
-    a.scale_exp = j->scale_exp;
-    a.distinct = d.distinct;
-    e = launch_inject_gather(j->precision, d.F[0], a, u);
+    InjectArgs ia{};
+    ia.rec_idx = d.rec_idx;
+    ia.n_rec = 0;
+    ia.resp = d.resp;
+    ia.resp_steps = j->n_steps;
+    ia.gather_step = -1;
+    ia.src_idx = d.src_idx;
+    ia.src_kind = d.src_kind;
+    ia.n_src = j->n_src;
+    ia.sig_f = d.sig;
+    ia.sig_d = nullptr;
+    ia.n_samples = j->n_samples;
+    ia.inject_step = 0;
+    ia.soft_overwrite = d.soft_overwrite;
+    ia.scale_exp = j->scale_exp;
+    ia.distinct = d.distinct;
+    e = launch_inject_gather(j->precision, d.F[0], ia, u);
   }
+  if (e == hipSuccess && lead) {
+    switch (j->precision) {
+    case PFDTD_F32: e = launch_sweep_f32(sp, a, lead, u); break;
+    case PFDTD_F16: e = launch_sweep_f16(sp, args_as<h16>(a), lead, u); break;
+    default: e = launch_sweep_bf16(sp, args_as<b16>(a), lead, u); break;
+    }
+  }
+  if (e == hipSuccess && fused)
+    e = hipMemcpyAsync(p->d_args + slot, &a, sizeof(a), hipMemcpyHostToDevice, u);
   if (e == hipSuccess) e = hipMemcpyAsync(p->d_jobs + slot, &d, sizeof(d), hipMemcpyHostToDevice, u);
   if (e == hipSuccess) e = hipMemcpyAsync(p->d_state + slot, &st0, sizeof(st0), hipMemcpyHostToDevice, u);
   // the host arrays above are read by the copies: wait for this job's set-up only
@@ -795,9 +843,13 @@ int pfdtd_pool_submit(pfdtd_pool *p, const pfdtd_job *j, int64_t *job_id) {
   h.n_rec = j->n_rec;
   h.voxels = N;
   h.tiles = (int)tiles;
+  h.bxy = (int64_t)sp.nbx * sp.nby;
+  h.zi = Z - 2;
+  h.steps_enqueued = lead;
   h.off = off;
   h.bytes = L.total;
   h.d_resp = d.resp;
+  p->voxel_steps += (double)N * lead;
   p->jobs[h.id] = h;
   p->slot_job[slot] = h.id;
   p->dirty = true;
@@ -840,7 +892,7 @@ int pfdtd_pool_advance(pfdtd_pool *p, int *n_active) {
   for (int64_t id : p->members) {
     PoolJobHost &j = p->jobs[id];
     const int64_t before = j.steps_enqueued;
-    j.steps_enqueued = std::min<int64_t>(j.n_steps, before + p->bundle);
+    j.steps_enqueued = std::min<int64_t>(j.n_steps, before + bundle_steps(p));
     p->voxel_steps += (double)j.voxels * (double)(j.steps_enqueued - before);
     if (j.steps_enqueued >= j.n_steps) {
       j.phase = kFinishing;

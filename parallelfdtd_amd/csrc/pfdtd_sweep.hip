@@ -167,13 +167,23 @@ constexpr uint32_t kDrop = 0x80000000u;  // offset bit that puts a store out of 
 
 }  // namespace
 
+template <typename S>
+using SweepArgsOf = SweepArgs<S, typename CoefOf<typename Fmt<S>::C>::T, typename Fmt<S>::C>;
+// Arguments of a sweep in constant memory: the kernel's own, or a pool job's.
+template <typename S>
+using ConstSweepArgs = const __attribute__((address_space(4))) SweepArgsOf<S> *;
+
+// One block of a sweep: tile `tile` of nbx x nby x (z-chunks of zc slices), fields fA, fB to fC, fD,
+// first step `step`.
 template <typename S, int L, int LM, int TY, int WY, int NC, int HX>
-__global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_kernel(
-    SweepArgs<S, typename CoefOf<typename Fmt<S>::C>::T, typename Fmt<S>::C> a) {
+__device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned tile, int slot, int zc,
+                                            const S *__restrict__ gA, const S *__restrict__ gB,
+                                            S *__restrict__ gC, S *__restrict__ gD, int step) {
 #pragma clang fp contract(off)
   typedef typename Fmt<S>::C C;
   typedef typename CoefOf<C>::T CE;
-  typedef const __attribute__((address_space(4))) SweepArgs<S, CE, C> *ConstArgs;
+  typedef ConstSweepArgs<S> ConstArgs;
+  const auto &a = *args;
   typedef Cols<C, NC> V;
   typedef Raw<S, NC> R;
   typedef typename std::conditional<NC == 2, uint32_t, uint16_t>::type PM;
@@ -186,11 +196,6 @@ __global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_kernel(
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int X = a.X, Y = a.Y, Z = a.Z;
   const unsigned ncol = (unsigned)a.ncol;
-  // XCD-aware order: every XCD walks a contiguous run of tiles
-  const unsigned total = gridDim.x, lin = blockIdx.x, full = total & ~7u;
-  unsigned tile = lin < full ? (lin & 7u) * (full >> 3) + (lin >> 3) : lin;
-  const int slot = (int)(tile % (unsigned)a.n_slots);
-  tile /= (unsigned)a.n_slots;
   const unsigned nxy = (unsigned)(a.nbx * a.nby);
   const unsigned tl = tile % nxy;
   const int bzi = (int)(tile / nxy);
@@ -199,15 +204,9 @@ __global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_kernel(
   const unsigned band_rows = min(bg, (unsigned)a.nby - band * bg);
   const int byi = (int)(band * bg + in_band % band_rows);
   const int bxi = (int)(in_band / band_rows);
-  const int64_t soff = (int64_t)slot * a.slot_elems;
-  const S *__restrict__ gA = a.A + soff;
-  const S *__restrict__ gB = a.B + soff;
-  S *__restrict__ gC = a.Cn + soff;
-  S *__restrict__ gD = a.Dn + soff;
-
   const int x0 = bxi * OX - HX + NC * lane;           // this lane's first column
   const int yw = byi * OY - LM + wave * TY;           // this wave's first row
-  const int z0 = 1 + bzi * a.zc, z1 = min(z0 + a.zc, Z - 1);
+  const int z0 = 1 + bzi * zc, z1 = min(z0 + zc, Z - 1);
 
   // LDS: coefficient rows | halo rows [2][L][WY][2][64] | packed rows [WY][RING][TY][64]
   extern __shared__ __align__(16) unsigned char s_dyn[];
@@ -254,7 +253,7 @@ __global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_kernel(
     ev_end = ((ConstI32)a.ev_ptr)[et + 1];
   }
   auto ev_at = [&](int n, int i) -> int {
-    ConstArgs ka = (ConstArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    ConstArgs ka = args;
     asm volatile("" : "+s"(ka));
     return ((ConstI32)ka->events)[4 * n + i];
   };
@@ -451,7 +450,7 @@ __global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_kernel(
         if constexpr (KIND == 2) {
           // the event arguments are re-read here, so that they hold no scalar registers across
           // the sweep
-          ConstArgs ka = (ConstArgs)__builtin_amdgcn_kernarg_segment_ptr();
+          ConstArgs ka = args;
           asm volatile("" : "+s"(ka));
           const ConstI32 gev = (ConstI32)ka->events;
           for (int n = ev; n < ev_end && gev[4 * n] <= k; ++n) {
@@ -462,12 +461,12 @@ __global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_kernel(
               if (xe != x0 + c) continue;
               if (id < 0) {  // receiver
                 if (own_x && ((own_rows >> r) & 1u) && s >= z0 && s < z1)
-                  ka->resp[(int64_t)(id & 0x7FFFFFFF) * ka->resp_steps + ka->step + i - 1] =
+                  ka->resp[(int64_t)(id & 0x7FFFFFFF) * ka->resp_steps + step + i - 1] =
                       (double)t[i].v[c] * ka->inv_scale;
-              } else if (ka->step + i < ka->inject_end) {
+              } else if (step + i < ka->inject_end) {
                 C smp = (C)0;
-                if (ka->step + i < ka->n_samples)
-                  smp = (C)ka->sig[(int64_t)id * ka->n_samples + ka->step + i];
+                if (step + i < ka->n_samples)
+                  smp = (C)ka->sig[(int64_t)id * ka->n_samples + step + i];
                 smp = smp * ka->scale;
                 const bool hard = ka->src_kind[id] == 0 || ka->soft_overwrite;
                 t[i].v[c] = Fmt<S>::round(hard ? smp : t[i].v[c] + smp);
@@ -529,6 +528,70 @@ __global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_kernel(
     body(std::integral_constant<int, 0>(), k);
     if (++k > ke) break;
   }
+}
+
+// XCD-aware order: consecutive block ids are dealt round-robin to the 8 XCDs; every XCD walks a
+// contiguous run of tiles.
+__device__ __forceinline__ unsigned xcd_tile() {
+  const unsigned total = gridDim.x, lin = blockIdx.x, full = total & ~7u;
+  return lin < full ? (lin & 7u) * (full >> 3) + (lin >> 3) : lin;
+}
+
+// A context's sweep: the slots of a batch innermost, so that one XCD's L2 serves a tile's entries
+// to all of them.
+template <typename S, int L, int LM, int TY, int WY, int NC, int HX>
+__global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_kernel(SweepArgsOf<S> a) {
+  const unsigned tile = xcd_tile();
+  const int slot = (int)(tile % (unsigned)a.n_slots);
+  const int64_t off = (int64_t)slot * a.slot_elems;
+  sweep_block<S, L, LM, TY, WY, NC, HX>(
+      (ConstSweepArgs<S>)__builtin_amdgcn_kernarg_segment_ptr(), tile / (unsigned)a.n_slots, slot,
+      a.zc, a.A + off, a.B + off, a.Cn + off, a.Dn + off, a.step);
+}
+
+// Round `round` of a bundle for every job of a pool launch: L steps per job. A block finds its job by
+// a binary search over the launch table. The state holds the step and buffers at the start of the
+// bundle; rounds alternate between the two pairs of buffers.
+template <typename S, int L, int LM, int TY, int WY, int NC, int HX>
+__global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_pool_kernel(
+    const SweepArgsOf<S> *__restrict__ args, const PoolJobDev *__restrict__ jobs,
+    const PoolState *__restrict__ state, PoolLaunch pl, int zc, int round) {
+  const int tile = (int)xcd_tile();
+  int lo = 0, hi = pl.n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi) >> 1;
+    if (pl.tile_end[mid] > tile)
+      hi = mid;
+    else
+      lo = mid + 1;
+  }
+  const int job = pl.slot[lo];
+  const PoolState st = state[job];
+  const PoolJobDev &J = jobs[job];
+  const int step = st.step + round * L;
+  if (step >= J.n_steps) return;  // the whole block: no barrier has been reached
+  int o1, o2;
+  pool_spare(st.cur, st.past, o1, o2);
+  const bool odd = round & 1;
+  sweep_block<S, L, LM, TY, WY, NC, HX>(
+      (ConstSweepArgs<S>)(args + job), (unsigned)(tile - (lo ? pl.tile_end[lo - 1] : 0)), 0, zc,
+      (const S *)J.F[odd ? o2 : st.cur], (const S *)J.F[odd ? o1 : st.past],
+      (S *)J.F[odd ? st.past : o1], (S *)J.F[odd ? st.cur : o2], step);
+}
+
+// After a bundle of `rounds` rounds: the step and buffers of every job of the launch.
+__global__ __launch_bounds__(kPoolMaxJobs) void pool_rotate_kernel(
+    const PoolJobDev *__restrict__ jobs, PoolState *__restrict__ state, PoolLaunch pl, int rounds,
+    int levels) {
+  if ((int)threadIdx.x >= pl.n) return;
+  const int job = pl.slot[threadIdx.x];
+  const PoolState st = state[job];
+  const int left = (jobs[job].n_steps - st.step + levels - 1) / levels;
+  const int n = min(rounds, max(left, 0));
+  int o1, o2;
+  pool_spare(st.cur, st.past, o1, o2);
+  state[job] = (n & 1) ? PoolState{st.step + n * levels, o2, o1}
+                       : PoolState{st.step + n * levels, st.cur, st.past};
 }
 
 // Coefficient entry per voxel: row min(K, 6) of ncol material columns, or kStageRows * ncol outside.
@@ -628,6 +691,31 @@ hipError_t launch_interleave(int elem_bytes, const void *field, int64_t N, int64
   return hipGetLastError();
 }
 
+// Slices per z-chunk for a launch over n grids of bxy[i] blocks per chunk and zi[i] slices. One block
+// per CU: a launch takes as many rounds as 256 goes into its blocks, and a round the chunk's slices
+// plus the 2 (levels - 1) of its neighbours' and about two more to start. The chunk length with the
+// least of both: on 256x256x256 FP32 24 slices (231 blocks) take 34 us per step, 16 slices (two
+// rounds) 50 and 32 slices 42; on 1024x768x384 48-64 slices 345, 32 and 96 slices 354 and 371.
+int sweep_zchunk(int n, const int64_t *bxy, const int *zi, int levels) {
+  int top = 1, best_c = 1;
+  for (int i = 0; i < n; ++i) top = std::max(top, zi[i]);
+  double best = 0;
+  for (int nz = 1; nz <= top; ++nz) {
+    const int c = (top + nz - 1) / nz;
+    if (nz > 1 && c == (top + nz - 2) / (nz - 1)) continue;
+    int64_t blocks = 0;
+    for (int i = 0; i < n; ++i) blocks += bxy[i] * ((zi[i] + c - 1) / c);
+    const double full = (double)((blocks + 255) / 256);
+    const double rounds = blocks <= 1024 ? full : std::min(full, blocks / 256.0 + 0.4);
+    const double cost = rounds * (c + 2 * (levels - 1) + 2);
+    if (nz == 1 || cost < best) {
+      best = cost;
+      best_c = c;
+    }
+  }
+  return best_c;
+}
+
 namespace {
 
 // Tile of the sweep per storage type: columns per lane, rows per wave, waves, most levels, halo
@@ -668,54 +756,32 @@ SweepPlan plan_of(int X, int Y, int Z, int zc, int slots) {
   p.band = 2;
   const int zi = Z - 2;
   const int64_t bxy = (int64_t)p.nbx * p.nby * slots;
-  if (zc < 1) {
-    // One block per CU: a launch takes as many rounds as 256 goes into its blocks, and a round the
-    // chunk's slices plus the 2 (LM - 1) of its neighbours' and about two more to start. The chunk
-    // count with the least of both: on 256x256x256 FP32 24 slices (231 blocks) take 34 us per step,
-    // 16 slices (two rounds) 50 and 32 slices 42; on 1024x768x384 48-64 slices 345, 32 and 96
-    // slices 354 and 371.
-    double best = 0;
-    for (int nz = 1; nz <= zi; ++nz) {
-      const int c = (zi + nz - 1) / nz;
-      if (nz > 1 && c == (zi + nz - 2) / (nz - 1)) continue;
-      const int64_t blocks = bxy * ((zi + c - 1) / c);
-      const double full = (double)((blocks + 255) / 256);
-      const double rounds = blocks <= 1024 ? full : std::min(full, blocks / 256.0 + 0.4);
-      const double cost = rounds * (c + 2 * (T::LM - 1) + 2);
-      if (nz == 1 || cost < best) {
-        best = cost;
-        zc = c;
-      }
-    }
-  }
+  if (zc < 1) zc = sweep_zchunk(1, &bxy, &zi, T::LM);
   p.zc = std::min(zc, zi);
   p.blocks = bxy * ((zi + p.zc - 1) / p.zc);
   return p;
 }
 
 template <typename S, int L>
-hipError_t launch_levels(const SweepPlan &p, SweepArgs<S, typename CoefOf<typename Fmt<S>::C>::T, typename Fmt<S>::C> &a,
-                         hipStream_t stream) {
+size_t sweep_lds(int ncol) {
   typedef SweepTile<S> T;
   typedef typename Fmt<S>::C C;
-  typedef typename CoefOf<C>::T CE;
-  constexpr int RING = sweep_ring(L);
-  const size_t lds = sizeof(CE) * (kStageRows * (size_t)a.ncol + 1) +
-                     sizeof(Cols<C, T::NC>) * 2 * L * T::WY * 2 * 64 +
-                     2 * T::NC * (size_t)T::WY * RING * T::TY * 64;
+  return sizeof(typename CoefOf<C>::T) * (kStageRows * (size_t)ncol + 1) +
+         sizeof(Cols<C, T::NC>) * 2 * L * T::WY * 2 * 64 +
+         2 * T::NC * (size_t)T::WY * sweep_ring(L) * T::TY * 64;
+}
+
+template <typename S, int L>
+hipError_t launch_levels(const SweepPlan &p, const SweepArgsOf<S> &a, hipStream_t stream) {
+  typedef SweepTile<S> T;
+  const size_t lds = sweep_lds<S, L>(a.ncol);
   hipLaunchKernelGGL((srl_sweep_kernel<S, L, T::LM, T::TY, T::WY, T::NC, T::HX>), dim3((unsigned)p.blocks),
                      dim3(64 * T::WY), lds, stream, a);
   return hipGetLastError();
 }
 
 template <typename S, typename A>
-hipError_t launch_any(const SweepPlan &p, A &a, int levels, hipStream_t stream) {
-  a.pitch = p.pitch;
-  a.air_words = p.words;
-  a.zc = p.zc;
-  a.nbx = p.nbx;
-  a.nby = p.nby;
-  a.band = p.band;
+hipError_t launch_any(const SweepPlan &p, const A &a, int levels, hipStream_t stream) {
   switch (levels) {
   case 1: return launch_levels<S, 1>(p, a, stream);
   case 2: return launch_levels<S, 2>(p, a, stream);
@@ -733,7 +799,37 @@ hipError_t launch_any(const SweepPlan &p, A &a, int levels, hipStream_t stream) 
   return hipErrorInvalidValue;
 }
 
+static_assert(SweepTile<float>::LM == kPoolLevels && SweepTile<h16>::LM == kPoolLevels, "");
+
+template <typename S>
+hipError_t launch_pool(int tiles, const void *args, const PoolJobDev *jobs, const PoolState *st,
+                       const PoolLaunch &pl, int zc, int round, hipStream_t stream) {
+  typedef SweepTile<S> T;
+  const size_t lds = sweep_lds<S, T::LM>(pl.ncol_max);
+  hipLaunchKernelGGL((srl_sweep_pool_kernel<S, T::LM, T::LM, T::TY, T::WY, T::NC, T::HX>),
+                     dim3((unsigned)tiles), dim3(64 * T::WY), lds, stream, (const SweepArgsOf<S> *)args, jobs, st, pl, zc, round);
+  return hipGetLastError();
+}
+
 }  // namespace
+
+hipError_t launch_sweep_pool(int precision, int tiles, const void *args, const PoolJobDev *jobs,
+                             const PoolState *st, const PoolLaunch &pl, int zc, int round,
+                             hipStream_t stream) {
+  switch (precision) {
+  case PFDTD_F32: return launch_pool<float>(tiles, args, jobs, st, pl, zc, round, stream);
+  case PFDTD_F16: return launch_pool<h16>(tiles, args, jobs, st, pl, zc, round, stream);
+  case PFDTD_BF16: return launch_pool<b16>(tiles, args, jobs, st, pl, zc, round, stream);
+  default: return hipErrorInvalidValue;
+  }
+}
+
+hipError_t launch_pool_rotate(const PoolJobDev *jobs, PoolState *st, const PoolLaunch &pl,
+                              int rounds, int levels, hipStream_t stream) {
+  hipLaunchKernelGGL(pool_rotate_kernel, dim3(1), dim3(kPoolMaxJobs), 0, stream, jobs, st, pl,
+                     rounds, levels);
+  return hipGetLastError();
+}
 
 SweepPlan plan_sweep(int precision, int X, int Y, int Z, int zc, int slots) {
   switch (precision) {
@@ -744,6 +840,46 @@ SweepPlan plan_sweep(int precision, int X, int Y, int Z, int zc, int slots) {
   }
 }
 
+void sweep_events(const SweepPlan &p, int slots, const std::vector<SweepPoint> &rec,
+                  const std::vector<SweepPoint> &src, std::vector<int32_t> &ptr,
+                  std::vector<int32_t> &data) {
+  const int ntile = p.nby * p.wy * p.nbx;
+  struct Ev {
+    int tile;
+    const SweepPoint *q;
+  };
+  std::vector<Ev> ev;
+  auto add = [&](const SweepPoint &q, int bx, int by, int row) {
+    ev.push_back(Ev{q.slot * ntile + (by * p.wy + row / p.ty) * p.nbx + bx, &q});
+  };
+  for (const SweepPoint &q : rec)
+    add(q, q.x / p.ox, q.y / p.oy, q.y % p.oy + p.lm);
+  for (const SweepPoint &q : src)
+    for (int by = std::max(0, (q.y - p.lm) / p.oy - 1); by < p.nby; ++by) {
+      const int row = q.y - by * p.oy + p.lm;
+      if (row < 0) break;
+      if (row >= p.wy * p.ty) continue;
+      for (int bx = std::max(0, (q.x - p.hx) / p.ox - 1); bx < p.nbx; ++bx) {
+        const int col = q.x - bx * p.ox + p.hx;
+        if (col < 0) break;
+        if (col < p.w) add(q, bx, by, row);
+      }
+    }
+  std::stable_sort(ev.begin(), ev.end(), [](const Ev &a, const Ev &b) {
+    return a.tile != b.tile ? a.tile < b.tile : a.q->z < b.q->z;
+  });
+  ptr.assign((size_t)slots * ntile + 1, 0);
+  data.resize(4 * ev.size());
+  for (size_t i = 0; i < ev.size(); ++i) {
+    ++ptr[(size_t)ev[i].tile + 1];
+    data[4 * i] = ev[i].q->z;
+    data[4 * i + 1] = ev[i].q->x;
+    data[4 * i + 2] = ev[i].q->y;
+    data[4 * i + 3] = ev[i].q->id;
+  }
+  for (size_t i = 1; i < ptr.size(); ++i) ptr[i] += ptr[i - 1];
+}
+
 hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint64_t *out, int X, int Y,
                            int Z, int ncol, hipStream_t stream) {
   const dim3 grid((unsigned)p.nbx, (unsigned)(p.nby * p.wy), (unsigned)std::min(p.words, 65535));
@@ -752,19 +888,19 @@ hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint64_t *out
   return hipGetLastError();
 }
 
-hipError_t launch_sweep_f32(const SweepPlan &p, SweepArgs<float, CoefF, float> a, int levels,
+hipError_t launch_sweep_f32(const SweepPlan &p, const SweepArgsOf<float> &a, int levels,
                             hipStream_t stream) {
   return launch_any<float>(p, a, levels, stream);
 }
-hipError_t launch_sweep_f16(const SweepPlan &p, SweepArgs<h16, CoefF, float> a, int levels,
+hipError_t launch_sweep_f16(const SweepPlan &p, const SweepArgsOf<h16> &a, int levels,
                             hipStream_t stream) {
   return launch_any<h16>(p, a, levels, stream);
 }
-hipError_t launch_sweep_bf16(const SweepPlan &p, SweepArgs<b16, CoefF, float> a, int levels,
+hipError_t launch_sweep_bf16(const SweepPlan &p, const SweepArgsOf<b16> &a, int levels,
                              hipStream_t stream) {
   return launch_any<b16>(p, a, levels, stream);
 }
-hipError_t launch_sweep_f64(const SweepPlan &p, SweepArgs<double, CoefD, double> a, int levels,
+hipError_t launch_sweep_f64(const SweepPlan &p, const SweepArgsOf<double> &a, int levels,
                             hipStream_t stream) {
   return launch_any<double>(p, a, levels, stream);
 }
