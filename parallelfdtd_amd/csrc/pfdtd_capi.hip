@@ -835,7 +835,7 @@ int ensure_sweep(pfdtd_ctx *c, const SweepPlan &p, bool *ok) {
                             p.pitch, ncol, c->stream);
   }
   if (e == hipSuccess && (!c->entry_ok || !same)) {
-    e = grow(c->d_row_bits, c->air_cap, 2 * (size_t)p.nbx * p.nby * p.wy * p.words);
+    e = grow(c->d_row_bits, c->air_cap, sweep_row_words(p));
     if (e == hipSuccess)
       e = launch_row_bits(p, c->d_entry, c->d_row_bits, (int)c->X, (int)c->Y, (int)c->Z, ncol,
                           c->stream);

@@ -234,7 +234,7 @@ template <typename S, typename CT, typename C>
 struct SweepArgs {
   const uint16_t *pm;  // coefficient entry per voxel, rows of `pitch` elements
   int pitch;
-  const uint64_t *row_bits;  // per wave tile, two bytes per slice: its rows of plain air, solid rows
+  const uint64_t *row_bits;  // per wave tile, three bytes per slice: rows of plain air, solid, unchanged
   int air_words;             // words per wave tile
   const int32_t *ev_ptr;     // per (slot, wave tile): first event, then one past the last
   const int32_t *events;     // {z, x, y, source index or receiver index | 1 << 31}, by z
@@ -270,6 +270,10 @@ struct SweepPlan {
   int nbx, nby, zc, band, words, pitch;
   int64_t blocks;
 };
+// Words of a plan's row bits.
+inline size_t sweep_row_words(const SweepPlan &p) {
+  return 3 * (size_t)p.nbx * p.nby * p.wy * p.words;
+}
 SweepPlan plan_sweep(int precision, int X, int Y, int Z, int zc, int slots);
 // Fills the tile geometry of a sweep's arguments.
 template <typename A>

@@ -212,7 +212,7 @@ JobLayout layout_job(int X, int Y, int Z, size_t es, int n_src, int n_samples, i
   L.pos = take((size_t)N);
   L.mat = take((size_t)N);
   L.entry = fused ? take(sizeof(uint16_t) * (size_t)sp.pitch * Y * Z) : 0;
-  L.row_bits = fused ? take(2 * sizeof(uint64_t) * wave_tiles * sp.words) : 0;
+  L.row_bits = fused ? take(sizeof(uint64_t) * sweep_row_words(sp)) : 0;
   L.labels = take((size_t)N);
   L.coef = take(sizeof(CoefF) * kCoefEntries);
   L.src_idx = take(sizeof(int64_t) * (size_t)n_src);

@@ -27,10 +27,22 @@
 // although five columns would do; 16 (96 owned columns) 3.07.
 //
 // Rows of plain air at every level of an iteration take the air entry as an immediate (nine VALU
-// operations per node); rows with nothing to update at any level are zeros; the others gather
-// every node's table entry from LDS, the gathers of the next level in flight during the last. The
-// choice is made by two bits per row and slice built once per domain. Made once for all rows of an
-// iteration instead, it keeps both the old and the new queue entries live (75 registers more).
+// operations per node); rows with nothing to update at any level are zeros. Of the others, those whose
+// entries are the same on the iteration's slices -- along walls, pillars and the sides of boxes --
+// gather one entry per node for all levels; the rest gather every node's entry at every level from
+// LDS, the gathers of the next level in flight during the last. The choice is made by three bits per
+// row and slice built once per domain. Made once for all rows of an iteration instead, it keeps both
+// the old and the new queue entries live (75 registers more). Entries the slice above shares stay in
+// their registers and are not loaded again.
+//
+// Within a CU the sweep is bound by issue: two waves of a SIMD issue some 1200 instructions each per
+// slice, about 3.5 ns for two dependent FP32 additions and 1.3 for independent ones, so a lane's
+// two columns are written side by side. us per step, one entry per node and level -> one per node ->
+// columns side by side, and accesses behind the choice of the row: 1024x768x384 hall FP32 355 -> 320 ->
+// 309, 256x256x256 FP32 33.4 -> 29.5 -> 27.3, 701x523x307 BF16 158 -> 142 -> 123, 130x98x66 FP32
+// 12.2 -> 11.5 -> 10.8, 1024x768x384 FP64 750 -> 712 -> 725, 2048x1536x768 FP16 2004 -> 1962 -> 1955.
+// Sixteen waves of 3 rows each (four waves per SIMD, 4 levels to fit 128 registers) take 371 on the
+// hall and 28.6 on 256x256x256.
 //
 // Loads, stores and masks. Slices are accessed through buffer descriptors: rows and columns past
 // the grid read 0, stores that a lane or row does not own are given an offset past the slice and
@@ -161,7 +173,7 @@ typedef const __attribute__((address_space(4))) uint64_t *ConstU64;
 
 // Slices of packed rows a wave keeps in LDS: the L - 1 slices above the first level's, rounded up
 // to a power of two.
-constexpr int sweep_ring(int L) { return L <= 2 ? 1 : L == 3 ? 2 : L <= 5 ? 4 : 8; }
+constexpr int sweep_ring(int L) { return L <= 2 ? 1 : L == 3 ? 2 : 4; }
 
 constexpr uint32_t kDrop = 0x80000000u;  // offset bit that puts a store out of range
 
@@ -187,11 +199,10 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
   typedef Cols<C, NC> V;
   typedef Raw<S, NC> R;
   typedef typename std::conditional<NC == 2, uint32_t, uint16_t>::type PM;
-  static_assert(TY >= 2 && TY <= 8 && L >= 1 && L <= LM && LM <= 8 && HX >= LM && HX % NC == 0, "");
+  static_assert(TY >= 2 && TY <= 8 && L >= 1 && L <= LM && LM <= 5 && HX >= LM && HX % NC == 0, "");
   constexpr int W = 64 * NC, OX = W - 2 * HX;
   constexpr int H = WY * TY, OY = H - 2 * LM;
   constexpr int RING = sweep_ring(L);
-  constexpr uint64_t kRowAir = L == 8 ? 0x0101010101010101ull : 0x0101010101010101ull & ((1ull << (8 * L % 64)) - 1ull);
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const int X = a.X, Y = a.Y, Z = a.Z;
@@ -228,7 +239,8 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
   const uint32_t pcol = (uint32_t)((yw * a.pitch + x0) * 2);
   // owned columns of this lane, owned rows of this wave
   const bool own_x = NC * lane >= HX && NC * lane < HX + OX && x0 < X;
-  const uint32_t vst = own_x ? vcol : kDrop;
+  const bool pair = NC == 1 || x0 + 1 < X;  // the lane's columns both lie in the grid
+  const uint32_t vst = own_x && pair ? vcol : kDrop, vst1 = own_x && !pair ? vcol : kDrop;
   uint32_t own_rows = 0;
 #pragma unroll
   for (int r = 0; r < TY; ++r) {
@@ -238,14 +250,15 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
   bool col_ok[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) col_ok[c] = x0 + c > 0 && x0 + c < X - 1;
-  const bool x_odd = NC == 2 && (X & 1);
+  // the tile with the last column of an odd width, which is stored on its own
+  const bool odd_edge = NC == 2 && (X & 1) && bxi == a.nbx - 1;
   const C air_tk = a.air.tk, lam2 = a.lam2;
   const uint32_t air_pm = a.air_pm, air_mask = a.air_mask, out_pm = kStageRows * ncol * 0x10001u;
 
-  // air and solid rows of this wave's tile (a byte each per slice, 8 slices per word), and its
-  // events by z
+  // air, solid and unchanged rows of this wave's tile (a byte each per slice, 8 slices per word), and
+  // its events by z
   const int wt = (byi * WY + wave) * a.nbx + bxi;
-  const ConstU64 gair = (ConstU64)(a.row_bits + 2 * (size_t)wt * a.air_words);
+  const ConstU64 gair = (ConstU64)(a.row_bits + 3 * (size_t)wt * a.air_words);
   int ev = 0, ev_end = 0;
   {
     const int et = slot * (a.nby * WY * a.nbx) + wt;
@@ -294,27 +307,35 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
   };
   const int wu = wave > 0 ? wave - 1 : 0, wd = wave < WY - 1 ? wave + 1 : WY - 1;
 
-  // row bytes of the current and the next 8 slices: x plain air, y solid (or not updated); every
-  // row of a slice outside 1..Z-2 is solid
+  // row bytes of the current and the next 8 slices: plain air, solid (or not updated), and the entries
+  // of the slice below; every row of a slice outside 1..Z-2 is solid
   struct Rows {
-    uint64_t air, solid;
+    uint64_t air, solid, same;
   };
   Rows bw, bn;
   auto load_rows = [&](int w) -> Rows {
-    if (w >= a.air_words) return Rows{0, 0};
-    return Rows{gair[2 * w], gair[2 * w + 1]};
+    if (w >= a.air_words) return Rows{0, 0, 0};
+    return Rows{gair[3 * w], gair[3 * w + 1], gair[3 * w + 2]};
   };
   struct RowBits {
-    uint32_t air, solid;
+    uint32_t air, solid, same;
   };
   auto row_bits = [&](int k, bool step) -> RowBits {
-    if (k < 1 || k > Z - 2) return RowBits{0u, 0xFFu};
+    if (k < 1 || k > Z - 2) return RowBits{0u, 0xFFu, 0u};
     if (step && (k & 7) == 0) {
       bw = bn;
       bn = load_rows((k >> 3) + 1);
     }
     const int sh = 8 * (k & 7);
-    return RowBits{(uint32_t)(bw.air >> sh) & air_mask, (uint32_t)(bw.solid >> sh) & 0xFFu};
+    return RowBits{(uint32_t)(bw.air >> sh) & air_mask, (uint32_t)(bw.solid >> sh) & 0xFFu,
+                   (uint32_t)(bw.same >> sh) & 0xFFu};
+  };
+  // the rows set in each of the n newest bytes of a history
+  auto all_of = [](uint64_t h, int n) -> uint32_t {
+    uint32_t v = 0xFFu;
+#pragma unroll
+    for (int j = 0; j < n; ++j) v &= (uint32_t)(h >> (8 * j));
+    return v;
   };
 
   const int kb = z0 - (L - 1), ke = z1 - 1 + (L - 1);
@@ -342,9 +363,10 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
     else
       hi = mid;
   }
-  // row bytes of slices k, k-1, ...: those below the chunk count as air and solid (their levels
-  // are not used)
+  // row bytes of slices k, k-1, ...: those below the chunk count as air, solid and unchanged (their
+  // levels are not used)
   uint64_t hist = ~0ull, hist_s = ~0ull;
+  uint32_t hist_u = ~0u;
   {
     const int kf = kb < 1 ? 1 : kb;
     bw = load_rows(kf >> 3);
@@ -352,6 +374,10 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
   }
   RowBits rows_k = row_bits(kb, false);
   if ((rows_k.air | rows_k.solid) != 0xFFu) load_pm(kb);
+  // vmcnt(0): nothing may be in flight when the loop is entered. The compiler's wait for a row's
+  // loads counts the accesses issued after them on whichever way into the loop has fewest, so the
+  // few behind the first slice's loads would otherwise be the count on every iteration.
+  __builtin_amdgcn_s_waitcnt(0x0F70);
   __syncthreads();
 
   auto body = [&](auto cur_c, int k) __attribute__((always_inline)) {
@@ -359,12 +385,16 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
     // slices prev = cur ^ 1 hold k-1 (level i: k-1-i), cur hold k (k-i)
     hist = (hist << 8) | rows_k.air;
     hist_s = (hist_s << 8) | rows_k.solid;
+    hist_u = (hist_u << 8) | rows_k.same;
     const int hb = (k - 1) & 1;
     uint32_t ev_rows = 0;  // rows with an event on one of the slices k-L+1 .. k
     if (ev < ev_end) {
       while (ev < ev_end && ev_at(ev, 0) < k - (L - 1)) ++ev;
       for (int n = ev; n < ev_end && ev_at(n, 0) <= k; ++n) ev_rows |= 1u << (ev_at(n, 2) - yw);
     }
+    // the rows that are air, solid, of unchanged entries at every level, or have events: a byte each
+    const uint32_t kinds = all_of(hist, L) | (all_of(hist_s, L) << 8) |
+                           (all_of(hist_u, L - 1) << 16) | (ev_rows << 24);
     const RowBits rows_next = row_bits(k + 1, true);
     const auto ra = a_rsrc(k + 2), rb = b_rsrc(k + 1);
     const int sC = k - (L - 2), sD = k - (L - 1);
@@ -382,7 +412,9 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
     }
 
     // One row of every level. KIND 0: plain air at all of them; 1: the table; 2: the table and
-    // this row's events; 3: solid at all of them.
+    // this row's events; 3: solid at all of them; 4: the table, each node with one entry at all of
+    // them.
+    typename R::T raw_c{}, raw_d{};
     auto row = [&](auto kind, int r) __attribute__((always_inline)) {
       constexpr int KIND = decltype(kind)::value;
       constexpr bool TABLE = KIND == 1 || KIND == 2;
@@ -408,6 +440,12 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
         gather(1);
         __builtin_amdgcn_sched_barrier(0);
       }
+      CE one[NC];
+      if constexpr (KIND == 4) {
+#pragma unroll
+        for (int c = 0; c < NC; ++c) one[c] = s_coef[c == 0 ? pmr[r] & 0xFFFFu : pmr[r] >> 16];
+        __builtin_amdgcn_sched_barrier(0);
+      }
 #pragma unroll
       for (int i = 1; i <= L; ++i) {
         const V zn = t[i - 1];
@@ -424,24 +462,39 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
           }
         }
         const bool row_ok = !((hist_s >> (8 * (i - 1) + r)) & 1ull);
+        // both columns' chains side by side: one alone leaves its wave waiting on every result
+        if constexpr (KIND == 3) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) {
-          if constexpr (KIND == 3) {
-            t[i].v[c] = (C)0;
-            continue;
-          }
-          C u = zn.v[c] + zp.v[c];
-          u = u + yn.v[c];
-          u = u + yp.v[c];
-          u = u + x_next(ce, c);
-          u = u + x_prev(ce, c);
+          for (int c = 0; c < NC; ++c) t[i].v[c] = (C)0;
+        } else {
+          C u[NC], m[NC], o[NC];
+          auto each = [&](auto f) __attribute__((always_inline)) {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) f(c);
+            if constexpr (NC > 1) __builtin_amdgcn_sched_barrier(0);
+          };
+          each([&](int c) { u[c] = zn.v[c] + zp.v[c]; });
+          each([&](int c) { u[c] = u[c] + yn.v[c]; });
+          each([&](int c) { u[c] = u[c] + yp.v[c]; });
+          each([&](int c) { u[c] = u[c] + x_next(ce, c); });
+          each([&](int c) { u[c] = u[c] + x_prev(ce, c); });
           if constexpr (KIND == 0) {
-            t[i].v[c] = (air_tk * ce.v[c] + lam2 * u) - past.v[c];
-          } else if constexpr (TABLE) {
-            const CE &n = e[i & 1][c];
-            C v = n.inv * ((n.tk * ce.v[c] + lam2 * u) - n.omb * past.v[c]);
-            sw_keep(v);
-            t[i].v[c] = (row_ok && col_ok[c]) ? v : (C)0;
+            each([&](int c) { m[c] = air_tk * ce.v[c]; });
+            each([&](int c) { u[c] = lam2 * u[c]; });
+            each([&](int c) { u[c] = m[c] + u[c]; });
+            each([&](int c) { t[i].v[c] = u[c] - past.v[c]; });
+          } else {
+            auto entry = [&](int c) -> const CE & { return KIND == 4 ? one[c] : e[i & 1][c]; };
+            each([&](int c) { m[c] = entry(c).tk * ce.v[c]; });
+            each([&](int c) { u[c] = lam2 * u[c]; });
+            each([&](int c) { o[c] = entry(c).omb * past.v[c]; });
+            each([&](int c) { u[c] = m[c] + u[c]; });
+            each([&](int c) { u[c] = u[c] - o[c]; });
+            each([&](int c) {
+              C v = entry(c).inv * u[c];
+              sw_keep(v);
+              t[i].v[c] = ((KIND == 4 || row_ok) && col_ok[c]) ? v : (C)0;
+            });
           }
         }
         // rounded to the storage type once: the stored bits and the value the next level reads
@@ -456,55 +509,64 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
           for (int n = ev; n < ev_end && gev[4 * n] <= k; ++n) {
             if (gev[4 * n] != s || gev[4 * n + 2] != yw + r) continue;
             const int xe = gev[4 * n + 1], id = gev[4 * n + 3];
+            if (id < 0) {  // receiver
+              const bool owned = own_x && ((own_rows >> r) & 1u) && s >= z0 && s < z1;
+              const auto rr = sw_rsrc(ka->resp + (int64_t)(id & 0x7FFFFFFF) * ka->resp_steps,
+                                      (uint32_t)ka->resp_steps * 8u);
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-              if (xe != x0 + c) continue;
-              if (id < 0) {  // receiver
-                if (own_x && ((own_rows >> r) & 1u) && s >= z0 && s < z1)
-                  ka->resp[(int64_t)(id & 0x7FFFFFFF) * ka->resp_steps + step + i - 1] =
-                      (double)t[i].v[c] * ka->inv_scale;
-              } else if (step + i < ka->inject_end) {
-                C smp = (C)0;
-                if (step + i < ka->n_samples)
-                  smp = (C)ka->sig[(int64_t)id * ka->n_samples + step + i];
-                smp = smp * ka->scale;
-                const bool hard = ka->src_kind[id] == 0 || ka->soft_overwrite;
-                t[i].v[c] = Fmt<S>::round(hard ? smp : t[i].v[c] + smp);
+              for (int c = 0; c < NC; ++c) {
+                const double v = (double)t[i].v[c] * ka->inv_scale;
+                __builtin_amdgcn_raw_buffer_store_b64(
+                    __builtin_bit_cast(u32x2, v), rr,
+                    (int)((uint32_t)(step + i - 1) * 8u | (owned && xe == x0 + c ? 0u : kDrop)), 0, 0);
+              }
+            } else if (step + i < ka->inject_end) {
+              C smp = (C)0;
+              if (step + i < ka->n_samples)
+                smp = ((const __attribute__((address_space(4))) C *)ka->sig)[(int64_t)id * ka->n_samples + step + i];
+              smp = smp * ka->scale;
+              const bool hard = ((ConstI32)ka->src_kind)[id] == 0 || ka->soft_overwrite;
+#pragma unroll
+              for (int c = 0; c < NC; ++c) {
+                const C v = Fmt<S>::round(hard ? smp : t[i].v[c] + smp);
+                t[i].v[c] = xe == x0 + c ? v : t[i].v[c];
               }
             }
           }
         }
         if constexpr (KIND == 2) raw = R::pack(t[i]);
-        if (i >= L - 1 && i >= 1) {
-          const uint32_t off = (vst + r * rstep) | (((own_rows >> r) & 1u) ? 0u : kDrop);
-          const auto rs = i == L ? rD : rC;
-          if (KIND != 0 && x_odd) {
-#pragma unroll
-            for (int c = 0; c < NC; ++c)
-              R::st1(rs, (off | (x0 + c < X ? 0u : kDrop)) + c * (uint32_t)sizeof(S), raw, c);
-          } else {
-            R::st(rs, off, raw);
-          }
-        }
+        if (i == L - 1) raw_c = raw;
+        if (i == L) raw_d = raw;
       }
-      if constexpr (TABLE && L > 1) s_pm[((k & (RING - 1)) * TY + r) * 64] = (PM)pmr[r];
+      if constexpr ((TABLE || KIND == 4) && L > 1) s_pm[((k & (RING - 1)) * TY + r) * 64] = (PM)pmr[r];
 #pragma unroll
       for (int i = 0; i < L; ++i) q[i][cur ^ 1][r] = t[i];
-      __builtin_amdgcn_sched_barrier(0);
-      pl[r] = R::ld(ra, vcol + r * rstep);
-      pq[r] = R::ld(rb, vcol + r * rstep);
     };
     // the choice is made row by row: one choice for all rows would keep every queue entry of
     // the iteration live beside its replacement
     auto rows = [&](int r) __attribute__((always_inline)) {
-      if ((ev_rows >> r) & 1u)
+      if ((kinds >> (24 + r)) & 1u)
         row(std::integral_constant<int, 2>(), r);
-      else if (((hist >> r) & kRowAir) == kRowAir)
+      else if ((kinds >> r) & 1u)
         row(std::integral_constant<int, 0>(), r);
-      else if (((hist_s >> r) & kRowAir) == kRowAir)
+      else if ((kinds >> (8 + r)) & 1u)
         row(std::integral_constant<int, 3>(), r);
+      else if ((kinds >> (16 + r)) & 1u)
+        row(std::integral_constant<int, 4>(), r);
       else
         row(std::integral_constant<int, 1>(), r);
+      // The accesses are the same on every way here: a wait for a row's loads counts the accesses
+      // issued since on the way with fewest, and the compiler makes ways past all of the kinds.
+      __builtin_amdgcn_sched_barrier(0);
+      const uint32_t drop = ((own_rows >> r) & 1u) ? 0u : kDrop;
+      if (L >= 2) R::st(rC, (vst + r * rstep) | drop, raw_c);
+      R::st(rD, (vst + r * rstep) | drop, raw_d);
+      if (odd_edge) {
+        if (L >= 2) R::st1(rC, (vst1 + r * rstep) | drop, raw_c, 0);
+        R::st1(rD, (vst1 + r * rstep) | drop, raw_d, 0);
+      }
+      pl[r] = R::ld(ra, vcol + r * rstep);
+      pq[r] = R::ld(rb, vcol + r * rstep);
     };
 #pragma unroll
     for (int r = 1; r < TY - 1; ++r) rows(r);
@@ -517,7 +579,8 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
       *halo_at(hb ^ 1, i, wave, 1) = q[i][cur ^ 1][TY - 1];
     }
     rows_k = rows_next;
-    if ((rows_k.air | rows_k.solid) != 0xFFu) load_pm(k + 1);
+    // entries of the slice below stay in their registers
+    if ((rows_k.air | rows_k.solid | rows_k.same) != 0xFFu) load_pm(k + 1);
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
@@ -621,10 +684,11 @@ hipError_t launch_pack_entry(const uint8_t *pos, const uint8_t *mat, uint16_t *p
   return hipGetLastError();
 }
 
-// Two bytes per (wave tile, slice), 8 slices to a pair of words: bit r of the first is set when the
+// Three bytes per (wave tile, slice), 8 slices to three words: bit r of the first is set when the
 // tile's row r is plain air over its whole window (and inside the grid), of the second when no
-// voxel of it is updated (outside voxels, or past the grid). Bits past the tile's rows are set in
-// both. A wave per tile and word.
+// voxel of it is updated (outside voxels, or past the grid), of the third when its entries are
+// those of the slice below (never on slice 1 or outside 1..Z-2). Bits past the tile's rows are set
+// in all. A wave per tile and word.
 __global__ __launch_bounds__(64) void row_bits_kernel(const uint16_t *__restrict__ pm, int pitch,
                                                       uint64_t *__restrict__ out, int X, int Y,
                                                       int Z, int nbx, int ox, int hx, int w,
@@ -635,14 +699,14 @@ __global__ __launch_bounds__(64) void row_bits_kernel(const uint16_t *__restrict
   const int xs = bx * ox - hx, ys = (tw / wy) * oy - lm + (tw % wy) * ty;
   const bool x_in = xs >= 0 && xs + w <= X;
   for (int word = blockIdx.z; word < words; word += gridDim.z) {
-    uint64_t air = 0, solid = 0;
+    uint64_t air = 0, solid = 0, same = 0;
     for (int b = 0; b < 8; ++b) {
       const int z = 8 * word + b;
-      uint32_t ma = (0xFFu << ty) & 0xFFu, ms = ma;
+      uint32_t ma = (0xFFu << ty) & 0xFFu, ms = ma, mu = ma;
       const uint16_t *slice = pm + (size_t)min(z, Z - 1) * (size_t)pitch * (size_t)Y;
       for (int r = 0; r < ty; ++r) {
         const int y = ys + r;
-        bool not_air = !x_in, not_solid = false;
+        bool not_air = !x_in, not_solid = false, changed = z < 2 || z > Z - 2;
         if (y < 0 || y >= Y || z >= Z) {
           not_air = true;
         } else {
@@ -651,18 +715,22 @@ __global__ __launch_bounds__(64) void row_bits_kernel(const uint16_t *__restrict
             const unsigned v = slice[(size_t)y * pitch + xs + c];
             not_air = not_air || v < 6u * ncol || v >= kStageRows * ncol;
             not_solid = not_solid || v < kStageRows * ncol;
+            if (!changed) changed = v != slice[(size_t)y * pitch + xs + c - (size_t)pitch * Y];
           }
         }
         if (__ballot(not_air) == 0) ma |= 1u << r;
         if (__ballot(not_solid) == 0) ms |= 1u << r;
+        if (__ballot(changed) == 0) mu |= 1u << r;
       }
       air |= (uint64_t)ma << (8 * b);
       solid |= (uint64_t)ms << (8 * b);
+      same |= (uint64_t)mu << (8 * b);
     }
     if (lane == 0) {
-      const size_t o = 2 * (((size_t)tw * nbx + bx) * words + word);
+      const size_t o = 3 * (((size_t)tw * nbx + bx) * words + word);
       out[o] = air;
       out[o + 1] = solid;
+      out[o + 2] = same;
     }
   }
 }
@@ -791,9 +859,6 @@ hipError_t launch_any(const SweepPlan &p, const A &a, int levels, hipStream_t st
     break;
   case 5:
     if constexpr (SweepTile<S>::LM >= 5) return launch_levels<S, 5>(p, a, stream);
-    break;
-  case 6:
-    if constexpr (SweepTile<S>::LM >= 6) return launch_levels<S, 6>(p, a, stream);
     break;
   }
   return hipErrorInvalidValue;
