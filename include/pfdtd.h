@@ -40,7 +40,7 @@ extern "C" {
 /* FP32 arithmetic, binary16 storage of P^n and D^n = P^n - P^{n-1} (difference form, power-of-two
  * scaled; no reference counterpart): a storage rounding of P no longer changes the velocity
  * P^n - P^{n-1}, which cuts the in-band error growth of the scheme's marginal low-frequency
- * modes. pfdtd_run only, through the two-column sweep: forward update, X even, no batch, no
+ * modes. pfdtd_run only, through the several-level sweep: forward update, X even, no batch, no
  * source on the slices z = 0 or Z-1. pfdtd_get_fields_raw returns P and D. */
 #define PFDTD_F16_DIFF 4
 
@@ -64,8 +64,8 @@ extern "C" {
                                 three-level sweep: 58 columns) */
 #define PFDTD_SWEEP_WIDE 2   /* FP32: blocks of 4 x 4 wave tiles (240 columns, 1024 threads) */
 #define PFDTD_SWEEP_PAIR 3   /* 16-bit storage, X even: two columns per lane (124-column wave
-                                tiles in blocks of 2 x 2, the difference form 1 x 4; one
-                                32-bit access per pair); otherwise as AUTO */
+                                tiles in blocks of 2 x 2; one 32-bit access per pair);
+                                otherwise as AUTO */
 
 typedef struct pfdtd_ctx pfdtd_ctx;
 
@@ -287,17 +287,20 @@ int pfdtd_set_kernel_timing(pfdtd_ctx *ctx, int enabled);
  * PROGRESS_MOD in src/kernels/kernels3d.h:36). The reference polls the interrupt every step
  * (kernels3d.cu:86); polling here costs one stream synchronisation per interval. */
 int pfdtd_set_poll_interval(pfdtd_ctx *ctx, int steps);
-/* Time levels advanced per sweep of the field (1, 2 or 3; 0 = default: 3 for FP32 and FP64
- * (unbatched or grouped batches), else 2 -- the faster settings on MI355X) and slices per z-chunk of the sweep
- * (0 = automatic: the longest of 32 (16-bit storage: 22 for the two-column sweep, 16 for the
- * difference form and one column), 16 and 8 slices that gives the two-level sweep 4096 blocks; the three-level sweep 2048 blocks, from 32 slices (FP64: 96)
+/* Time levels advanced per sweep of the field (1, 2 or 3; 0 = default: the several-level sweep, 5
+ * levels (FP64: 4), where it can run -- no source on slice z = 0 or Z-1, sweep shape AUTO, room for
+ * its planes -- else 3 for FP32 and FP64 (unbatched or grouped batches) and 2 otherwise; the
+ * difference form always takes the several-level sweep) and slices per z-chunk of the sweep
+ * (0 = automatic: the several-level sweep by the blocks it gives; the longest of 32 (16-bit
+ * storage: 22 for the two-column sweep, 16 for one column), 16 and 8 slices that gives the two-level sweep 4096 blocks; the three-level sweep 2048 blocks, from 32 slices (FP64: 96)
  * down). With 2, pfdtd_run advances pairs of
  * steps in one kernel that reads P^n, P^{n-1} and the byte planes once and writes P^{n+1} and
- * P^{n+2}; with 3 (forward update; the centred one and the difference form take 2), triples of
+ * P^{n+2}; with 3 (forward update; the centred one takes 2), triples of
  * steps in one kernel that writes only P^{n+2} and P^{n+3}. Sources are injected and receivers
  * gathered inside the kernel; four field buffers. A remainder of one step takes a single-step
  * update (so does every step while a source sits on slice z = 0 or z = Z-1), four steps left
- * take two pairs. Non-grouped batches advance one level per sweep. Results are bit-identical
+ * take two pairs. Non-grouped batches advance one level per sweep
+ * with an explicit setting and are held slot by slot for the several-level sweep. Results are bit-identical
  * to single steps. No reference counterpart: the reference's loop (kernels3d.cu:83-191)
  * launches one update per step. */
 int pfdtd_set_time_levels(pfdtd_ctx *ctx, int levels, int zchunk);

@@ -651,8 +651,6 @@ Fused2Args<S, CT, C> fused_args(const pfdtd_ctx *c, const CT *coef, CT air, C la
   a.sig_d = c->d_sig_d;
   a.n_samples = c->n_samples;
   a.inject_step = (c->n_src > 0 && step + 1 < c->resp_steps) ? step + 1 : -1;
-  a.levels = 2;
-  a.diff = c->precision == PFDTD_F16_DIFF ? 1 : 0;
   if (slot_major(c) && c->lgB > 0) {
     a.n_slots = 1 << c->lgB;
     a.slot_elems = c->N;
@@ -669,14 +667,8 @@ Fused2Args<S, CT, C> fused_args(const pfdtd_ctx *c, const CT *coef, CT air, C la
   return a;
 }
 
-// Steps `step` and `step+1` in one sweep: P^{step+1} lands in d_Pp2, P^{step+2} in d_P2. The
-// difference form stores P in d_P2 and D in d_Pp2 after `levels` steps (2, or 1 for its last).
-hipError_t launch_update2_any(pfdtd_ctx *c, const FusedGeom &g, int step, int levels = 2) {
-  if (c->precision == PFDTD_F16_DIFF) {
-    auto a = fused_args<h16>(c, c->d_coef_f, c->air_f, c->lam2_f, step, g.pair);
-    a.levels = levels;
-    return launch_update2_f16(g, a, c->stream);
-  }
+// Steps `step` and `step+1` in one sweep: P^{step+1} lands in d_Pp2, P^{step+2} in d_P2.
+hipError_t launch_update2_any(pfdtd_ctx *c, const FusedGeom &g, int step) {
   switch (c->precision) {
   case PFDTD_F32:
     return launch_update2_f32(
@@ -702,7 +694,6 @@ template <typename S, typename CT, typename C>
 Fused2Args<S, CT, C> fused3_args(const pfdtd_ctx *c, const CT *coef, CT air, C lam2, int step) {
   auto a = fused_args<S>(c, coef, air, lam2, step, false);
   a.air_rows = c->d_air_rows3;
-  a.levels = 3;
   a.gather_step2 = c->n_rec > 0 ? step + 1 : -1;
   a.inject_step2 = (c->n_src > 0 && step + 2 < c->resp_steps) ? step + 2 : -1;
   return a;
@@ -895,7 +886,7 @@ SweepArgs<S, CT, C> sweep_args(const pfdtd_ctx *c, const SweepPlan &p, const CT 
 }
 
 // Steps `step` .. `step + levels - 1` in one sweep, gathers and injections included; the new
-// current and past fields are in d_P and d_Pp afterwards.
+// current and past fields (the difference form: P and D) are in d_P and d_Pp afterwards.
 hipError_t run_sweep(pfdtd_ctx *c, const SweepPlan &p, int step, int levels, int inject_end) {
   hipError_t e;
   auto args = [&](auto tag) {
@@ -908,10 +899,11 @@ hipError_t run_sweep(pfdtd_ctx *c, const SweepPlan &p, int step, int levels, int
                                                step, inject_end), levels, c->stream);
     break;
   case PFDTD_F16: e = launch_sweep_f16(p, args(h16{}), levels, c->stream); break;
+  case PFDTD_F16_DIFF: e = launch_sweep_diff(p, args(h16{}), levels, c->stream); break;
   case PFDTD_BF16: e = launch_sweep_bf16(p, args(b16{}), levels, c->stream); break;
   default: e = launch_sweep_f32(p, args(float{}), levels, c->stream);
   }
-  if (levels > 1) {
+  if (levels > 1 || c->precision == PFDTD_F16_DIFF) {
     std::swap(c->d_P, c->d_P2);
     std::swap(c->d_Pp, c->d_Pp2);
   } else {  // one level writes P^{n+1} only: P^n becomes the past field
@@ -1445,7 +1437,7 @@ int pfdtd_run(pfdtd_ctx *c, int precision, int n_steps, pfdtd_interrupt_cb inter
   const bool diff = precision == PFDTD_F16_DIFF;
   if (diff && (!fused_eligible(c) || c->scheme != 0 || c->X % 2 != 0 || c->lgB > 0 ||
                c->X * c->Y * 2 >= ((int64_t)1 << 31)))
-    return fail(PFDTD_E_STATE, "the difference form runs through the two-column sweep only: forward "
+    return fail(PFDTD_E_STATE, "the difference form runs through the several-level sweep only: forward "
                 "update, X even, X*Y below 2^30, no batch, no source on the slices z = 0 or Z-1");
   rc = zero_fields(c);
   if (rc) return rc;
@@ -1469,23 +1461,23 @@ int pfdtd_run(pfdtd_ctx *c, int precision, int n_steps, pfdtd_interrupt_cb inter
     HIP_TRY(launch_inject_gather(p_storage(c->precision), c->d_P, ia, c->stream));
   }
 
-  bool sweep = !diff && sweep_eligible(c);
+  bool sweep = diff || sweep_eligible(c);
   SweepPlan sp{};
   if (sweep) {
     sp = plan_sweep(c->precision, (int)c->X, (int)c->Y, (int)c->Z, c->fzc, batch_slots(c));
     rc = ensure_sweep(c, sp, &sweep);
     if (rc) return rc;
+    if (diff && !sweep)
+      return fail(PFDTD_E_NOMEM, "no room for the entry plane the difference form's sweep reads");
   }
   bool fused = !sweep && fused_eligible(c);
   rc = ensure_pm(c, &fused);
   if (rc) return rc;
   const FusedGeom fg = plan_fused((int)c->X, (int)c->Y, (int)c->Z, c->fzc, c->precision,
-                                  diff ? PFDTD_SWEEP_PAIR : c->fshape, c->scheme, batch_slots(c));
-  if (diff && (!fused || !fg.pair))
-    return fail(PFDTD_E_NOMEM, "no room for the packed plane the two-column sweep reads");
-  // three levels per sweep with the forward scheme when asked for (not the difference form);
-  // the centred scheme takes the two-level sweep
-  const bool three = fused && !diff && c->scheme == 0 && levels_for(c, c->precision) == 3;
+                                  c->fshape, c->scheme, batch_slots(c));
+  // three levels per sweep with the forward scheme when asked for; the centred scheme takes the
+  // two-level sweep
+  const bool three = fused && c->scheme == 0 && levels_for(c, c->precision) == 3;
   FusedGeom fg3;
   if (three) {
     fg3 = plan_fused3((int)c->X, (int)c->Y, (int)c->Z, c->fzc, c->precision, c->fshape,
@@ -1532,24 +1524,11 @@ int pfdtd_run(pfdtd_ctx *c, int precision, int n_steps, pfdtd_interrupt_cb inter
         ++nev;
         // P^{step+2} (d_P2): gather step+1, inject step+2
         const int next = step + 2 < n_steps ? step + 2 : -1;
-        InjectArgs ia = inject_args(c, step + 1, next);
-        if (diff) ia.dfield = c->d_Pp2;
-        HIP_TRY(launch_inject_gather(p_storage(c->precision), c->d_P2, ia, c->stream));
+        HIP_TRY(launch_inject_gather(c->precision, c->d_P2, inject_args(c, step + 1, next), c->stream));
         std::swap(c->d_P, c->d_P2);
         std::swap(c->d_Pp, c->d_Pp2);
         k += 2;
         c->upd_launches += 2;
-      } else if (diff) {
-        // the difference form's odd last step: one level of the sweep (gather of `step` and the
-        // injection of step+1 happen inside it)
-        if (c->kernel_timing) HIP_TRY(hipEventRecord(c->events[2 * nev], c->stream));
-        HIP_TRY(launch_update2_any(c, fg, step, 1));
-        if (c->kernel_timing) HIP_TRY(hipEventRecord(c->events[2 * nev + 1], c->stream));
-        ++nev;
-        std::swap(c->d_P, c->d_P2);
-        std::swap(c->d_Pp, c->d_Pp2);
-        k += 1;
-        c->upd_launches += 1;
       } else {
         if (c->kernel_timing) HIP_TRY(hipEventRecord(c->events[2 * nev], c->stream));
         HIP_TRY(launch_update_any(c, g));

@@ -170,12 +170,10 @@ struct Fused2Args {
   double *resp;
   int resp_steps;
   int gather_step;
-  int levels = 2;  // time levels of this launch (1 only for the difference form's last step)
   // three-level sweep: the receivers of step gather_step2 are gathered on P^{n+2} before the
   // sources of step inject_step2 are injected into it (-1: none)
   int gather_step2 = -1;
   int inject_step2 = -1;
-  int diff = 0;    // 1: the difference form (B holds D = P^n - P^{n-1}; 16-bit storage only)
   // Grouped batch (slot-outermost fields): the launch advances n_slots source configurations,
   // slot s's fields at element offset s * slot_elems; sources and receivers carry their slot.
   int n_slots = 1;
@@ -312,6 +310,9 @@ hipError_t launch_sweep_f32(const SweepPlan &p, const SweepArgs<float, CoefF, fl
                             hipStream_t stream);
 hipError_t launch_sweep_f16(const SweepPlan &p, const SweepArgs<h16, CoefF, float> &a, int levels,
                             hipStream_t stream);
+// The difference form: D^n in B, P^{n+L} to Dn and D^{n+L} to Cn.
+hipError_t launch_sweep_diff(const SweepPlan &p, const SweepArgs<h16, CoefF, float> &a, int levels,
+                             hipStream_t stream);
 hipError_t launch_sweep_bf16(const SweepPlan &p, const SweepArgs<b16, CoefF, float> &a, int levels,
                              hipStream_t stream);
 hipError_t launch_sweep_f64(const SweepPlan &p, const SweepArgs<double, CoefD, double> &a, int levels,

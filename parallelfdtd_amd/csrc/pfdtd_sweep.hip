@@ -44,6 +44,11 @@
 // Sixteen waves of 3 rows each (four waves per SIMD, 4 levels to fit 128 registers) take 371 on the
 // hall and 28.6 on 256x256x256.
 //
+// The difference form (A holds P^n, B holds D^n = P^n - P^{n-1}; P^{n+L} to Dn and D^{n+L} to Cn, both
+// from the last level) also keeps every level's rounded differences of one slice; the past value of a
+// node is P - D in FP32, and a sample keeps it. 249 VGPRs. 640x480x320 hall, 400 steps: 66.7 ms with
+// the two-level sweep of independent waves -> 52.7.
+//
 // Loads, stores and masks. Slices are accessed through buffer descriptors: rows and columns past
 // the grid read 0, stores that a lane or row does not own are given an offset past the slice and
 // dropped, so the body has no masked branches. The loads of the next slice are issued as soon as a
@@ -187,7 +192,7 @@ using ConstSweepArgs = const __attribute__((address_space(4))) SweepArgsOf<S> *;
 
 // One block of a sweep: tile `tile` of nbx x nby x (z-chunks of zc slices), fields fA, fB to fC, fD,
 // first step `step`.
-template <typename S, int L, int LM, int TY, int WY, int NC, int HX>
+template <typename S, int L, int LM, int TY, int WY, int NC, int HX, bool DIFF>
 __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned tile, int slot, int zc,
                                             const S *__restrict__ gA, const S *__restrict__ gB,
                                             S *__restrict__ gC, S *__restrict__ gD, int step) {
@@ -247,6 +252,10 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
     const int br = wave * TY + r, y = yw + r;
     if (br >= LM && br < LM + OY && y < Y) own_rows |= 1u << r;
   }
+  uint32_t upd_rows = 0;  // rows of 1..Y-2 (the difference form)
+#pragma unroll
+  for (int r = 0; r < TY; ++r)
+    if (yw + r > 0 && yw + r < Y - 1) upd_rows |= 1u << r;
   bool col_ok[NC];
 #pragma unroll
   for (int c = 0; c < NC; ++c) col_ok[c] = x0 + c > 0 && x0 + c < X - 1;
@@ -272,7 +281,8 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
   };
 
   V q[L][2][TY];  // level 0: P^n, level i: P^{n+i}; two slices each
-  typename R::T pl[TY], pq[TY];  // raw P^n[k+1] and P^{n-1}[k]
+  typename R::T pl[TY], pq[TY];  // raw P^n[k+1] and P^{n-1}[k] (the difference form: D^n[k])
+  typename R::T qd[L][TY];       // the difference form: raw D of level i's slice k-i (i > 0)
   uint32_t pmr[TY];              // packed entries of slice k where it is not all air
 #pragma unroll
   for (int i = 0; i < L; ++i)
@@ -283,7 +293,11 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
 #pragma unroll
         for (int c = 0; c < NC; ++c) q[i][b][r].v[c] = (C)0;
 #pragma unroll
-  for (int r = 0; r < TY; ++r) pmr[r] = 0;
+  for (int r = 0; r < TY; ++r) {
+    pmr[r] = 0;
+#pragma unroll
+    for (int i = 0; i < L; ++i) qd[i][r] = typename R::T{};
+  }
 
   auto a_rsrc = [&](int k) {
     const bool in = k >= 0 && k < Z;
@@ -398,8 +412,8 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
     const RowBits rows_next = row_bits(k + 1, true);
     const auto ra = a_rsrc(k + 2), rb = b_rsrc(k + 1);
     const int sC = k - (L - 2), sD = k - (L - 1);
-    const bool inC = L >= 2 && sC >= z0 && sC < z1, inD = sD >= z0 && sD < z1;
-    const auto rC = sw_rsrc(gC + (inC ? (size_t)sC * XY : 0), inC ? sbytes : 0u);
+    const bool inD = sD >= z0 && sD < z1, inC = DIFF ? inD : L >= 2 && sC >= z0 && sC < z1;
+    const auto rC = sw_rsrc(gC + (inC ? (size_t)(DIFF ? sD : sC) * XY : 0), inC ? sbytes : 0u);
     const auto rD = sw_rsrc(gD + (inD ? (size_t)sD * XY : 0), inD ? sbytes : 0u);
     // row offsets are formed where used: kept across the sweep they would hold 2 TY registers
     uint32_t rstep = (uint32_t)X * (uint32_t)sizeof(S);
@@ -424,6 +438,7 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
       V t[L + 1];
       t[0] = R::up(pl[r]);
       const V past0 = R::up(pq[r]);
+      typename R::T d_in = pq[r], d_out{};
       auto gather = [&](int i) __attribute__((always_inline)) {
         if ((hist >> (8 * (i - 1) + r)) & 1ull)
           pm[i] = air_pm;
@@ -453,7 +468,13 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
         const V ce = q[i - 1][cur][r];
         const V yn = r + 1 < TY ? q[i - 1][cur][r + 1 < TY ? r + 1 : r] : hd[i - 1];
         const V yp = r > 0 ? q[i - 1][cur][r > 0 ? r - 1 : r] : hu[i - 1];
-        const V past = i == 1 ? past0 : q[i >= 2 ? i - 2 : 0][cur ^ 1][r];
+        V past = i == 1 ? past0 : q[i >= 2 ? i - 2 : 0][cur ^ 1][r];
+        V e_new;  // the level's difference, before rounding
+        if constexpr (DIFF) {
+          const V d = R::up(d_in);
+#pragma unroll
+          for (int c = 0; c < NC; ++c) past.v[c] = ce.v[c] - d.v[c];
+        }
         const int s = k - (i - 1);
         if constexpr (TABLE) {
           if (i < L) {  // the next level's entries are in flight during this level
@@ -465,7 +486,10 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
         // both columns' chains side by side: one alone leaves its wave waiting on every result
         if constexpr (KIND == 3) {
 #pragma unroll
-          for (int c = 0; c < NC; ++c) t[i].v[c] = (C)0;
+          for (int c = 0; c < NC; ++c) {
+            t[i].v[c] = (C)0;
+            e_new.v[c] = col_ok[c] && ((upd_rows >> r) & 1u) ? (C)0 - ce.v[c] : (C)0;
+          }
         } else {
           C u[NC], m[NC], o[NC];
           auto each = [&](auto f) __attribute__((always_inline)) {
@@ -483,6 +507,7 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
             each([&](int c) { u[c] = lam2 * u[c]; });
             each([&](int c) { u[c] = m[c] + u[c]; });
             each([&](int c) { t[i].v[c] = u[c] - past.v[c]; });
+            if constexpr (DIFF) each([&](int c) { e_new.v[c] = t[i].v[c] - ce.v[c]; });
           } else {
             auto entry = [&](int c) -> const CE & { return KIND == 4 ? one[c] : e[i & 1][c]; };
             each([&](int c) { m[c] = entry(c).tk * ce.v[c]; });
@@ -495,11 +520,18 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
               sw_keep(v);
               t[i].v[c] = ((KIND == 4 || row_ok) && col_ok[c]) ? v : (C)0;
             });
+            if constexpr (DIFF)
+              each([&](int c) {
+                C d = t[i].v[c] - ce.v[c];
+                sw_keep(d);
+                e_new.v[c] = col_ok[c] && (KIND == 4 || ((upd_rows >> r) & 1u)) ? d : (C)0;
+              });
           }
         }
         // rounded to the storage type once: the stored bits and the value the next level reads
         typename R::T raw = R::pack(t[i]);
         if (i < L || KIND == 2) t[i] = R::up(raw);
+        if constexpr (DIFF) d_out = R::pack(e_new);
         if constexpr (KIND == 2) {
           // the event arguments are re-read here, so that they hold no scalar registers across
           // the sweep
@@ -529,13 +561,28 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
 #pragma unroll
               for (int c = 0; c < NC; ++c) {
                 const C v = Fmt<S>::round(hard ? smp : t[i].v[c] + smp);
+                if constexpr (DIFF) {  // the difference keeps the past value
+                  V d = R::up(d_out);
+                  const C e = v - (t[i].v[c] - d.v[c]);
+                  d.v[c] = xe == x0 + c ? e : d.v[c];
+                  d_out = R::pack(d);
+                }
                 t[i].v[c] = xe == x0 + c ? v : t[i].v[c];
               }
             }
           }
         }
         if constexpr (KIND == 2) raw = R::pack(t[i]);
-        if (i == L - 1) raw_c = raw;
+        if constexpr (DIFF) {
+          if (i < L) {  // the next level's difference gives way to this one's
+            d_in = qd[i < L ? i : 0][r];
+            qd[i < L ? i : 0][r] = d_out;
+          } else {
+            raw_c = d_out;
+          }
+        } else {
+          if (i == L - 1) raw_c = raw;
+        }
         if (i == L) raw_d = raw;
       }
       if constexpr ((TABLE || KIND == 4) && L > 1) s_pm[((k & (RING - 1)) * TY + r) * 64] = (PM)pmr[r];
@@ -559,10 +606,10 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
       // issued since on the way with fewest, and the compiler makes ways past all of the kinds.
       __builtin_amdgcn_sched_barrier(0);
       const uint32_t drop = ((own_rows >> r) & 1u) ? 0u : kDrop;
-      if (L >= 2) R::st(rC, (vst + r * rstep) | drop, raw_c);
+      if (L >= 2 || DIFF) R::st(rC, (vst + r * rstep) | drop, raw_c);
       R::st(rD, (vst + r * rstep) | drop, raw_d);
       if (odd_edge) {
-        if (L >= 2) R::st1(rC, (vst1 + r * rstep) | drop, raw_c, 0);
+        if (L >= 2 || DIFF) R::st1(rC, (vst1 + r * rstep) | drop, raw_c, 0);
         R::st1(rD, (vst1 + r * rstep) | drop, raw_d, 0);
       }
       pl[r] = R::ld(ra, vcol + r * rstep);
@@ -602,12 +649,12 @@ __device__ __forceinline__ unsigned xcd_tile() {
 
 // A context's sweep: the slots of a batch innermost, so that one XCD's L2 serves a tile's entries
 // to all of them.
-template <typename S, int L, int LM, int TY, int WY, int NC, int HX>
+template <typename S, int L, int LM, int TY, int WY, int NC, int HX, bool DIFF>
 __global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_kernel(SweepArgsOf<S> a) {
   const unsigned tile = xcd_tile();
   const int slot = (int)(tile % (unsigned)a.n_slots);
   const int64_t off = (int64_t)slot * a.slot_elems;
-  sweep_block<S, L, LM, TY, WY, NC, HX>(
+  sweep_block<S, L, LM, TY, WY, NC, HX, DIFF>(
       (ConstSweepArgs<S>)__builtin_amdgcn_kernarg_segment_ptr(), tile / (unsigned)a.n_slots, slot,
       a.zc, a.A + off, a.B + off, a.Cn + off, a.Dn + off, a.step);
 }
@@ -636,7 +683,7 @@ __global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_pool_kernel(
   int o1, o2;
   pool_spare(st.cur, st.past, o1, o2);
   const bool odd = round & 1;
-  sweep_block<S, L, LM, TY, WY, NC, HX>(
+  sweep_block<S, L, LM, TY, WY, NC, HX, false>(
       (ConstSweepArgs<S>)(args + job), (unsigned)(tile - (lo ? pl.tile_end[lo - 1] : 0)), 0, zc,
       (const S *)J.F[odd ? o2 : st.cur], (const S *)J.F[odd ? o1 : st.past],
       (S *)J.F[odd ? st.past : o1], (S *)J.F[odd ? st.cur : o2], step);
@@ -839,26 +886,26 @@ size_t sweep_lds(int ncol) {
          2 * T::NC * (size_t)T::WY * sweep_ring(L) * T::TY * 64;
 }
 
-template <typename S, int L>
+template <typename S, int L, bool DIFF>
 hipError_t launch_levels(const SweepPlan &p, const SweepArgsOf<S> &a, hipStream_t stream) {
   typedef SweepTile<S> T;
   const size_t lds = sweep_lds<S, L>(a.ncol);
-  hipLaunchKernelGGL((srl_sweep_kernel<S, L, T::LM, T::TY, T::WY, T::NC, T::HX>), dim3((unsigned)p.blocks),
-                     dim3(64 * T::WY), lds, stream, a);
+  hipLaunchKernelGGL((srl_sweep_kernel<S, L, T::LM, T::TY, T::WY, T::NC, T::HX, DIFF>),
+                     dim3((unsigned)p.blocks), dim3(64 * T::WY), lds, stream, a);
   return hipGetLastError();
 }
 
-template <typename S, typename A>
+template <typename S, bool DIFF = false, typename A>
 hipError_t launch_any(const SweepPlan &p, const A &a, int levels, hipStream_t stream) {
   switch (levels) {
-  case 1: return launch_levels<S, 1>(p, a, stream);
-  case 2: return launch_levels<S, 2>(p, a, stream);
-  case 3: return launch_levels<S, 3>(p, a, stream);
+  case 1: return launch_levels<S, 1, DIFF>(p, a, stream);
+  case 2: return launch_levels<S, 2, DIFF>(p, a, stream);
+  case 3: return launch_levels<S, 3, DIFF>(p, a, stream);
   case 4:
-    if constexpr (SweepTile<S>::LM >= 4) return launch_levels<S, 4>(p, a, stream);
+    if constexpr (SweepTile<S>::LM >= 4) return launch_levels<S, 4, DIFF>(p, a, stream);
     break;
   case 5:
-    if constexpr (SweepTile<S>::LM >= 5) return launch_levels<S, 5>(p, a, stream);
+    if constexpr (SweepTile<S>::LM >= 5) return launch_levels<S, 5, DIFF>(p, a, stream);
     break;
   }
   return hipErrorInvalidValue;
@@ -899,6 +946,7 @@ hipError_t launch_pool_rotate(const PoolJobDev *jobs, PoolState *st, const PoolL
 SweepPlan plan_sweep(int precision, int X, int Y, int Z, int zc, int slots) {
   switch (precision) {
   case PFDTD_F64: return plan_of<double>(X, Y, Z, zc, slots);
+  case PFDTD_F16_DIFF:
   case PFDTD_F16: return plan_of<h16>(X, Y, Z, zc, slots);
   case PFDTD_BF16: return plan_of<b16>(X, Y, Z, zc, slots);
   default: return plan_of<float>(X, Y, Z, zc, slots);
@@ -960,6 +1008,10 @@ hipError_t launch_sweep_f32(const SweepPlan &p, const SweepArgsOf<float> &a, int
 hipError_t launch_sweep_f16(const SweepPlan &p, const SweepArgsOf<h16> &a, int levels,
                             hipStream_t stream) {
   return launch_any<h16>(p, a, levels, stream);
+}
+hipError_t launch_sweep_diff(const SweepPlan &p, const SweepArgsOf<h16> &a, int levels,
+                             hipStream_t stream) {
+  return launch_any<h16, true>(p, a, levels, stream);
 }
 hipError_t launch_sweep_bf16(const SweepPlan &p, const SweepArgsOf<b16> &a, int levels,
                              hipStream_t stream) {

@@ -133,3 +133,18 @@ def test_interleaved_batch_agrees_with_grouped_and_steps(gpu, prec, B, dims):
     for a, b in zip(*out):
         assert np.array_equal(a, b)
     assert all(f.any() for f in out[0][1])  # every slot holds its own source
+
+
+@pytest.mark.parametrize("dx,dy,z,zchunk", [(-2, 1, 9, 0), (0, -1, 12, 3), (2, 0, 21, 5), (8, 5, 8, 1)])
+@pytest.mark.parametrize("n_steps", [23, 4])
+def test_difference_form_at_tile_borders(gpu, dx, dy, z, zchunk, n_steps):
+    """P and D of the difference form either side of a tile border, every remainder of the levels,
+    sources in solid voxels and on two tiles' shared columns."""
+    from test_gpu_diff import run_diff
+    ox, oy = OWNED[N.F16]
+    sc = scene(980 + dx, (ox + dx, 2 * oy + dy, z), n_steps, n_boxes=12)
+    sc.src_xyz[0] = [ox - 3, oy, z // 2]
+    sc.labels[z // 2, oy + 3, 5:9] = 1
+    sc.src_xyz[1] = [6, oy + 3, z // 2]
+    sc.rec_xyz[0] = sc.src_xyz[0]
+    run_diff(sc, 9, zchunk=zchunk, poll=7)
