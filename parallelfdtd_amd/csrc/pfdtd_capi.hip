@@ -779,10 +779,10 @@ int build_sweep_events(pfdtd_ctx *c, const SweepPlan &p) {
   return PFDTD_OK;
 }
 
-// Whether the sweep can take runs of this precision: the forward scheme, slices below 2^31 bytes,
-// the automatic settings, and no source on the never-updated slices.
+// Whether the sweep can take runs of this precision: slices below 2^31 bytes, the
+// automatic settings, and no source on the never-updated slices.
 bool sweep_takes(const pfdtd_ctx *c, int precision) {
-  if (c->scheme != 0 || c->levels != 0 || c->fshape != PFDTD_SWEEP_AUTO) return false;
+  if (c->levels != 0 || c->fshape != PFDTD_SWEEP_AUTO) return false;
   if (precision == PFDTD_F16_DIFF || boundary_source(c)) return false;
   return (uint64_t)c->X * (uint64_t)c->Y * elem_size(precision) < (1ull << 31);
 }
@@ -823,13 +823,13 @@ int ensure_sweep(pfdtd_ctx *c, const SweepPlan &p, bool *ok) {
     e = grow(c->d_entry, c->entry_cap, (size_t)p.pitch * c->Y * c->Z);
     if (e == hipSuccess)
       e = launch_pack_entry(c->d_pos, c->d_mat, c->d_entry, (int)c->X, (int)c->Y, (int)c->Z,
-                            p.pitch, ncol, c->stream);
+                            p.pitch, ncol, c->scheme, c->stream);
   }
   if (e == hipSuccess && (!c->entry_ok || !same)) {
     e = grow(c->d_row_bits, c->air_cap, sweep_row_words(p));
     if (e == hipSuccess)
       e = launch_row_bits(p, c->d_entry, c->d_row_bits, (int)c->X, (int)c->Y, (int)c->Z, ncol,
-                          c->stream);
+                          c->scheme, c->stream);
   }
   if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
@@ -864,8 +864,9 @@ SweepArgs<S, CT, C> sweep_args(const pfdtd_ctx *c, const SweepPlan &p, const CT 
   a.coef = coef;
   a.ncol = coef_cols(c);
   a.air = air;
-  a.air_mask = c->air_uniform && air.inv == 1 && air.omb == 1 ? 0xFFu : 0u;
-  a.air_pm = 6u * (uint32_t)a.ncol * 0x10001u;
+  a.centred = c->scheme == 2;
+  a.air_mask = a.centred || (c->air_uniform && air.inv == 1 && air.omb == 1) ? 0xFFu : 0u;
+  a.air_pm = a.centred ? 0x800080u : 6u * (uint32_t)a.ncol * 0x10001u;
   a.lam2 = lam2;
   a.src_kind = c->d_src_kind;
   a.sig = sig;

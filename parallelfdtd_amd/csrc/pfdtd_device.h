@@ -174,20 +174,39 @@ constexpr int kTX = 256;
 // coefficient entry of (number of DIR bits D, material) holds {1/(1+beta), beta-1, 2-6 lam2}
 // with beta = table * lambda * D, evaluated on the host in the reference's order.
 template <typename C>
-__device__ __forceinline__ C centred_node(unsigned pb, unsigned mb, C pc, C zp, C zm, C yp, C ym,
-                                          C xp, C xm, C past,
-                                          const typename CoefOf<C>::T *__restrict__ coef,
-                                          unsigned cs, const typename CoefOf<C>::T &air, C lam2) {
-#pragma clang fp contract(off)
+struct CentredNode {
+  typename CoefOf<C>::T e;
+  C dx, dy, dz, in;     // DIR bits and the inside bit
+  uint32_t px, py, mz;  // SIGN bits: +x, +y, -z stand in
+};
+template <typename C>
+__device__ __forceinline__ CentredNode<C> centred_entry(unsigned pb, unsigned mb,
+                                                        const typename CoefOf<C>::T *__restrict__ coef,
+                                                        unsigned cs,
+                                                        const typename CoefOf<C>::T &air) {
   const unsigned dxb = pb & 1u, dyb = (pb >> 1) & 1u, dzb = (pb >> 2) & 1u;
-  typename CoefOf<C>::T e = air;
-  if (pb != 0x80u) e = coef[(dxb + dyb + dzb) * cs + mb];
-  const C sx = (pb & 0x10u) ? xp : xm;  // p_x[sign_x]
-  const C sy = (pb & 0x20u) ? yp : ym;  // p_y[sign_y]
-  const C sz = (pb & 0x40u) ? zm : zp;  // p_z[sign_z]: p_z[1] is z-1
-  C sb = sx * (C)dxb;
-  sb = sb + sy * (C)dyb;
-  sb = sb + sz * (C)dzb;
+  CentredNode<C> n;
+  n.e = air;
+  if (pb != 0x80u) n.e = coef[(dxb + dyb + dzb) * cs + mb];
+  n.dx = (C)dxb;
+  n.dy = (C)dyb;
+  n.dz = (C)dzb;
+  n.in = (C)(pb >> 7);
+  n.px = pb & 0x10u;
+  n.py = pb & 0x20u;
+  n.mz = pb & 0x40u;
+  return n;
+}
+template <typename C>
+__device__ __forceinline__ C centred_eval(const CentredNode<C> &n, C pc, C zp, C zm, C yp, C ym,
+                                          C xp, C xm, C past, C lam2) {
+#pragma clang fp contract(off)
+  const C sx = n.px ? xp : xm;  // p_x[sign_x]
+  const C sy = n.py ? yp : ym;  // p_y[sign_y]
+  const C sz = n.mz ? zm : zp;  // p_z[sign_z]: p_z[1] is z-1
+  C sb = sx * n.dx;
+  sb = sb + sy * n.dy;
+  sb = sb + sz * n.dz;
   // (p_x[0]+p_x[1]+p_y[0]+p_y[1]+p_z[0]+p_z[1]+S_boundary)*lambda^2, left to right
   C s = xm + xp;
   s = s + ym;
@@ -196,10 +215,18 @@ __device__ __forceinline__ C centred_node(unsigned pb, unsigned mb, C pc, C zp, 
   s = s + zm;
   s = s + sb;
   s = s * lam2;
-  C t = s - e.tk * pc;
-  t = t + e.omb * past;
-  t = t * (C)(pb >> 7);
-  return t * e.inv;
+  C t = s - n.e.tk * pc;
+  t = t + n.e.omb * past;
+  t = t * n.in;
+  return t * n.e.inv;
+}
+template <typename C>
+__device__ __forceinline__ C centred_node(unsigned pb, unsigned mb, C pc, C zp, C zm, C yp, C ym,
+                                          C xp, C xm, C past,
+                                          const typename CoefOf<C>::T *__restrict__ coef,
+                                          unsigned cs, const typename CoefOf<C>::T &air, C lam2) {
+  return centred_eval(centred_entry<C>(pb, mb, coef, cs, air), pc, zp, zm, yp, ym, xp, xm, past,
+                      lam2);
 }
 
 // centred_node for an air voxel (position byte 0x80: inside, no DIR or SIGN bit), whatever its

@@ -260,6 +260,7 @@ struct SweepArgs {
   int nbx, nby, band;
   int n_slots;
   int64_t slot_elems;
+  int centred;  // 1: the centred boundaries (scheme 2)
 };
 
 struct SweepPlan {
@@ -303,9 +304,9 @@ hipError_t launch_sweep_pool(int precision, int tiles, const void *args, const P
 hipError_t launch_pool_rotate(const PoolJobDev *jobs, PoolState *st, const PoolLaunch &pl,
                               int rounds, int levels, hipStream_t stream);
 hipError_t launch_pack_entry(const uint8_t *pos, const uint8_t *mat, uint16_t *pm, int X, int Y,
-                             int Z, int pitch, int ncol, hipStream_t stream);
+                             int Z, int pitch, int ncol, int scheme, hipStream_t stream);
 hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint64_t *out, int X, int Y,
-                           int Z, int ncol, hipStream_t stream);
+                           int Z, int ncol, int scheme, hipStream_t stream);
 hipError_t launch_sweep_f32(const SweepPlan &p, const SweepArgs<float, CoefF, float> &a, int levels,
                             hipStream_t stream);
 hipError_t launch_sweep_f16(const SweepPlan &p, const SweepArgs<h16, CoefF, float> &a, int levels,

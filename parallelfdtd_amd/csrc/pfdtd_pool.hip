@@ -774,9 +774,9 @@ int pfdtd_pool_submit(pfdtd_pool *p, const pfdtd_job *j, int64_t *job_id) {
   for (int b = 0; b < 4 && e == hipSuccess; ++b)
     if (d.F[b]) e = hipMemsetAsync(d.F[b], 0, es * (size_t)N, u);
   if (e == hipSuccess && fused)
-    e = launch_pack_entry(d.pos, d.mat, (uint16_t *)(base + L.entry), X, Y, Z, sp.pitch, d.ncol, u);
+    e = launch_pack_entry(d.pos, d.mat, (uint16_t *)(base + L.entry), X, Y, Z, sp.pitch, d.ncol, 0, u);
   if (e == hipSuccess && fused)
-    e = launch_row_bits(sp, a.pm, (uint64_t *)(base + L.row_bits), X, Y, Z, d.ncol, u);
+    e = launch_row_bits(sp, a.pm, (uint64_t *)(base + L.row_bits), X, Y, Z, d.ncol, 0, u);
   if (e == hipSuccess && fused)
     e = hipMemcpyAsync(base + L.ev_ptr, ev_ptr.data(), sizeof(int32_t) * ev_ptr.size(), hipMemcpyHostToDevice, u);
   if (e == hipSuccess && !ev_data.empty())

@@ -49,6 +49,11 @@
 // node is P - D in FP32, and a sample keeps it. 249 VGPRs. 640x480x320 hall, 400 steps: 66.7 ms with
 // the two-level sweep of independent waves -> 52.7.
 //
+// The centred boundaries take the same tiles: the entry plane holds position and material bytes, and the
+// DIR and SIGN bits pick the neighbour that stands in for a missing one (15 VALU operations per air node,
+// about 35 otherwise). 448x264x135 FP32, 300 steps in segments of 25: the sweeps 73 us per step with two
+// levels of independent waves, 45 with five here.
+//
 // Loads, stores and masks. Slices are accessed through buffer descriptors: rows and columns past
 // the grid read 0, stores that a lane or row does not own are given an offset past the slice and
 // dropped, so the body has no masked branches. The loads of the next slice are issued as soon as a
@@ -180,6 +185,8 @@ typedef const __attribute__((address_space(4))) uint64_t *ConstU64;
 // to a power of two.
 constexpr int sweep_ring(int L) { return L <= 2 ? 1 : L == 3 ? 2 : 4; }
 
+constexpr int kForward = 0, kDiff = 1, kCentred = 2;  // modes of the sweep
+
 constexpr uint32_t kDrop = 0x80000000u;  // offset bit that puts a store out of range
 
 }  // namespace
@@ -192,7 +199,7 @@ using ConstSweepArgs = const __attribute__((address_space(4))) SweepArgsOf<S> *;
 
 // One block of a sweep: tile `tile` of nbx x nby x (z-chunks of zc slices), fields fA, fB to fC, fD,
 // first step `step`.
-template <typename S, int L, int LM, int TY, int WY, int NC, int HX, bool DIFF>
+template <typename S, int L, int LM, int TY, int WY, int NC, int HX, int MODE>
 __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned tile, int slot, int zc,
                                             const S *__restrict__ gA, const S *__restrict__ gB,
                                             S *__restrict__ gC, S *__restrict__ gD, int step) {
@@ -200,6 +207,7 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
   typedef typename Fmt<S>::C C;
   typedef typename CoefOf<C>::T CE;
   typedef ConstSweepArgs<S> ConstArgs;
+  constexpr bool DIFF = MODE == kDiff, CENTRED = MODE == kCentred;
   const auto &a = *args;
   typedef Cols<C, NC> V;
   typedef Raw<S, NC> R;
@@ -262,7 +270,11 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
   // the tile with the last column of an odd width, which is stored on its own
   const bool odd_edge = NC == 2 && (X & 1) && bxi == a.nbx - 1;
   const C air_tk = a.air.tk, lam2 = a.lam2;
-  const uint32_t air_pm = a.air_pm, air_mask = a.air_mask, out_pm = kStageRows * ncol * 0x10001u;
+  CE air_e{};
+  air_e.inv = a.air.inv;
+  air_e.omb = a.air.omb;
+  air_e.tk = air_tk;
+  const uint32_t air_pm = a.air_pm, air_mask = a.air_mask, out_pm = CENTRED ? 0u : kStageRows * ncol * 0x10001u;
 
   // air, solid and unchanged rows of this wave's tile (a byte each per slice, 8 slices per word), and
   // its events by z
@@ -435,6 +447,12 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
       // every level's entries first: the gathers then overlap the arithmetic
       uint32_t pm[L + 1];
       CE e[2][NC];
+      CentredNode<C> cn[2][NC];
+      auto entry_of = [&](uint32_t v, int c) { return c == 0 ? v & 0xFFFFu : v >> 16; };
+      auto centred_of = [&](uint32_t v, int c) {
+        const uint32_t w = entry_of(v, c);
+        return centred_entry<C>(w & 0xFFu, w >> 8, s_coef, ncol, air_e);
+      };
       V t[L + 1];
       t[0] = R::up(pl[r]);
       const V past0 = R::up(pq[r]);
@@ -445,7 +463,12 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
         else if ((hist_s >> (8 * (i - 1) + r)) & 1ull)
           pm[i] = out_pm;
 #pragma unroll
-        for (int c = 0; c < NC; ++c) e[i & 1][c] = s_coef[c == 0 ? pm[i] & 0xFFFFu : pm[i] >> 16];
+        for (int c = 0; c < NC; ++c) {
+          if constexpr (CENTRED)
+            cn[i & 1][c] = centred_of(pm[i], c);
+          else
+            e[i & 1][c] = s_coef[entry_of(pm[i], c)];
+        }
       };
       if constexpr (TABLE) {
 #pragma unroll
@@ -458,7 +481,12 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
       CE one[NC];
       if constexpr (KIND == 4) {
 #pragma unroll
-        for (int c = 0; c < NC; ++c) one[c] = s_coef[c == 0 ? pmr[r] & 0xFFFFu : pmr[r] >> 16];
+        for (int c = 0; c < NC; ++c) {
+          if constexpr (CENTRED)
+            cn[0][c] = centred_of(pmr[r], c);
+          else
+            one[c] = s_coef[entry_of(pmr[r], c)];
+        }
         __builtin_amdgcn_sched_barrier(0);
       }
 #pragma unroll
@@ -489,6 +517,22 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
           for (int c = 0; c < NC; ++c) {
             t[i].v[c] = (C)0;
             e_new.v[c] = col_ok[c] && ((upd_rows >> r) & 1u) ? (C)0 - ce.v[c] : (C)0;
+          }
+        } else if constexpr (CENTRED) {
+#pragma unroll
+          for (int c = 0; c < NC; ++c) {
+            const C xn = x_next(ce, c), xp = x_prev(ce, c);
+            C v;
+            if constexpr (KIND == 0) {
+              v = centred_air<C>(ce.v[c], zn.v[c], zp.v[c], yn.v[c], yp.v[c], xn, xp, past.v[c], air_e,
+                                 lam2);
+            } else {
+              v = centred_eval<C>(cn[KIND == 4 ? 0 : i & 1][c], ce.v[c], zn.v[c], zp.v[c], yn.v[c],
+                                  yp.v[c], xn, xp, past.v[c], lam2);
+              sw_keep(v);
+              v = ((KIND == 4 || row_ok) && col_ok[c]) ? v : (C)0;
+            }
+            t[i].v[c] = v;
           }
         } else {
           C u[NC], m[NC], o[NC];
@@ -649,12 +693,12 @@ __device__ __forceinline__ unsigned xcd_tile() {
 
 // A context's sweep: the slots of a batch innermost, so that one XCD's L2 serves a tile's entries
 // to all of them.
-template <typename S, int L, int LM, int TY, int WY, int NC, int HX, bool DIFF>
+template <typename S, int L, int LM, int TY, int WY, int NC, int HX, int MODE>
 __global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_kernel(SweepArgsOf<S> a) {
   const unsigned tile = xcd_tile();
   const int slot = (int)(tile % (unsigned)a.n_slots);
   const int64_t off = (int64_t)slot * a.slot_elems;
-  sweep_block<S, L, LM, TY, WY, NC, HX, DIFF>(
+  sweep_block<S, L, LM, TY, WY, NC, HX, MODE>(
       (ConstSweepArgs<S>)__builtin_amdgcn_kernarg_segment_ptr(), tile / (unsigned)a.n_slots, slot,
       a.zc, a.A + off, a.B + off, a.Cn + off, a.Dn + off, a.step);
 }
@@ -683,7 +727,7 @@ __global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_pool_kernel(
   int o1, o2;
   pool_spare(st.cur, st.past, o1, o2);
   const bool odd = round & 1;
-  sweep_block<S, L, LM, TY, WY, NC, HX, false>(
+  sweep_block<S, L, LM, TY, WY, NC, HX, kForward>(
       (ConstSweepArgs<S>)(args + job), (unsigned)(tile - (lo ? pl.tile_end[lo - 1] : 0)), 0, zc,
       (const S *)J.F[odd ? o2 : st.cur], (const S *)J.F[odd ? o1 : st.past],
       (S *)J.F[odd ? st.past : o1], (S *)J.F[odd ? st.cur : o2], step);
@@ -704,30 +748,34 @@ __global__ __launch_bounds__(kPoolMaxJobs) void pool_rotate_kernel(
                        : PoolState{st.step + n * levels, st.cur, st.past};
 }
 
-// Coefficient entry per voxel: row min(K, 6) of ncol material columns, or kStageRows * ncol outside.
+// Coefficient entry per voxel: row min(K, 6) of ncol material columns, or kStageRows * ncol outside;
+// the centred scheme's entries are the position byte | material << 8.
 __global__ __launch_bounds__(256) void pack_entry_kernel(const uint8_t *__restrict__ pos,
                                                          const uint8_t *__restrict__ mat,
                                                          uint16_t *__restrict__ pm, int X,
-                                                         int pitch, int64_t rows, unsigned ncol) {
+                                                         int pitch, int64_t rows, unsigned ncol,
+                                                         int centred) {
   const int64_t n = rows * pitch;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < n; i += (int64_t)gridDim.x * 256) {
     const int64_t row = i / pitch;
     const int x = (int)(i - row * pitch);
-    unsigned v = kStageRows * ncol;
+    unsigned v = centred ? 0u : kStageRows * ncol;
     if (x < X) {
       const unsigned p = pos[row * X + x], m = mat[row * X + x];
-      if (p & 0x80u) v = min(p & 0x7Fu, 6u) * ncol + min(m, ncol - 1);
+      if (centred)
+        v = p | min(m, ncol - 1) << 8;
+      else if (p & 0x80u) v = min(p & 0x7Fu, 6u) * ncol + min(m, ncol - 1);
     }
     pm[i] = (uint16_t)v;
   }
 }
 
 hipError_t launch_pack_entry(const uint8_t *pos, const uint8_t *mat, uint16_t *pm, int X, int Y,
-                             int Z, int pitch, int ncol, hipStream_t stream) {
+                             int Z, int pitch, int ncol, int scheme, hipStream_t stream) {
   const int64_t rows = (int64_t)Y * Z, n = rows * pitch;
   const unsigned grid = (unsigned)std::min<int64_t>((n + 255) / 256, 65536);
   hipLaunchKernelGGL(pack_entry_kernel, dim3(grid), dim3(256), 0, stream, pos, mat, pm, X, pitch,
-                     rows, (unsigned)ncol);
+                     rows, (unsigned)ncol, scheme == 2);
   return hipGetLastError();
 }
 
@@ -740,7 +788,7 @@ __global__ __launch_bounds__(64) void row_bits_kernel(const uint16_t *__restrict
                                                       uint64_t *__restrict__ out, int X, int Y,
                                                       int Z, int nbx, int ox, int hx, int w,
                                                       int oy, int lm, int wy, int ty, int words,
-                                                      unsigned ncol) {
+                                                      unsigned ncol, int centred) {
   const int lane = threadIdx.x;
   const int bx = blockIdx.x, tw = blockIdx.y;
   const int xs = bx * ox - hx, ys = (tw / wy) * oy - lm + (tw % wy) * ty;
@@ -760,8 +808,9 @@ __global__ __launch_bounds__(64) void row_bits_kernel(const uint16_t *__restrict
           for (int c = lane; c < w; c += 64) {
             if (xs + c < 0 || xs + c >= X) continue;
             const unsigned v = slice[(size_t)y * pitch + xs + c];
-            not_air = not_air || v < 6u * ncol || v >= kStageRows * ncol;
-            not_solid = not_solid || v < kStageRows * ncol;
+            const bool out = centred ? !(v & 0x80u) : v >= kStageRows * ncol;
+            not_air = not_air || (centred ? (v & 0xFFu) != 0x80u : v < 6u * ncol || out);
+            not_solid = not_solid || !out;
             if (!changed) changed = v != slice[(size_t)y * pitch + xs + c - (size_t)pitch * Y];
           }
         }
@@ -886,26 +935,26 @@ size_t sweep_lds(int ncol) {
          2 * T::NC * (size_t)T::WY * sweep_ring(L) * T::TY * 64;
 }
 
-template <typename S, int L, bool DIFF>
+template <typename S, int L, int MODE>
 hipError_t launch_levels(const SweepPlan &p, const SweepArgsOf<S> &a, hipStream_t stream) {
   typedef SweepTile<S> T;
   const size_t lds = sweep_lds<S, L>(a.ncol);
-  hipLaunchKernelGGL((srl_sweep_kernel<S, L, T::LM, T::TY, T::WY, T::NC, T::HX, DIFF>),
+  hipLaunchKernelGGL((srl_sweep_kernel<S, L, T::LM, T::TY, T::WY, T::NC, T::HX, MODE>),
                      dim3((unsigned)p.blocks), dim3(64 * T::WY), lds, stream, a);
   return hipGetLastError();
 }
 
-template <typename S, bool DIFF = false, typename A>
+template <typename S, int MODE = kForward, typename A>
 hipError_t launch_any(const SweepPlan &p, const A &a, int levels, hipStream_t stream) {
   switch (levels) {
-  case 1: return launch_levels<S, 1, DIFF>(p, a, stream);
-  case 2: return launch_levels<S, 2, DIFF>(p, a, stream);
-  case 3: return launch_levels<S, 3, DIFF>(p, a, stream);
+  case 1: return launch_levels<S, 1, MODE>(p, a, stream);
+  case 2: return launch_levels<S, 2, MODE>(p, a, stream);
+  case 3: return launch_levels<S, 3, MODE>(p, a, stream);
   case 4:
-    if constexpr (SweepTile<S>::LM >= 4) return launch_levels<S, 4, DIFF>(p, a, stream);
+    if constexpr (SweepTile<S>::LM >= 4) return launch_levels<S, 4, MODE>(p, a, stream);
     break;
   case 5:
-    if constexpr (SweepTile<S>::LM >= 5) return launch_levels<S, 5, DIFF>(p, a, stream);
+    if constexpr (SweepTile<S>::LM >= 5) return launch_levels<S, 5, MODE>(p, a, stream);
     break;
   }
   return hipErrorInvalidValue;
@@ -994,31 +1043,36 @@ void sweep_events(const SweepPlan &p, int slots, const std::vector<SweepPoint> &
 }
 
 hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint64_t *out, int X, int Y,
-                           int Z, int ncol, hipStream_t stream) {
+                           int Z, int ncol, int scheme, hipStream_t stream) {
   const dim3 grid((unsigned)p.nbx, (unsigned)(p.nby * p.wy), (unsigned)std::min(p.words, 65535));
   hipLaunchKernelGGL(row_bits_kernel, grid, dim3(64), 0, stream, pm, p.pitch, out, X, Y, Z, p.nbx,
-                     p.ox, p.hx, p.w, p.oy, p.lm, p.wy, p.ty, p.words, (unsigned)ncol);
+                     p.ox, p.hx, p.w, p.oy, p.lm, p.wy, p.ty, p.words, (unsigned)ncol,
+                     scheme == 2);
   return hipGetLastError();
 }
 
 hipError_t launch_sweep_f32(const SweepPlan &p, const SweepArgsOf<float> &a, int levels,
                             hipStream_t stream) {
+  if (a.centred) return launch_any<float, kCentred>(p, a, levels, stream);
   return launch_any<float>(p, a, levels, stream);
 }
 hipError_t launch_sweep_f16(const SweepPlan &p, const SweepArgsOf<h16> &a, int levels,
                             hipStream_t stream) {
+  if (a.centred) return launch_any<h16, kCentred>(p, a, levels, stream);
   return launch_any<h16>(p, a, levels, stream);
 }
 hipError_t launch_sweep_diff(const SweepPlan &p, const SweepArgsOf<h16> &a, int levels,
                              hipStream_t stream) {
-  return launch_any<h16, true>(p, a, levels, stream);
+  return launch_any<h16, kDiff>(p, a, levels, stream);
 }
 hipError_t launch_sweep_bf16(const SweepPlan &p, const SweepArgsOf<b16> &a, int levels,
                              hipStream_t stream) {
+  if (a.centred) return launch_any<b16, kCentred>(p, a, levels, stream);
   return launch_any<b16>(p, a, levels, stream);
 }
 hipError_t launch_sweep_f64(const SweepPlan &p, const SweepArgsOf<double> &a, int levels,
                             hipStream_t stream) {
+  if (a.centred) return launch_any<double, kCentred>(p, a, levels, stream);
   return launch_any<double>(p, a, levels, stream);
 }
 }  // namespace pfdtd

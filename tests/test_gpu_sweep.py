@@ -148,3 +148,28 @@ def test_difference_form_at_tile_borders(gpu, dx, dy, z, zchunk, n_steps):
     sc.src_xyz[1] = [6, oy + 3, z // 2]
     sc.rec_xyz[0] = sc.src_xyz[0]
     run_diff(sc, 9, zchunk=zchunk, poll=7)
+
+
+@pytest.mark.parametrize("prec", list(OWNED))
+@pytest.mark.parametrize("dx,dy,z,zchunk,n_steps", [(-1, 1, 9, 0, 23), (0, 0, 12, 3, 9), (1, -1, 21, 5, 7),
+                                                    (9, 6, 30, 7, 14)])
+def test_centred_scheme_agrees_with_single_steps(gpu, prec, dx, dy, z, zchunk, n_steps):
+    """The centred boundaries through the sweep and through single steps, whose parity with the oracle
+    is tested elsewhere: responses and both fields bit for bit."""
+    from test_gpu_centred import centred_room
+    ox, oy = OWNED[prec]
+    sc = centred_room(1010 + dx, (ox + dx, 2 * oy + dy, z), n_steps=n_steps)
+    sc.src_xyz[0] = [ox // 2, oy, 1]
+    raw = {N.F32: np.float32, N.F64: np.float64, N.F16: np.float16, N.BF16: np.uint16}[prec]
+    out = []
+    for levels in (0, 1):
+        with Solver() as s:
+            s.set_update_type(N.SRL)
+            s.set_time_levels(levels, zchunk)
+            s.load_scene(sc)
+            s.prepare_fields(prec, 9 if prec in (N.F16, N.BF16) else 0)
+            s.run(sc.n_steps, prec)
+            out.append((s.responses(), *s.fields_raw(raw)))
+    assert np.abs(out[1][0]).max() > 0
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
