@@ -14,6 +14,7 @@ import os
 import shlex
 import subprocess
 import sys
+from concurrent.futures import ThreadPoolExecutor
 from pathlib import Path
 
 PKG = Path(__file__).resolve().parent
@@ -33,8 +34,9 @@ HIP_FLAGS = [
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
 ]
 
-LIB_SOURCES = ["pfdtd_kernels.hip", "pfdtd_fused.hip", "pfdtd_sweep.hip", "pfdtd_capi.hip", "pfdtd_pool.hip",
-               "pfdtd_voxel.hip", "pfdtd_probe.hip"]
+LIB_SOURCES = ["pfdtd_sweep_f16.hip", "pfdtd_sweep_f32.hip", "pfdtd_sweep_bf16.hip", "pfdtd_sweep_f64.hip",
+               "pfdtd_fused.hip", "pfdtd_kernels.hip", "pfdtd_sweep.hip", "pfdtd_capi.hip",
+               "pfdtd_pool.hip", "pfdtd_voxel.hip", "pfdtd_probe.hip"]
 
 
 def _run(cmd: list[str], cwd: Path | None = None) -> None:
@@ -45,13 +47,16 @@ def _run(cmd: list[str], cwd: Path | None = None) -> None:
 def build_lib(out: Path | None = None) -> Path:
     """Compile libpfdtd.so (kernels + C ABI) with hipcc."""
     out = out or PKG / "libpfdtd.so"
-    objs = []
     objdir = PKG / "_build"
     objdir.mkdir(exist_ok=True)
-    for src in LIB_SOURCES:
+
+    def compile_one(src: str) -> str:
         obj = objdir / (Path(src).stem + ".o")
         _run([HIPCC, *HIP_FLAGS, "-I", str(ROOT / "include"), "-c", str(CSRC / src), "-o", str(obj)])
-        objs.append(str(obj))
+        return str(obj)
+
+    with ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as ex:
+        objs = list(ex.map(compile_one, LIB_SOURCES))
     tmp = out.with_suffix(".so.tmp")
     _run([HIPCC, "--offload-arch=gfx950", "-shared", "-fPIC", "-o", str(tmp), *objs])
     os.replace(tmp, out)

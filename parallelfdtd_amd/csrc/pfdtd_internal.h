@@ -74,7 +74,8 @@ struct UpdateArgs {
   int scheme;  // 0 forward (Bilbao) boundaries, 2 centred (Kowalczyk) boundaries
 };
 
-// ---- serving pool (pfdtd_pool.hip; the sweep over its jobs lives in pfdtd_sweep.hip)
+// ---- serving pool (pfdtd_pool.hip; the sweep over its jobs lives in
+// pfdtd_sweep_kernel.h)
 constexpr int kPoolMaxJobs = 64;
 constexpr int kPoolLevels = 5;  // steps per round: the levels of the sweep's FP32 and 16-bit tiles
 
@@ -225,7 +226,7 @@ hipError_t launch_update3_f16(const FusedGeom &g, const Fused2Args<h16, CoefF, f
 hipError_t launch_update3_bf16(const FusedGeom &g, const Fused2Args<b16, CoefF, float> &a,
                                hipStream_t stream);
 
-// Several-level sweep (pfdtd_sweep.hip): reads P^n (A) and P^{n-1} (B), writes P^{n+L-1} (Cn) and
+// Several-level sweep (pfdtd_sweep_kernel.h): reads P^n (A) and P^{n-1} (B), writes P^{n+L-1} (Cn) and
 // P^{n+L} (Dn) with the sources of steps n+1 .. n+L injected and the receivers of steps
 // n .. n+L-1 gathered on the way.
 template <typename S, typename CT, typename C>
@@ -264,6 +265,8 @@ struct SweepArgs {
 };
 
 struct SweepPlan {
+  int tile;              // 0: the large tile, 1: the small one
+  double us;             // modelled time of a launch
   int nc, ty, wy, lm;    // columns per lane, rows per wave, waves per block, most levels
   int w, hx, ox, oy;     // window columns, halo columns, owned columns and rows of a block
   int nbx, nby, zc, band, words, pitch;
@@ -273,7 +276,7 @@ struct SweepPlan {
 inline size_t sweep_row_words(const SweepPlan &p) {
   return 3 * (size_t)p.nbx * p.nby * p.wy * p.words;
 }
-SweepPlan plan_sweep(int precision, int X, int Y, int Z, int zc, int slots);
+SweepPlan plan_sweep(int precision, int X, int Y, int Z, int zc, int slots, bool pool = false);
 // Fills the tile geometry of a sweep's arguments.
 template <typename A>
 void sweep_geometry(const SweepPlan &p, A &a) {
@@ -284,7 +287,13 @@ void sweep_geometry(const SweepPlan &p, A &a) {
   a.nby = p.nby;
   a.band = p.band;
 }
-int sweep_zchunk(int n, const int64_t *bxy, const int *zi, int levels);
+// Cost model of a sweep's launches in us: t0 + slices * (a + b * blocks on a CU), up to cap of them.
+struct SweepRate {
+  double t0, a, b;
+  int cap;
+};
+int sweep_zchunk(int n, const int64_t *bxy, const int *zi, int levels,
+                 const SweepRate &rate = SweepRate{0, 1, 0, 1});
 // A source or receiver as the sweep's event lists take it.
 struct SweepPoint {
   int32_t x, y, z, slot, id;  // id: source index, or receiver index | 1 << 31
@@ -301,6 +310,12 @@ void sweep_events(const SweepPlan &p, int slots, const std::vector<SweepPoint> &
 hipError_t launch_sweep_pool(int precision, int tiles, const void *args, const PoolJobDev *jobs,
                              const PoolState *st, const PoolLaunch &pl, int zc, int round,
                              hipStream_t stream);
+hipError_t launch_pool_f32(int tiles, const void *args, const PoolJobDev *jobs, const PoolState *st,
+                           const PoolLaunch &pl, int zc, int round, hipStream_t stream);
+hipError_t launch_pool_f16(int tiles, const void *args, const PoolJobDev *jobs, const PoolState *st,
+                           const PoolLaunch &pl, int zc, int round, hipStream_t stream);
+hipError_t launch_pool_bf16(int tiles, const void *args, const PoolJobDev *jobs, const PoolState *st,
+                            const PoolLaunch &pl, int zc, int round, hipStream_t stream);
 hipError_t launch_pool_rotate(const PoolJobDev *jobs, PoolState *st, const PoolLaunch &pl,
                               int rounds, int levels, hipStream_t stream);
 hipError_t launch_pack_entry(const uint8_t *pos, const uint8_t *mat, uint16_t *pm, int X, int Y,

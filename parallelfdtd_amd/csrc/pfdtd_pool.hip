@@ -199,7 +199,7 @@ struct JobLayout {
 JobLayout layout_job(int X, int Y, int Z, size_t es, int n_src, int n_samples, int n_rec,
                      int n_steps, bool fused, int precision) {
   const int64_t N = (int64_t)X * Y * Z;
-  const SweepPlan sp = plan_sweep(precision, X, Y, Z, 1, 1);
+  const SweepPlan sp = plan_sweep(precision, X, Y, Z, 1, 1, true);
   const size_t wave_tiles = (size_t)sp.nbx * sp.nby * sp.wy;
   JobLayout L{};
   size_t o = 0;
@@ -693,7 +693,7 @@ int pfdtd_pool_submit(pfdtd_pool *p, const pfdtd_job *j, int64_t *job_id) {
   d.gx = (X + kPoolTW - 1) / kPoolTW;
   d.gy = (Y + rows_per_tile - 1) / rows_per_tile;
   const int gz = (Z - 2 + p->zc - 1) / p->zc;
-  const SweepPlan sp = plan_sweep(j->precision, X, Y, Z, 0, 1);
+  const SweepPlan sp = plan_sweep(j->precision, X, Y, Z, 0, 1, true);
   const int64_t tiles = fused ? (int64_t)sp.nbx * sp.nby * (Z - 2) : (int64_t)d.gx * d.gy * gz;
   if (tiles > (int64_t)1 << 30) {
     arena_free(p, off, L.total);

@@ -1,0 +1,16 @@
+// pfdtd_sweep_bf16.hip -- the several-level sweep's kernels for BF16 fields.
+#include "pfdtd_sweep_kernel.h"
+
+namespace pfdtd {
+
+hipError_t launch_sweep_bf16(const SweepPlan &p, const SweepArgsOf<b16> &a, int levels,
+                           hipStream_t stream) {
+  if (a.centred) return launch_any<b16, kCentred>(p, a, levels, stream);
+  return launch_any<b16>(p, a, levels, stream);
+}
+hipError_t launch_pool_bf16(int tiles, const void *args, const PoolJobDev *jobs, const PoolState *st,
+                           const PoolLaunch &pl, int zc, int round, hipStream_t stream) {
+  return launch_pool<b16>(tiles, args, jobs, st, pl, zc, round, stream);
+}
+
+}  // namespace pfdtd

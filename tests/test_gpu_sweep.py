@@ -160,6 +160,7 @@ def test_centred_scheme_agrees_with_single_steps(gpu, prec, dx, dy, z, zchunk, n
     ox, oy = OWNED[prec]
     sc = centred_room(1010 + dx, (ox + dx, 2 * oy + dy, z), n_steps=n_steps)
     sc.src_xyz[0] = [ox // 2, oy, 1]
+    sc.rec_xyz[0] = [ox // 2 + 1, oy, 1]
     raw = {N.F32: np.float32, N.F64: np.float64, N.F16: np.float16, N.BF16: np.uint16}[prec]
     out = []
     for levels in (0, 1):
@@ -170,6 +171,46 @@ def test_centred_scheme_agrees_with_single_steps(gpu, prec, dx, dy, z, zchunk, n
             s.prepare_fields(prec, 9 if prec in (N.F16, N.BF16) else 0)
             s.run(sc.n_steps, prec)
             out.append((s.responses(), *s.fields_raw(raw)))
-    assert np.abs(out[1][0]).max() > 0
+    assert out[1][1].any()
+    for a, b in zip(*out):
+        assert np.array_equal(a, b)
+
+
+SMALL = {N.F32: (56, 18), N.F64: (56, 26), N.F16: (56, 18), N.BF16: (56, 18)}  # of the small tile
+
+
+@pytest.mark.parametrize("prec", list(SMALL))
+@pytest.mark.parametrize("dx,dy,z,zchunk", [(-1, 1, 9, 0), (0, 0, 12, 3), (1, -1, 21, 5), (8, 5, 8, 1)])
+@pytest.mark.parametrize("n_steps", [23, 4])
+def test_small_tile_borders(gpu, prec, dx, dy, z, zchunk, n_steps):
+    """Rooms the small tile takes: two tiles and a little more or less along x and y."""
+    ox, oy = SMALL[prec]
+    sc = scene(990 + dx, (2 * ox + dx, 2 * oy + dy, z), n_steps, n_boxes=12)
+    sc.src_xyz[0] = [ox - 3, oy, z // 2]
+    sc.rec_xyz[0] = [ox, oy - 1, z // 2]
+    sc.rec_xyz[1] = sc.src_xyz[0]
+    assert_same(*run_both(sc, prec, levels=0, zchunk=zchunk))
+
+
+@pytest.mark.parametrize("prec", list(OWNED))
+@pytest.mark.parametrize("dims", [(331, 150, 60), (224, 113, 97)])
+def test_large_tile_agrees_with_single_steps(gpu, prec, dims):
+    """Enough sources at once for the large tile, several tiles along x and y, each slot its own
+    source, against single steps of the same batch."""
+    B = 8
+    sc = scene(1000, dims, 19, n_boxes=20, n_src=B, n_rec=4 * B)
+    out = []
+    for levels in (0, 1):
+        with Solver() as s:
+            s.set_time_levels(levels, 0)
+            s.load_scene(sc)
+            s.set_batch_layout(N.BATCH_GROUPED)
+            s.set_batch(B)
+            s.set_source_slots(np.arange(B))
+            s.set_receiver_slots(np.arange(4 * B) % B)
+            s.prepare_fields(prec, 9 if prec in (N.F16, N.BF16) else 0)
+            s.run(sc.n_steps, prec)
+            raw = {N.F32: np.float32, N.F64: np.float64, N.F16: np.float16, N.BF16: np.uint16}[prec]
+            out.append((s.responses(), *s.fields_raw(raw)))
     for a, b in zip(*out):
         assert np.array_equal(a, b)
