@@ -177,8 +177,18 @@ template <typename C>
 struct CentredNode {
   typename CoefOf<C>::T e;
   C dx, dy, dz, in;     // DIR bits and the inside bit
-  uint32_t px, py, mz;  // SIGN bits: +x, +y, -z stand in
+  uint32_t px, py, mz;  // all ones where +x, +y, -z stand in (SIGN bits), else 0
 };
+// a where m is all ones, b where it is 0: one v_bfi_b32 per 32 bits instead of a select on a lane mask.
+__device__ __forceinline__ float pick_bits(uint32_t m, float a, float b) {
+  const uint32_t x = __float_as_uint(a), y = __float_as_uint(b);
+  return __uint_as_float((x & m) | (y & ~m));
+}
+__device__ __forceinline__ double pick_bits(uint32_t m, double a, double b) {
+  const uint32_t xh = (uint32_t)__double2hiint(a), xl = (uint32_t)__double2loint(a);
+  const uint32_t yh = (uint32_t)__double2hiint(b), yl = (uint32_t)__double2loint(b);
+  return __hiloint2double((int)((xh & m) | (yh & ~m)), (int)((xl & m) | (yl & ~m)));
+}
 template <typename C>
 __device__ __forceinline__ CentredNode<C> centred_entry(unsigned pb, unsigned mb,
                                                         const typename CoefOf<C>::T *__restrict__ coef,
@@ -192,18 +202,19 @@ __device__ __forceinline__ CentredNode<C> centred_entry(unsigned pb, unsigned mb
   n.dy = (C)dyb;
   n.dz = (C)dzb;
   n.in = (C)(pb >> 7);
-  n.px = pb & 0x10u;
-  n.py = pb & 0x20u;
-  n.mz = pb & 0x40u;
+  n.px = 0u - ((pb >> 4) & 1u);
+  n.py = 0u - ((pb >> 5) & 1u);
+  n.mz = 0u - ((pb >> 6) & 1u);
+  asm("" : "+v"(n.px), "+v"(n.py), "+v"(n.mz));
   return n;
 }
 template <typename C>
 __device__ __forceinline__ C centred_eval(const CentredNode<C> &n, C pc, C zp, C zm, C yp, C ym,
                                           C xp, C xm, C past, C lam2) {
 #pragma clang fp contract(off)
-  const C sx = n.px ? xp : xm;  // p_x[sign_x]
-  const C sy = n.py ? yp : ym;  // p_y[sign_y]
-  const C sz = n.mz ? zm : zp;  // p_z[sign_z]: p_z[1] is z-1
+  const C sx = pick_bits(n.px, xp, xm);  // p_x[sign_x]
+  const C sy = pick_bits(n.py, yp, ym);  // p_y[sign_y]
+  const C sz = pick_bits(n.mz, zm, zp);  // p_z[sign_z]: p_z[1] is z-1
   C sb = sx * n.dx;
   sb = sb + sy * n.dy;
   sb = sb + sz * n.dz;
