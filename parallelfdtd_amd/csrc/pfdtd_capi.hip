@@ -84,7 +84,7 @@ struct pfdtd_ctx {
   uint16_t *d_entry = nullptr;
   size_t entry_cap = 0;
   bool entry_ok = false;
-  uint64_t *d_row_bits = nullptr;
+  uint32_t *d_row_bits = nullptr;
   size_t air_cap = 0;
   int32_t *d_ev_ptr = nullptr, *d_events = nullptr;
   size_t ev_ptr_cap = 0, ev_cap = 0;

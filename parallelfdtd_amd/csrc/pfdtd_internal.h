@@ -233,8 +233,7 @@ template <typename S, typename CT, typename C>
 struct SweepArgs {
   const uint16_t *pm;  // coefficient entry per voxel, rows of `pitch` elements
   int pitch;
-  const uint64_t *row_bits;  // per wave tile, three bytes per slice: rows of plain air, solid, unchanged
-  int air_words;             // words per wave tile
+  const uint32_t *row_bits;  // a word per wave tile and slice: rows of plain air, solid, unchanged
   const int32_t *ev_ptr;     // per (slot, wave tile): first event, then one past the last
   const int32_t *events;     // {z, x, y, source index or receiver index | 1 << 31}, by z
   const S *A;
@@ -274,14 +273,13 @@ struct SweepPlan {
 };
 // Words of a plan's row bits.
 inline size_t sweep_row_words(const SweepPlan &p) {
-  return 3 * (size_t)p.nbx * p.nby * p.wy * p.words;
+  return (size_t)p.nbx * p.nby * p.wy * p.words;
 }
 SweepPlan plan_sweep(int precision, int X, int Y, int Z, int zc, int slots, bool pool = false);
 // Fills the tile geometry of a sweep's arguments.
 template <typename A>
 void sweep_geometry(const SweepPlan &p, A &a) {
   a.pitch = p.pitch;
-  a.air_words = p.words;
   a.zc = p.zc;
   a.nbx = p.nbx;
   a.nby = p.nby;
@@ -320,7 +318,7 @@ hipError_t launch_pool_rotate(const PoolJobDev *jobs, PoolState *st, const PoolL
                               int rounds, int levels, hipStream_t stream);
 hipError_t launch_pack_entry(const uint8_t *pos, const uint8_t *mat, uint16_t *pm, int X, int Y,
                              int Z, int pitch, int ncol, int scheme, hipStream_t stream);
-hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint64_t *out, int X, int Y,
+hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint32_t *out, int X, int Y,
                            int Z, int ncol, int scheme, hipStream_t stream);
 hipError_t launch_sweep_f32(const SweepPlan &p, const SweepArgs<float, CoefF, float> &a, int levels,
                             hipStream_t stream);

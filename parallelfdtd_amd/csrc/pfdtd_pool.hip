@@ -212,7 +212,7 @@ JobLayout layout_job(int X, int Y, int Z, size_t es, int n_src, int n_samples, i
   L.pos = take((size_t)N);
   L.mat = take((size_t)N);
   L.entry = fused ? take(sizeof(uint16_t) * (size_t)sp.pitch * Y * Z) : 0;
-  L.row_bits = fused ? take(sizeof(uint64_t) * sweep_row_words(sp)) : 0;
+  L.row_bits = fused ? take(sizeof(uint32_t) * sweep_row_words(sp)) : 0;
   L.labels = take((size_t)N);
   L.coef = take(sizeof(CoefF) * kCoefEntries);
   L.src_idx = take(sizeof(int64_t) * (size_t)n_src);
@@ -735,7 +735,7 @@ int pfdtd_pool_submit(pfdtd_pool *p, const pfdtd_job *j, int64_t *job_id) {
     sweep_events(sp, 1, rec, src, ev_ptr, ev_data);
     sweep_geometry(sp, a);
     a.pm = (const uint16_t *)(base + L.entry);
-    a.row_bits = (const uint64_t *)(base + L.row_bits);
+    a.row_bits = (const uint32_t *)(base + L.row_bits);
     a.ev_ptr = (const int32_t *)(base + L.ev_ptr);
     a.events = (const int32_t *)(base + L.events);
     a.A = (const float *)d.F[0];
@@ -776,7 +776,7 @@ int pfdtd_pool_submit(pfdtd_pool *p, const pfdtd_job *j, int64_t *job_id) {
   if (e == hipSuccess && fused)
     e = launch_pack_entry(d.pos, d.mat, (uint16_t *)(base + L.entry), X, Y, Z, sp.pitch, d.ncol, 0, u);
   if (e == hipSuccess && fused)
-    e = launch_row_bits(sp, a.pm, (uint64_t *)(base + L.row_bits), X, Y, Z, d.ncol, 0, u);
+    e = launch_row_bits(sp, a.pm, (uint32_t *)(base + L.row_bits), X, Y, Z, d.ncol, 0, u);
   if (e == hipSuccess && fused)
     e = hipMemcpyAsync(base + L.ev_ptr, ev_ptr.data(), sizeof(int32_t) * ev_ptr.size(), hipMemcpyHostToDevice, u);
   if (e == hipSuccess && !ev_data.empty())

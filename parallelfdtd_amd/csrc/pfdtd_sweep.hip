@@ -51,55 +51,44 @@ hipError_t launch_pack_entry(const uint8_t *pos, const uint8_t *mat, uint16_t *p
   return hipGetLastError();
 }
 
-// Three bytes per (wave tile, slice), 8 slices to three words: bit r of the first is set when the
-// tile's row r is plain air over its whole window (and inside the grid), of the second when no
-// voxel of it is updated (outside voxels, or past the grid), of the third when its entries are
-// those of the slice below (never on slice 1 or outside 1..Z-2). Bits past the tile's rows are set
-// in all. A wave per tile and word.
+// A word per (wave tile, slice): bit r of the first byte is set when the tile's row r is plain air over
+// its whole window (and inside the grid), of the second when no voxel of it is updated (outside voxels,
+// past the grid, slices 0 and Z-1), of the third when its entries are those of the slice below (never on
+// slices 0, 1 and Z-1). Bits past the tile's rows are set in all. A wave per tile and slice.
 __global__ __launch_bounds__(64) void row_bits_kernel(const uint16_t *__restrict__ pm, int pitch,
-                                                      uint64_t *__restrict__ out, int X, int Y,
+                                                      uint32_t *__restrict__ out, int X, int Y,
                                                       int Z, int nbx, int ox, int hx, int w,
-                                                      int oy, int lm, int wy, int ty, int words,
+                                                      int oy, int lm, int wy, int ty,
                                                       unsigned ncol, int centred) {
   const int lane = threadIdx.x;
   const int bx = blockIdx.x, tw = blockIdx.y;
   const int xs = bx * ox - hx, ys = (tw / wy) * oy - lm + (tw % wy) * ty;
   const bool x_in = xs >= 0 && xs + w <= X;
-  for (int word = blockIdx.z; word < words; word += gridDim.z) {
-    uint64_t air = 0, solid = 0, same = 0;
-    for (int b = 0; b < 8; ++b) {
-      const int z = 8 * word + b;
-      uint32_t ma = (0xFFu << ty) & 0xFFu, ms = ma, mu = ma;
-      const uint16_t *slice = pm + (size_t)min(z, Z - 1) * (size_t)pitch * (size_t)Y;
-      for (int r = 0; r < ty; ++r) {
-        const int y = ys + r;
-        bool not_air = !x_in, not_solid = false, changed = z < 2 || z > Z - 2;
-        if (y < 0 || y >= Y || z >= Z) {
-          not_air = true;
-        } else {
-          for (int c = lane; c < w; c += 64) {
-            if (xs + c < 0 || xs + c >= X) continue;
-            const unsigned v = slice[(size_t)y * pitch + xs + c];
-            const bool out = centred ? !(v & 0x80u) : v >= kStageRows * ncol;
-            not_air = not_air || (centred ? (v & 0xFFu) != 0x80u : v < 6u * ncol || out);
-            not_solid = not_solid || !out;
-            if (!changed) changed = v != slice[(size_t)y * pitch + xs + c - (size_t)pitch * Y];
-          }
+  const uint32_t past = (0xFFu << ty) & 0xFFu;
+  for (int z = blockIdx.z; z < Z; z += gridDim.z) {
+    const bool shell = z == 0 || z == Z - 1;
+    uint32_t ma = past, ms = shell ? 0xFFu : past, mu = past;
+    const uint16_t *slice = pm + (size_t)z * (size_t)pitch * (size_t)Y;
+    for (int r = 0; r < ty && !shell; ++r) {
+      const int y = ys + r;
+      bool not_air = !x_in, not_solid = false, changed = z < 2;
+      if (y < 0 || y >= Y) {
+        not_air = true;
+      } else {
+        for (int c = lane; c < w; c += 64) {
+          if (xs + c < 0 || xs + c >= X) continue;
+          const unsigned v = slice[(size_t)y * pitch + xs + c];
+          const bool out_v = centred ? !(v & 0x80u) : v >= kStageRows * ncol;
+          not_air = not_air || (centred ? (v & 0xFFu) != 0x80u : v < 6u * ncol || out_v);
+          not_solid = not_solid || !out_v;
+          if (!changed) changed = v != slice[(size_t)y * pitch + xs + c - (size_t)pitch * Y];
         }
-        if (__ballot(not_air) == 0) ma |= 1u << r;
-        if (__ballot(not_solid) == 0) ms |= 1u << r;
-        if (__ballot(changed) == 0) mu |= 1u << r;
       }
-      air |= (uint64_t)ma << (8 * b);
-      solid |= (uint64_t)ms << (8 * b);
-      same |= (uint64_t)mu << (8 * b);
+      if (__ballot(not_air) == 0) ma |= 1u << r;
+      if (__ballot(not_solid) == 0) ms |= 1u << r;
+      if (__ballot(changed) == 0) mu |= 1u << r;
     }
-    if (lane == 0) {
-      const size_t o = 3 * (((size_t)tw * nbx + bx) * words + word);
-      out[o] = air;
-      out[o + 1] = solid;
-      out[o + 2] = same;
-    }
+    if (lane == 0) out[((size_t)tw * nbx + bx) * Z + z] = ma | ms << 8 | mu << 16;
   }
 }
 
@@ -178,7 +167,7 @@ SweepPlan plan_of(int X, int Y, int Z, int zc, int slots) {
   p.oy = T::TY * T::WY - 2 * T::LM;
   p.nbx = (X + p.ox - 1) / p.ox;
   p.nby = (Y + p.oy - 1) / p.oy;
-  p.words = (Z + 7) / 8;
+  p.words = Z;
   p.pitch = X + (X & 1);
   p.band = 2;
   const int zi = Z - 2;
@@ -275,11 +264,11 @@ void sweep_events(const SweepPlan &p, int slots, const std::vector<SweepPoint> &
   for (size_t i = 1; i < ptr.size(); ++i) ptr[i] += ptr[i - 1];
 }
 
-hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint64_t *out, int X, int Y,
+hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint32_t *out, int X, int Y,
                            int Z, int ncol, int scheme, hipStream_t stream) {
-  const dim3 grid((unsigned)p.nbx, (unsigned)(p.nby * p.wy), (unsigned)std::min(p.words, 65535));
+  const dim3 grid((unsigned)p.nbx, (unsigned)(p.nby * p.wy), (unsigned)std::min(Z, 65535));
   hipLaunchKernelGGL(row_bits_kernel, grid, dim3(64), 0, stream, pm, p.pitch, out, X, Y, Z, p.nbx,
-                     p.ox, p.hx, p.w, p.oy, p.lm, p.wy, p.ty, p.words, (unsigned)ncol,
+                     p.ox, p.hx, p.w, p.oy, p.lm, p.wy, p.ty, (unsigned)ncol,
                      scheme == 2);
   return hipGetLastError();
 }

@@ -211,7 +211,7 @@ __device__ __forceinline__ C x_prev(const Cols<C, NC> &q, int c) {
 }
 
 typedef const __attribute__((address_space(4))) int32_t *ConstI32;
-typedef const __attribute__((address_space(4))) uint64_t *ConstU64;
+typedef const __attribute__((address_space(4))) uint32_t *ConstU32;
 
 // Slices of packed rows a wave keeps in LDS: the L - 1 slices above the first level's, rounded up
 // to a power of two.
@@ -308,10 +308,10 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
   air_e.tk = air_tk;
   const uint32_t air_pm = a.air_pm, air_mask = a.air_mask, out_pm = CENTRED ? 0u : kStageRows * ncol * 0x10001u;
 
-  // air, solid and unchanged rows of this wave's tile (a byte each per slice, 8 slices per word), and
-  // its events by z
+  // air, solid and unchanged rows of this wave's tile (a byte each, a word per slice), and its events
+  // by z
   const int wt = (byi * WY + wave) * a.nbx + bxi;
-  const ConstU64 gair = (ConstU64)(a.row_bits + 3 * (size_t)wt * a.air_words);
+  const ConstU32 grows = (ConstU32)(a.row_bits + (size_t)wt * Z);
   int ev = 0, ev_end = 0;
   {
     const int et = slot * (a.nby * WY * a.nbx) + wt;
@@ -365,28 +365,14 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
   };
   const int wu = wave > 0 ? wave - 1 : 0, wd = wave < WY - 1 ? wave + 1 : WY - 1;
 
-  // row bytes of the current and the next 8 slices: plain air, solid (or not updated), and the entries
-  // of the slice below; every row of a slice outside 1..Z-2 is solid
-  struct Rows {
-    uint64_t air, solid, same;
-  };
-  Rows bw, bn;
-  auto load_rows = [&](int w) -> Rows {
-    if (w >= a.air_words) return Rows{0, 0, 0};
-    return Rows{gair[3 * w], gair[3 * w + 1], gair[3 * w + 2]};
-  };
+  // row bytes of a slice: plain air, solid (or not updated), and the entries of the slice below; every
+  // row of a slice outside 1..Z-2 is solid (so are the words of slices 0 and Z-1)
   struct RowBits {
     uint32_t air, solid, same;
   };
-  auto row_bits = [&](int k, bool step) -> RowBits {
-    if (k < 1 || k > Z - 2) return RowBits{0u, 0xFFu, 0u};
-    if (step && (k & 7) == 0) {
-      bw = bn;
-      bn = load_rows((k >> 3) + 1);
-    }
-    const int sh = 8 * (k & 7);
-    return RowBits{(uint32_t)(bw.air >> sh) & air_mask, (uint32_t)(bw.solid >> sh) & 0xFFu,
-                   (uint32_t)(bw.same >> sh) & 0xFFu};
+  auto row_word = [&](int k) -> uint32_t { return grows[k < 0 ? 0 : k > Z - 1 ? Z - 1 : k]; };
+  auto row_bits = [&](uint32_t w) -> RowBits {
+    return RowBits{w & air_mask, (w >> 8) & 0xFFu, (w >> 16) & 0xFFu};
   };
   // the rows set in each of the n newest bytes of a history
   auto all_of = [](uint64_t h, int n) -> uint32_t {
@@ -425,12 +411,8 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
   // levels are not used)
   uint64_t hist = ~0ull, hist_s = ~0ull;
   uint32_t hist_u = ~0u;
-  {
-    const int kf = kb < 1 ? 1 : kb;
-    bw = load_rows(kf >> 3);
-    bn = load_rows((kf >> 3) + 1);
-  }
-  RowBits rows_k = row_bits(kb, false);
+  RowBits rows_k = row_bits(row_word(kb));
+  uint32_t row_next = row_word(kb + 1);  // the words are loaded a slice ahead
   if ((rows_k.air | rows_k.solid) != 0xFFu) load_pm(kb);
   // vmcnt(0): nothing may be in flight when the loop is entered. The compiler's wait for a row's
   // loads counts the accesses issued after them on whichever way into the loop has fewest, so the
@@ -453,7 +435,8 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
     // the rows that are air, solid, of unchanged entries at every level, or have events: a byte each
     const uint32_t kinds = all_of(hist, L) | (all_of(hist_s, L) << 8) |
                            (all_of(hist_u, L - 1) << 16) | (ev_rows << 24);
-    const RowBits rows_next = row_bits(k + 1, true);
+    const RowBits rows_next = row_bits(row_next);
+    row_next = row_word(k + 2);
     const auto ra = a_rsrc(k + 2), rb = b_rsrc(k + 1);
     const int sC = k - (L - 2), sD = k - (L - 1);
     const bool inD = sD >= z0 && sD < z1, inC = DIFF ? inD : L >= 2 && sC >= z0 && sC < z1;
