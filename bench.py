@@ -50,10 +50,11 @@ from parallelfdtd_amd.solver import Solver  # noqa: E402
 METRIC = "Gvoxel-updates/s + % HBM roofline (FP32 vs FP16-store); p50/p99 IR latency"
 PEAK_GBS = 8000.0
 BYTES_PER_NODE = {N.F32: 14, N.F16: 8, N.BF16: 8, N.F64: 26}
-# HBM bytes per launch of the dominant FP32 kernel (three time levels per launch), from counters
-TRAFFIC_SUMMARY = ROOT / "profiles" / "srl_update3_c3_f32_hbm_traffic.md"
-# steps of the kernel-timing runs: whole launches of the two- and the three-level sweeps
-KERNEL_STEPS = 96
+# time levels per launch of the dominant FP32 kernel, and its HBM bytes per launch from counters
+LEVELS = 5
+TRAFFIC_SUMMARY = ROOT / "profiles" / "srl_sweep_c3_f32_hbm_traffic.md"
+# steps of the kernel-timing runs: whole launches of the several-level sweep (5 levels, FP64 4)
+KERNEL_STEPS = 100
 
 
 def log(msg: str) -> None:
@@ -168,7 +169,7 @@ def cpu_baseline(scene, steps: int = 300, nz: int = 66) -> dict:
 def shard_share(scene, steps: int, warmup: int, n_gpus: int = 8) -> dict:
     """One GPU's share of the room under a z-slab decomposition over n_gpus GPUs: Z/n_gpus
     updated slices plus the two halo slices, here closed by the ceiling material (the update
-    work is the same), FP32, the default sweep (three levels per launch)."""
+    work is the same), FP32, the default sweep (five levels per launch)."""
     Z = scene.labels.shape[0]
     nz = (Z - 2) // n_gpus + 2
     lab = np.ascontiguousarray(scene.labels[:nz].copy())
@@ -328,7 +329,7 @@ def main() -> int:
                 log(f"FP16 difference form: {fp16['difference_form']}")
 
     traffic = committed_traffic() if args.scale == 1 else None
-    launch_s = 3 * kms * 1e-3
+    launch_s = LEVELS * kms * 1e-3
     measured = traffic / launch_s / 1e9 if traffic else None
     out = {
         "metric": METRIC,
@@ -349,13 +350,13 @@ def main() -> int:
         "roofline": {"bound": "hbm", "achieved": round(achieved, 1), "peak": PEAK_GBS,
                      "unit": "GB/s", "frac": round(achieved / PEAK_GBS, 4),
                      "traffic": traffic,
-                     "achieved_kind": "algorithmic bytes (14 B per node-update, 3 updates per "
+                     "achieved_kind": f"algorithmic bytes (14 B per node-update, {LEVELS} updates per "
                                       "launch) / launch time; above 1 of peak because a launch "
-                                      "moves each field once for three steps",
+                                      f"moves each field once for {LEVELS} steps",
                      "achieved_measured": round(measured, 1) if measured else None,
                      "frac_measured": round(measured / PEAK_GBS, 4) if measured else None,
-                     "kernel": "srl_update3_kernel<float> (three time levels per launch)",
-                     "launch_ms": round(3 * kms, 4), "ms_per_step": round(kms, 4),
+                     "kernel": f"srl_sweep_kernel<float> ({LEVELS} time levels per launch)",
+                     "launch_ms": round(LEVELS * kms, 4), "ms_per_step": round(kms, 4),
                      "bytes_per_node_update": BYTES_PER_NODE[N.F32]},
         "fp16_storage": fp16,
     }

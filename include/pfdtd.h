@@ -322,9 +322,10 @@ int pfdtd_get_kernel_timing(pfdtd_ctx *ctx, double *update_ms_total, int64_t *up
 /* ---- serving pool ------------------------------------------------------------------- */
 /* A pool holds many independent impulse-response jobs (rooms of different sizes, each with
  * its own materials, sources, receivers, step count and FP32 / FP16 / BF16 storage) resident in
- * one HBM arena, and advances all of them together: one step of every resident job of one
- * storage type is one launch of a multi-job update kernel plus one launch of a multi-job
- * gather/inject kernel; `bundle_steps` steps are captured into a hipGraph that is replayed
+ * one HBM arena, and advances all of them together: five steps of every resident job of one
+ * storage type are one launch of a multi-job sweep, gathers and injections inside (jobs with a
+ * source on the first or last z slice: an update and a gather/inject launch per step);
+ * `bundle_steps` steps are captured into a hipGraph that is replayed
  * until a job joins or leaves. Jobs are admitted while their buffers fit in the arena's free
  * space and a slot is free (at most 64 resident), so a job submitted while others run starts
  * at the next bundle and overlaps them on the device. Every job's arithmetic is that of a
@@ -359,8 +360,8 @@ typedef struct pfdtd_job {
 /* arena_bytes <= 0: 7/8 of the device's free memory. */
 int pfdtd_pool_create(int device, int64_t arena_bytes, pfdtd_pool **out);
 int pfdtd_pool_destroy(pfdtd_pool *pool);
-/* Steps per bundle (default 32; rounded up to an even count, as jobs advance in rounds of two
- * steps), hipGraph replay (1, default) or direct launches (0), single-step update tiling
+/* Steps per bundle (default 32; rounded up to whole rounds of five steps, as jobs advance in the
+ * several-level sweep), hipGraph replay (1, default) or direct launches (0), single-step update tiling
  * (rows 1/2/4, z-chunk; only while empty) and the resident-job limit (1..64). */
 int pfdtd_pool_set_options(pfdtd_pool *pool, int bundle_steps, int use_graph, int rows,
                            int zchunk, int max_jobs);

@@ -17,11 +17,10 @@
 // three-level sweep computes 1.8 nodes and loads 4.5 rows per node-update it keeps, this one 1.5 (L =
 // 5) and 2.2.
 //
-// What bounds it (2048x1536x768 FP32, L = 5): 2.25-2.40 ms per step against 3.73-3.83 for the
-// three-level sweep of independent waves. Its arithmetic alone (no loads, no stores, all air) takes
-// 1.20 ms, the table rows 0.4 more, the loads alone 1.41, the stores alone 1.66: it is bound by the
-// traffic, 19.4 GB written and 1.5 passes of the two fields read per launch. FP64 (L = 4):
-// 1024x768x384 0.70 ms against 1.03. Tiles measured (ms per step, 2048x1536x768 FP32, same box): L = 4
+// What bounds it (2048x1536x768 FP32, L = 5): 2.06-2.33 ms per step against 3.73-3.83 for the
+// three-level sweep of independent waves, 19.4 GB written and 30.4 read per launch at 4.8 TB/s of a
+// copy's 5.5: the traffic. FP64 (L = 4): 1024x768x384 0.64 ms against 1.03. Rooms in the Infinity Cache
+// are bound by issue (below). Tiles measured before the last steps (ms per step, 2048x1536x768 FP32, same box): L = 4
 // 8 rows 2.95, 6 rows 2.96; L = 5 6 rows 2.52, 7 rows (spills) 2.55; L = 6 does not fit LDS. Windows: stores of
 // whole 64-byte lines matter (112 owned columns 2.99, 120 columns 3.26 with L = 4), so HX is 8
 // although five columns would do; 16 (96 owned columns) 3.07.
