@@ -54,41 +54,56 @@ hipError_t launch_pack_entry(const uint8_t *pos, const uint8_t *mat, uint16_t *p
 // A word per (wave tile, slice): bit r of the first byte is set when the tile's row r is plain air over
 // its whole window (and inside the grid), of the second when no voxel of it is updated (outside voxels,
 // past the grid, slices 0 and Z-1), of the third when its entries are those of the slice below (never on
-// slices 0, 1 and Z-1). Bits past the tile's rows are set in all. A wave per tile and slice.
+// slices 0, 1 and Z-1). Bits past the tile's rows are set in all. A wave per tile and run of slices, each
+// lane's columns of the slice below kept in registers, so every entry is loaded once per tile. On
+// 2048x1536x768 3.90 ms, a wave per slice with its slice below loaded again 9.26.
+constexpr int kRowRun = 32;
+template <int NC>
 __global__ __launch_bounds__(64) void row_bits_kernel(const uint16_t *__restrict__ pm, int pitch,
                                                       uint32_t *__restrict__ out, int X, int Y,
-                                                      int Z, int nbx, int ox, int hx, int w,
-                                                      int oy, int lm, int wy, int ty,
-                                                      unsigned ncol, int centred) {
+                                                      int Z, int nbx, int ox, int hx, int oy,
+                                                      int lm, int wy, int ty, unsigned ncol,
+                                                      int centred) {
   const int lane = threadIdx.x;
   const int bx = blockIdx.x, tw = blockIdx.y;
-  const int xs = bx * ox - hx, ys = (tw / wy) * oy - lm + (tw % wy) * ty;
-  const bool x_in = xs >= 0 && xs + w <= X;
+  const int xs = bx * ox - hx, ys = (tw / wy) * oy - lm + (tw % wy) * ty, x = xs + NC * lane;
+  const bool x_in = xs >= 0 && xs + 64 * NC <= X;
+  const bool in0 = x >= 0 && x < X, in1 = NC == 2 && x + 1 >= 0 && x + 1 < X;
   const uint32_t past = (0xFFu << ty) & 0xFFu;
-  for (int z = blockIdx.z; z < Z; z += gridDim.z) {
-    const bool shell = z == 0 || z == Z - 1;
-    uint32_t ma = past, ms = shell ? 0xFFu : past, mu = past;
-    const uint16_t *slice = pm + (size_t)z * (size_t)pitch * (size_t)Y;
-    for (int r = 0; r < ty && !shell; ++r) {
-      const int y = ys + r;
-      bool not_air = !x_in, not_solid = false, changed = z < 2;
-      if (y < 0 || y >= Y) {
-        not_air = true;
-      } else {
-        for (int c = lane; c < w; c += 64) {
-          if (xs + c < 0 || xs + c >= X) continue;
-          const unsigned v = slice[(size_t)y * pitch + xs + c];
-          const bool out_v = centred ? !(v & 0x80u) : v >= kStageRows * ncol;
-          not_air = not_air || (centred ? (v & 0xFFu) != 0x80u : v < 6u * ncol || out_v);
-          not_solid = not_solid || !out_v;
-          if (!changed) changed = v != slice[(size_t)y * pitch + xs + c - (size_t)pitch * Y];
+  const uint32_t use = (in0 ? 0xFFFFu : 0u) | (in1 ? 0xFFFF0000u : 0u);
+  auto entry = [&](int z, int y) -> uint32_t {
+    if (!use || y < 0 || y >= Y) return 0;
+    const uint16_t *q = pm + ((size_t)z * Y + y) * pitch + x;  // x and pitch even with two columns
+    return (NC == 2 ? *(const uint32_t *)q : (uint32_t)*q) & use;
+  };
+  auto is_out = [&](unsigned v) { return centred ? !(v & 0x80u) : v >= kStageRows * ncol; };
+  auto is_air = [&](unsigned v) {
+    return centred ? (v & 0xFFu) == 0x80u : v >= 6u * ncol && v < kStageRows * ncol;
+  };
+  for (int z0 = blockIdx.z * kRowRun; z0 < Z; z0 += gridDim.z * kRowRun) {
+    uint32_t below[8];
+#pragma unroll
+    for (int r = 0; r < 8; ++r) below[r] = r < ty && z0 > 0 ? entry(z0 - 1, ys + r) : 0;
+    for (int z = z0; z < min(z0 + kRowRun, Z); ++z) {
+      const bool shell = z == 0 || z == Z - 1;
+      uint32_t ma = past, ms = shell ? 0xFFu : past, mu = past;
+#pragma unroll
+      for (int r = 0; r < 8; ++r) {
+        if (r >= ty) break;
+        const int y = ys + r;
+        const uint32_t v = entry(z, y);
+        const bool not_air = !x_in || y < 0 || y >= Y || !is_air(v & 0xFFFFu) || (NC == 2 && !is_air(v >> 16));
+        const bool not_solid = y >= 0 && y < Y && ((in0 && !is_out(v & 0xFFFFu)) || (in1 && !is_out(v >> 16)));
+        const bool changed = z < 2 || v != below[r];
+        below[r] = v;
+        if (!shell) {
+          if (__ballot(not_air) == 0) ma |= 1u << r;
+          if (__ballot(not_solid) == 0) ms |= 1u << r;
+          if (__ballot(changed) == 0) mu |= 1u << r;
         }
       }
-      if (__ballot(not_air) == 0) ma |= 1u << r;
-      if (__ballot(not_solid) == 0) ms |= 1u << r;
-      if (__ballot(changed) == 0) mu |= 1u << r;
+      if (lane == 0) out[((size_t)tw * nbx + bx) * Z + z] = ma | ms << 8 | mu << 16;
     }
-    if (lane == 0) out[((size_t)tw * nbx + bx) * Z + z] = ma | ms << 8 | mu << 16;
   }
 }
 
@@ -266,10 +281,13 @@ void sweep_events(const SweepPlan &p, int slots, const std::vector<SweepPoint> &
 
 hipError_t launch_row_bits(const SweepPlan &p, const uint16_t *pm, uint32_t *out, int X, int Y,
                            int Z, int ncol, int scheme, hipStream_t stream) {
-  const dim3 grid((unsigned)p.nbx, (unsigned)(p.nby * p.wy), (unsigned)std::min(Z, 65535));
-  hipLaunchKernelGGL(row_bits_kernel, grid, dim3(64), 0, stream, pm, p.pitch, out, X, Y, Z, p.nbx,
-                     p.ox, p.hx, p.w, p.oy, p.lm, p.wy, p.ty, (unsigned)ncol,
-                     scheme == 2);
+  const dim3 grid((unsigned)p.nbx, (unsigned)(p.nby * p.wy), (unsigned)((Z + kRowRun - 1) / kRowRun));
+  if (p.nc == 2)
+    hipLaunchKernelGGL(row_bits_kernel<2>, grid, dim3(64), 0, stream, pm, p.pitch, out, X, Y, Z, p.nbx,
+                       p.ox, p.hx, p.oy, p.lm, p.wy, p.ty, (unsigned)ncol, scheme == 2);
+  else
+    hipLaunchKernelGGL(row_bits_kernel<1>, grid, dim3(64), 0, stream, pm, p.pitch, out, X, Y, Z, p.nbx,
+                       p.ox, p.hx, p.oy, p.lm, p.wy, p.ty, (unsigned)ncol, scheme == 2);
   return hipGetLastError();
 }
 
