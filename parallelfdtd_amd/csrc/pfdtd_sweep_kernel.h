@@ -20,7 +20,7 @@
 // What bounds it (2048x1536x768 FP32, L = 5): 2.06-2.33 ms per step against 3.73-3.83 for the
 // three-level sweep of independent waves, 19.4 GB written and 30.4 read per launch at 4.8 TB/s of a
 // copy's 5.5: the traffic. FP64 (L = 4): 1024x768x384 0.64 ms against 1.03. Rooms in the Infinity Cache
-// are bound by issue (below). Tiles measured before the last steps (ms per step, 2048x1536x768 FP32, same box): L = 4
+// are bound by issue (below). Tiles measured before the last steps (ms per step, 2048x1536x768 FP32, same card): L = 4
 // 8 rows 2.95, 6 rows 2.96; L = 5 6 rows 2.52, 7 rows (spills) 2.55; L = 6 does not fit LDS. Windows: stores of
 // whole 64-byte lines matter (112 owned columns 2.99, 120 columns 3.26 with L = 4), so HX is 8
 // although five columns would do; 16 (96 owned columns) 3.07.
@@ -51,7 +51,7 @@
 // The centred boundaries take the same tiles: the entry plane holds position and material bytes, and the
 // DIR and SIGN bits pick the neighbour that stands in for a missing one (15 VALU operations per air node,
 // about 35 otherwise). 448x264x135 FP32, 300 steps in segments of 25: the sweeps 73 us per step with two
-// levels of independent waves, 45 with five here.
+// levels of independent waves, 49 with five here.
 //
 // Loads, stores and masks. Slices are accessed through buffer descriptors: rows and columns past
 // the grid read 0, stores that a lane or row does not own are given an offset past the slice and
