@@ -405,6 +405,7 @@ int enqueue_bundle_kernels(pfdtd_pool *p) {
 }
 
 int rebuild_membership(pfdtd_pool *p) {
+  // of the sweep's jobs, in the order of their launch
   int64_t bxy[3][kPoolMaxJobs];
   int zi[3][kPoolMaxJobs];
   p->members.clear();
@@ -425,9 +426,10 @@ int rebuild_membership(pfdtd_pool *p) {
     if (f == 0) {
       p->tiles[q][0] += j.tiles;
       L.tile_end[L.n] = p->tiles[q][0];
+    } else {
+      bxy[q][L.n] = j.bxy;
+      zi[q][L.n] = j.zi;
     }
-    bxy[q][L.n] = j.bxy;
-    zi[q][L.n] = j.zi;
     ++L.n;
     p->members.push_back(j.id);
   }
