@@ -180,12 +180,12 @@ SweepPlan plan_of(int X, int Y, int Z, int zc, int slots) {
   p.hx = T::HX;
   p.ox = p.w - 2 * p.hx;
   p.oy = T::TY * T::WY - 2 * T::LM;
-  p.nbx = (X + p.ox - 1) / p.ox;
-  p.nby = (Y + p.oy - 1) / p.oy;
+  p.nbx = (int)(((int64_t)X + p.ox - 1) / p.ox);
+  p.nby = (int)(((int64_t)Y + p.oy - 1) / p.oy);
   p.words = Z;
-  p.pitch = X + (X & 1);
+  p.pitch = (int)((int64_t)X + (X & 1));
   p.band = 2;
-  const int zi = Z - 2;
+  const int zi = std::max(Z - 2, 1);  // a size query may ask for a room without an inner slice
   const int64_t bxy = (int64_t)p.nbx * p.nby * slots;
   const SweepRate rate{T::T0, T::A, T::B, T::CAP};
   if (zc < 1) zc = sweep_zchunk(1, &bxy, &zi, T::LM, rate);
