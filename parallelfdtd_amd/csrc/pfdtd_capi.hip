@@ -468,13 +468,18 @@ int check_runnable(pfdtd_ctx *c) {
   return PFDTD_OK;
 }
 
-int ensure_fields(pfdtd_ctx *c, int precision, int scale_exp) {
-  const size_t es = elem_size(precision);
-  if (!es) return fail(PFDTD_E_ARG, "unknown precision %d", precision);
+int check_fields(int precision, int scale_exp) {
+  if (!elem_size(precision)) return fail(PFDTD_E_ARG, "unknown precision %d", precision);
   if ((precision == PFDTD_F32 || precision == PFDTD_F64) && scale_exp != 0)
     return fail(PFDTD_E_ARG, "scale_exp applies to F16/BF16 storage only");
   if (scale_exp < -60 || scale_exp > 60) return fail(PFDTD_E_ARG, "scale_exp out of range");
-  const size_t bytes = es * ((size_t)c->N << c->lgB);
+  return PFDTD_OK;
+}
+
+// Buffers for a precision and scale that check_fields accepts; fails with PFDTD_E_NOMEM only, and
+// then no fields are held.
+int ensure_fields(pfdtd_ctx *c, int precision, int scale_exp) {
+  const size_t bytes = elem_size(precision) * ((size_t)c->N << c->lgB);
   const bool want4 = (c->lgB == 0 || slot_major(c)) && levels_for(c, precision) >= 2;
   if (c->d_P && c->field_bytes == bytes && (!want4 || c->d_P2)) {
     c->precision = precision;
@@ -795,12 +800,15 @@ bool sweep_eligible(const pfdtd_ctx *c) {
 // 4.27 with the single-step kernel of the interleaved layout, which reads and writes every field
 // at every step.
 int ensure_run_fields(pfdtd_ctx *c, int precision, int scale_exp, bool may_planar) {
+  // arguments first: a refused call leaves the fields and their arrangement as they are
+  int rc = check_fields(precision, scale_exp);
+  if (rc) return rc;
   const size_t bytes = elem_size(precision) * ((size_t)c->N << c->lgB);
   const bool want = may_planar && c->lgB > 0 && !c->grouped && sweep_takes(c, precision) &&
                     (c->planar_nomem == 0 || bytes < c->planar_nomem);
   const bool was = c->planar;
   c->planar = want;
-  int rc = ensure_fields(c, precision, scale_exp);
+  rc = ensure_fields(c, precision, scale_exp);
   if (rc == PFDTD_E_NOMEM && want) {
     c->planar_nomem = bytes;
     c->planar = false;
@@ -1433,13 +1441,13 @@ int pfdtd_run(pfdtd_ctx *c, int precision, int n_steps, pfdtd_interrupt_cb inter
   if (rc) return rc;
   const int scale = (precision == PFDTD_F16 || precision == PFDTD_BF16 ||
                      precision == PFDTD_F16_DIFF) ? c->scale_req : 0;
-  rc = ensure_run_fields(c, precision, scale, true);
-  if (rc) return rc;
   const bool diff = precision == PFDTD_F16_DIFF;
-  if (diff && (!fused_eligible(c) || c->scheme != 0 || c->X % 2 != 0 || c->lgB > 0 ||
+  if (diff && (c->levels == 1 || boundary_source(c) || c->scheme != 0 || c->X % 2 != 0 || c->lgB > 0 ||
                c->X * c->Y * 2 >= ((int64_t)1 << 31)))
     return fail(PFDTD_E_STATE, "the difference form runs through the several-level sweep only: forward "
                 "update, X even, X*Y below 2^30, no batch, no source on the slices z = 0 or Z-1");
+  rc = ensure_run_fields(c, precision, scale, true);
+  if (rc) return rc;
   rc = zero_fields(c);
   if (rc) return rc;
   rc = ensure_responses(c, n_steps);
