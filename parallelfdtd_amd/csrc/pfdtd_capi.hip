@@ -88,7 +88,7 @@ struct pfdtd_ctx {
   size_t air_cap = 0;
   int32_t *d_ev_ptr = nullptr, *d_events = nullptr;
   size_t ev_ptr_cap = 0, ev_cap = 0;
-  int sweep_key[4] = {0, 0, 0, 0};  // tile shape the air bits and events were built for
+  int sweep_key[4] = {0, 0, 0, 0};  // tile shape the row bits were built for (zeros: none)
   bool events_ok = false;
   int64_t dom_cap = 0;  // voxels the position/material buffers hold
   bool has_domain = false;
@@ -762,7 +762,7 @@ hipError_t grow(T *&p, size_t &cap, size_t need) {
 }
 
 // Sources and receivers of the sweep's wave tiles.
-int build_sweep_events(pfdtd_ctx *c, const SweepPlan &p) {
+hipError_t build_sweep_events(pfdtd_ctx *c, const SweepPlan &p) {
   std::vector<SweepPoint> rec, src;
   for (int r = 0; r < c->n_rec; ++r) {
     const int32_t *q = &c->rec_xyz[3 * r];
@@ -775,13 +775,14 @@ int build_sweep_events(pfdtd_ctx *c, const SweepPlan &p) {
   }
   std::vector<int32_t> ptr, data;
   sweep_events(p, batch_slots(c), rec, src, ptr, data);
-  HIP_TRY(grow(c->d_ev_ptr, c->ev_ptr_cap, ptr.size()));
-  HIP_TRY(grow(c->d_events, c->ev_cap, std::max<size_t>(data.size(), 4)));
-  HIP_TRY(hipStreamSynchronize(c->stream));
-  HIP_TRY(hipMemcpy(c->d_ev_ptr, ptr.data(), sizeof(int32_t) * ptr.size(), hipMemcpyHostToDevice));
-  if (!data.empty())
-    HIP_TRY(hipMemcpy(c->d_events, data.data(), sizeof(int32_t) * data.size(), hipMemcpyHostToDevice));
-  return PFDTD_OK;
+  hipError_t e = grow(c->d_ev_ptr, c->ev_ptr_cap, ptr.size());
+  if (e == hipSuccess) e = grow(c->d_events, c->ev_cap, std::max<size_t>(data.size(), 4));
+  if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+  if (e == hipSuccess)
+    e = hipMemcpy(c->d_ev_ptr, ptr.data(), sizeof(int32_t) * ptr.size(), hipMemcpyHostToDevice);
+  if (e == hipSuccess && !data.empty())
+    e = hipMemcpy(c->d_events, data.data(), sizeof(int32_t) * data.size(), hipMemcpyHostToDevice);
+  return e;
 }
 
 // Whether the sweep can take runs of this precision: slices below 2^31 bytes, the
@@ -821,38 +822,39 @@ int ensure_run_fields(pfdtd_ctx *c, int precision, int scale_exp, bool may_plana
   return rc;
 }
 
-// Entry plane, air bits and events for the sweep; *ok is cleared when there is no room for them.
+// Entry plane, row bits and events for the sweep; *ok is cleared when there is no room for them. Each is
+// marked as current only once it is built: one that fails leaves nothing of another tile behind.
 int ensure_sweep(pfdtd_ctx *c, const SweepPlan &p, bool *ok) {
   const int ncol = coef_cols(c);
   const int key[4] = {p.w, p.hx, p.oy, p.ty};
-  const bool same = std::equal(key, key + 4, c->sweep_key);
   hipError_t e = hipSuccess;
   if (!c->entry_ok) {
+    std::fill(c->sweep_key, c->sweep_key + 4, 0);
     e = grow(c->d_entry, c->entry_cap, (size_t)p.pitch * c->Y * c->Z);
     if (e == hipSuccess)
       e = launch_pack_entry(c->d_pos, c->d_mat, c->d_entry, (int)c->X, (int)c->Y, (int)c->Z,
                             p.pitch, ncol, c->scheme, c->stream);
+    c->entry_ok = e == hipSuccess;
   }
-  if (e == hipSuccess && (!c->entry_ok || !same)) {
+  if (e == hipSuccess && !std::equal(key, key + 4, c->sweep_key)) {
+    std::fill(c->sweep_key, c->sweep_key + 4, 0);
+    c->events_ok = false;
     e = grow(c->d_row_bits, c->air_cap, sweep_row_words(p));
     if (e == hipSuccess)
       e = launch_row_bits(p, c->d_entry, c->d_row_bits, (int)c->X, (int)c->Y, (int)c->Z, ncol,
                           c->scheme, c->stream);
+    if (e == hipSuccess) std::copy(key, key + 4, c->sweep_key);
+  }
+  if (e == hipSuccess && !c->events_ok) {
+    e = build_sweep_events(c, p);
+    c->events_ok = e == hipSuccess;
   }
   if (e == hipErrorOutOfMemory) {
     (void)hipGetLastError();
-    c->entry_ok = false;
     *ok = false;
     return PFDTD_OK;
   }
   if (e != hipSuccess) return fail(PFDTD_E_HIP, "sweep planes: %s", hipGetErrorString(e));
-  c->entry_ok = true;
-  if (!c->events_ok || !same) {
-    const int rc = build_sweep_events(c, p);
-    if (rc) return rc;
-    c->events_ok = true;
-  }
-  std::copy(key, key + 4, c->sweep_key);
   return PFDTD_OK;
 }
 

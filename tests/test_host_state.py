@@ -1,0 +1,61 @@
+"""The context's host code on the stand-in HIP runtime: what it holds and launches when an allocation
+fails, and what it gives back."""
+import numpy as np
+import pytest
+
+import hostrt
+from parallelfdtd_amd import native as N
+from parallelfdtd_amd import rooms
+from parallelfdtd_amd.solver import Solver
+
+
+@pytest.fixture(scope="module")
+def rt(tmp_path_factory):
+    r = hostrt.Runtime(hostrt.build(tmp_path_factory.mktemp("hostrt")))
+    kept, N._lib = N._lib, r.lib
+    yield r
+    N._lib = kept
+
+
+@pytest.fixture(autouse=True)
+def no_limits(rt):
+    yield
+    rt.fail_malloc(-1)
+    rt.budget(1 << 40)
+    rt.log()
+
+
+def scene(dims, n_src=2, n_rec=5, n_steps=12, seed=5):
+    return rooms.scene_random_small(seed, dims=dims, n_mat=3, n_boxes=2, n_src=n_src, n_rec=n_rec,
+                                    n_steps=n_steps)
+
+
+def sweeps(rt):
+    return [l for l in rt.log() if l.startswith(("sweep", "row_bits"))]
+
+
+FIELDS = 4  # allocations of a run whose failure refuses it: the four fields
+
+
+@pytest.mark.parametrize("first,then", [(N.F64, N.F32), (N.F32, N.F64)])
+@pytest.mark.parametrize("fail", range(9))
+def test_an_allocation_fails_at_a_change_of_tile(rt, first, then, fail):
+    """FP32 and FP64 take other tiles: planes and events are rebuilt at the change. Whichever allocation
+    fails there, the run falls back (or is refused for its fields), and every later sweep reads planes
+    and events of its own tile."""
+    with Solver() as s:
+        s.load_scene(scene((131, 50, 17), n_rec=40))
+        s.run(12, first)
+        assert all(l.endswith("bad=none") for l in sweeps(rt))
+        s.set_receivers(np.tile([[9, 9, 9]], (400, 1)))  # more events than there is room for so far
+        rt.fail_malloc(fail)
+        try:
+            s.run(12, then)
+            assert fail >= FIELDS
+        except N.PfdtdError as e:
+            assert e.code == N.E_NOMEM and fail < FIELDS + 1  # the responses after the fields
+        rt.fail_malloc(-1)
+        for prec in (first, then, first):
+            s.run(12, prec)
+            lines = sweeps(rt)
+            assert lines and all(l.endswith("bad=none") for l in lines), lines
