@@ -59,3 +59,33 @@ def test_an_allocation_fails_at_a_change_of_tile(rt, first, then, fail):
             s.run(12, prec)
             lines = sweeps(rt)
             assert lines and all(l.endswith("bad=none") for l in lines), lines
+
+
+def batch(s, dims, B, prec, layout=N.BATCH_INTERLEAVED):
+    s.load_scene(scene(dims, n_src=B, n_rec=B))
+    s.set_batch_layout(layout)
+    s.set_batch(B)
+    s.set_source_slots(np.arange(B))
+    s.set_receiver_slots(np.arange(B))
+    s.prepare_fields(prec, 9 if prec in (N.F16, N.BF16) else 0)
+
+
+@pytest.mark.parametrize("prec", [N.F32, N.F64, N.F16, N.BF16])
+def test_steps_of_a_prepared_batch_take_the_interleaved_update(rt, prec):
+    """One launch of the interleaved update per step, also without begin_steps, before and after a run
+    that held the fields slot by slot."""
+    with Solver() as s:
+        batch(s, (60, 40, 20), 8, prec)
+        rt.log()
+        s.step(0)
+        prepared = rt.log()
+        s.begin_steps(12, prec)
+        rt.log()
+        s.step(0)
+        assert rt.log()[:2] == prepared[:2] and len([l for l in prepared if "update" in l]) == 1, prepared
+        s.run(12, prec)
+        assert any(l.startswith("sweep") and "slots=8" in l for l in rt.log())
+        s.prepare_fields(prec, 9 if prec in (N.F16, N.BF16) else 0)
+        rt.log()
+        s.step(0)
+        assert rt.log()[:2] == prepared[:2]
