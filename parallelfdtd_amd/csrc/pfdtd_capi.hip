@@ -796,7 +796,8 @@ bool sweep_eligible(const pfdtd_ctx *c) {
 }
 
 // Fields for `use` (zeroed by the caller). Runs hold an interleaved batch that the sweep can take slot
-// by slot, if its four buffers fit: 32 sources on 512x384x256 take 1.9 ms per step that way against
+// by slot, if its four buffers take no more than half of the free memory (the interleaved layout does
+// with two, and what it leaves is other contexts'): 32 sources on 512x384x256 take 1.9 ms per step that way against
 // 4.27 with the single-step kernel of the interleaved layout, which reads and writes every field
 // at every step. Prepared fields have the buffers of a run, but stay interleaved for steps that follow
 // (32 sources on 256x200x120: 539 us per step against 799 slot by slot).
@@ -806,8 +807,13 @@ int ensure_fields_for(pfdtd_ctx *c, int precision, int scale_exp, Use use) {
   int rc = check_fields(precision, scale_exp);
   if (rc) return rc;
   const size_t bytes = elem_size(precision) * ((size_t)c->N << c->lgB);
-  const bool spare = use != Use::kSteps && c->lgB > 0 && !c->grouped && sweep_takes(c, precision) &&
-                     (c->planar_nomem == 0 || bytes < c->planar_nomem);
+  bool spare = use != Use::kSteps && c->lgB > 0 && !c->grouped && sweep_takes(c, precision) &&
+               (c->planar_nomem == 0 || bytes < c->planar_nomem);
+  if (spare && !(c->d_P2 && c->field_bytes == bytes)) {
+    size_t free_now = 0, total = 0;
+    HIP_TRY(hipMemGetInfo(&free_now, &total));
+    spare = 8 * bytes <= free_now + (c->d_P2 ? 4 : c->d_P ? 2 : 0) * c->field_bytes;
+  }
   const bool want4 = (c->lgB == 0 || c->grouped) && levels_for(c, precision) >= 2;
   const bool was = c->planar;
   c->planar = spare && use == Use::kRun;

@@ -89,3 +89,34 @@ def test_steps_of_a_prepared_batch_take_the_interleaved_update(rt, prec):
         rt.log()
         s.step(0)
         assert rt.log()[:2] == prepared[:2]
+
+
+@pytest.mark.parametrize("prec,es", [(N.F32, 4), (N.F16, 2)])
+def test_contexts_with_batches_fit_where_two_fields_each_fit(rt, prec, es):
+    """An interleaved batch does with two fields: a card with room for two such contexts, and a little
+    more, holds both, whatever the first one runs. With plenty of room a run takes four."""
+    dims, B = (120, 80, 40), 8
+    field = es * 120 * 80 * 40 * B
+    rt.budget(rt.used() + 4 * field + (5 << 20))
+    with Solver() as s, Solver() as t:
+        for x in (s, t):
+            batch(x, dims, B, prec)
+            x.run(12, prec)
+            assert not any("slots=8" in l for l in rt.log())
+    rt.budget(1 << 40)
+    with Solver() as s:
+        before = rt.used()
+        batch(s, dims, B, prec)
+        s.run(12, prec)
+        assert rt.used() - before > 4 * field
+        assert any("slots=8 bad=none" in l for l in rt.log())
+
+
+def test_responses_fit_beside_the_fields_of_a_batch(rt):
+    """A card with room for the two fields of an interleaved batch, its planes and its responses."""
+    dims, B, steps = (60, 40, 20), 8, 40000
+    field, resp = 4 * 60 * 40 * 20 * B, 8 * B * steps
+    rt.budget(rt.used() + 2 * field + resp + (2 << 20))
+    with Solver() as s:
+        batch(s, dims, B, N.F32)
+        s.run(steps, N.F32)
