@@ -385,6 +385,13 @@ int alloc_domain(pfdtd_ctx *c, int64_t X, int64_t Y, int64_t Z) {
     dfree(c->d_pm);
     c->dom_cap = 0;
   }
+  if (c->X != X || c->Y != Y || c->Z != Z) {  // the sweep's planes and events are those of a shape
+    dfree(c->d_entry);
+    dfree(c->d_row_bits);
+    dfree(c->d_ev_ptr);
+    dfree(c->d_events);
+    c->entry_cap = c->air_cap = c->ev_ptr_cap = c->ev_cap = 0;
+  }
   c->pm_ok = false;
   c->air3_ok = false;
   c->entry_ok = false;

@@ -120,3 +120,22 @@ def test_responses_fit_beside_the_fields_of_a_batch(rt):
     with Solver() as s:
         batch(s, dims, B, N.F32)
         s.run(steps, N.F32)
+
+
+@pytest.mark.parametrize("prec", [N.F32, N.F64, N.F16])
+def test_planes_of_a_room_are_given_back_with_it(rt, prec):
+    """A context that goes on to a room of another size holds what a fresh one on that room holds, and
+    fits a larger room where a fresh one fits."""
+    def on(*dims):
+        with Solver() as s:
+            for d in dims:
+                s.load_scene(scene(d))
+                s.run(12, prec)
+            return rt.used()
+
+    big, small, bigger = (150, 110, 80), (40, 30, 20), (160, 112, 84)
+    # what the context keeps of the larger room is no more than its few events
+    assert on(big, small) <= on(small) + 4096
+    held = on(bigger)
+    rt.budget(held + 4096)
+    on(big, bigger)
