@@ -1837,26 +1837,19 @@ int pfdtd_get_fields_raw(pfdtd_ctx *c, void *p_out, void *p_past_out, int64_t ca
   if (capacity_bytes < (int64_t)c->field_bytes) return fail(PFDTD_E_ARG, "output buffer too small");
   HIP_TRY(hipStreamSynchronize(c->stream));
   if (c->planar && c->lgB > 0) {
-    // [slot][voxel] to [voxel][slot], staged through a buffer of whole voxels
-    const size_t es = elem_size(c->precision), vox = es << c->lgB;
-    const int64_t chunk = std::max<int64_t>(1, std::min<int64_t>(c->N, (int64_t)((64u << 20) / vox)));
-    void *d_tmp = nullptr;
-    if (hipMalloc(&d_tmp, (size_t)chunk * vox) != hipSuccess) {
-      (void)hipGetLastError();
-      return fail(PFDTD_E_NOMEM, "no room to interleave the fields");
-    }
+    // [slot][voxel] to [voxel][slot], in the spare field: the next sweep writes all of it but the first
+    // and last slice of every slot, which are zeros
     hipError_t e = hipSuccess;
-    for (int f = 0; f < 2; ++f) {
-      char *out = (char *)(f ? p_past_out : p_out);
-      const void *src = f ? c->d_Pp : c->d_P;
-      for (int64_t v = 0; out && v < c->N && e == hipSuccess; v += chunk) {
-        const int64_t n = std::min(chunk, c->N - v);
-        e = launch_interleave((int)es, src, c->N, v, n, 1 << c->lgB, d_tmp, c->stream);
-        if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
-        if (e == hipSuccess) e = hipMemcpy(out + (size_t)v * vox, d_tmp, (size_t)n * vox, hipMemcpyDeviceToHost);
-      }
+    for (int f = 0; f < 2 && e == hipSuccess; ++f) {
+      void *out = f ? p_past_out : p_out;
+      if (!out) continue;
+      e = launch_interleave((int)elem_size(c->precision), f ? c->d_Pp : c->d_P, c->N, 1 << c->lgB, c->d_P2,
+                            c->stream);
+      if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
+      if (e == hipSuccess) e = hipMemcpy(out, c->d_P2, c->field_bytes, hipMemcpyDeviceToHost);
     }
-    (void)hipFree(d_tmp);
+    const hipError_t e2 = hipMemsetAsync(c->d_P2, 0, c->field_bytes, c->stream);
+    if (e == hipSuccess) e = e2;
     if (e != hipSuccess) return fail(PFDTD_E_HIP, "interleaved fields: %s", hipGetErrorString(e));
     return PFDTD_OK;
   }

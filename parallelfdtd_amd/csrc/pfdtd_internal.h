@@ -332,10 +332,9 @@ hipError_t launch_sweep_bf16(const SweepPlan &p, const SweepArgs<b16, CoefF, flo
 hipError_t launch_sweep_f64(const SweepPlan &p, const SweepArgs<double, CoefD, double> &a, int levels,
                             hipStream_t stream);
 
-// Voxels v0 .. v0 + n - 1 of a slot-major batch (element slot * N + voxel, elem_bytes each) to
-// [voxel][slot].
-hipError_t launch_interleave(int elem_bytes, const void *field, int64_t N, int64_t v0, int64_t n,
-                             int slots, void *out, hipStream_t stream);
+// A slot-major batch (element slot * N + voxel, elem_bytes each) to [voxel][slot].
+hipError_t launch_interleave(int elem_bytes, const void *field, int64_t N, int slots, void *out,
+                             hipStream_t stream);
 
 // Receiver gather of time index `gather_step` (skipped when < 0) followed by injection of
 // source samples of time index `inject_step` (skipped when < 0) into the same field.

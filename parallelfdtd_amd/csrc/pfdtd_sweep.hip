@@ -108,26 +108,25 @@ __global__ __launch_bounds__(64) void row_bits_kernel(const uint16_t *__restrict
 }
 
 template <typename T>
-__global__ __launch_bounds__(256) void interleave_kernel(const T *__restrict__ f, int64_t N,
-                                                         int64_t v0, int64_t n, int slots,
+__global__ __launch_bounds__(256) void interleave_kernel(const T *__restrict__ f, int64_t N, int slots,
                                                          T *__restrict__ out) {
-  const int64_t total = n * slots;
+  const int64_t total = N * slots;
   for (int64_t i = (int64_t)blockIdx.x * 256 + threadIdx.x; i < total; i += (int64_t)gridDim.x * 256)
-    out[i] = f[(i % slots) * N + v0 + i / slots];
+    out[i] = f[(i % slots) * N + i / slots];
 }
 
-hipError_t launch_interleave(int elem_bytes, const void *field, int64_t N, int64_t v0, int64_t n,
-                             int slots, void *out, hipStream_t stream) {
-  const dim3 grid((unsigned)std::min<int64_t>((n * slots + 255) / 256, 65536));
+hipError_t launch_interleave(int elem_bytes, const void *field, int64_t N, int slots, void *out,
+                             hipStream_t stream) {
+  const dim3 grid((unsigned)std::min<int64_t>((N * slots + 255) / 256, 65536));
   if (elem_bytes == 2)
     hipLaunchKernelGGL(interleave_kernel<uint16_t>, grid, dim3(256), 0, stream,
-                       (const uint16_t *)field, N, v0, n, slots, (uint16_t *)out);
+                       (const uint16_t *)field, N, slots, (uint16_t *)out);
   else if (elem_bytes == 4)
     hipLaunchKernelGGL(interleave_kernel<uint32_t>, grid, dim3(256), 0, stream,
-                       (const uint32_t *)field, N, v0, n, slots, (uint32_t *)out);
+                       (const uint32_t *)field, N, slots, (uint32_t *)out);
   else
     hipLaunchKernelGGL(interleave_kernel<uint64_t>, grid, dim3(256), 0, stream,
-                       (const uint64_t *)field, N, v0, n, slots, (uint64_t *)out);
+                       (const uint64_t *)field, N, slots, (uint64_t *)out);
   return hipGetLastError();
 }
 

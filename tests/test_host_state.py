@@ -139,3 +139,15 @@ def test_planes_of_a_room_are_given_back_with_it(rt, prec):
     held = on(bigger)
     rt.budget(held + 4096)
     on(big, bigger)
+
+
+@pytest.mark.parametrize("prec,raw", [(N.F32, np.float32), (N.F16, np.float16)])
+def test_fields_of_a_run_are_read_on_a_full_card(rt, prec, raw):
+    """A batch's fields are read out after a run without an allocation on the card."""
+    with Solver() as s:
+        batch(s, (60, 40, 20), 8, prec)
+        s.run(12, prec)
+        assert any("slots=8 bad=none" in l for l in rt.log())
+        rt.budget(rt.used())
+        P, Pp = s.fields_raw(raw)
+        assert P.shape == (20, 40, 60, 8)
