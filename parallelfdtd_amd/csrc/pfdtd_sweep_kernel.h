@@ -224,7 +224,28 @@ constexpr int sweep_ring(int L) { return L <= 2 ? 1 : L == 3 ? 2 : 4; }
 
 constexpr int kForward = 0, kDiff = 1, kCentred = 2;  // modes of the sweep
 
-constexpr uint32_t kDrop = 0x80000000u;  // offset bit that puts a store out of range
+constexpr uint32_t kDrop = 0x80000000u;  // offset bit that puts a store out of range (slices are below 2^31 bytes)
+
+// A lane's offsets in a slice of X columns, from its first column x0 in the first row yw of its wave, and
+// whether it drops the stores of its columns as a whole and of the first one alone (the last column of
+// an odd width). The drop bits are kept apart from the offsets: a row of a very wide grid added to a
+// dropped offset would carry it past 2^32 and back into the slice.
+struct SweepLane {
+  uint32_t off, drop, drop1;
+  __host__ __device__ uint32_t at(uint32_t row_off, uint32_t row_drop) const {
+    return (off + row_off) | drop | row_drop;
+  }
+  __host__ __device__ uint32_t at1(uint32_t row_off, uint32_t row_drop) const {
+    return (off + row_off) | drop1 | row_drop;
+  }
+};
+template <int NC, int HX>
+__host__ __device__ __forceinline__ SweepLane sweep_lane(int X, int x0, int yw, int lane, int elem) {
+  const bool own_x = NC * lane >= HX && NC * lane < 64 * NC - HX && x0 < X;
+  const bool pair = NC == 1 || x0 + 1 < X;  // the lane's columns both lie in the grid
+  return SweepLane{((uint32_t)yw * (uint32_t)X + (uint32_t)x0) * (uint32_t)elem,
+                   own_x && pair ? 0u : kDrop, own_x && !pair ? 0u : kDrop};
+}
 
 }  // namespace
 
@@ -285,12 +306,11 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
   const size_t XY = (size_t)X * (size_t)Y;
   const uint32_t sbytes = (uint32_t)(XY * sizeof(S));
   const size_t XYP = (size_t)a.pitch * (size_t)Y;
-  const uint32_t vcol = (uint32_t)((yw * X + x0) * (int)sizeof(S));
-  const uint32_t pcol = (uint32_t)((yw * a.pitch + x0) * 2);
+  const SweepLane sl = sweep_lane<NC, HX>(X, x0, yw, lane, (int)sizeof(S));
+  const uint32_t vcol = sl.off;
+  const uint32_t pcol = ((uint32_t)yw * (uint32_t)a.pitch + (uint32_t)x0) * 2u;
   // owned columns of this lane, owned rows of this wave
   const bool own_x = NC * lane >= HX && NC * lane < HX + OX && x0 < X;
-  const bool pair = NC == 1 || x0 + 1 < X;  // the lane's columns both lie in the grid
-  const uint32_t vst = own_x && pair ? vcol : kDrop, vst1 = own_x && !pair ? vcol : kDrop;
   uint32_t own_rows = 0;
 #pragma unroll
   for (int r = 0; r < TY; ++r) {
@@ -670,11 +690,11 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
       // issued since on the way with fewest, and the compiler makes ways past all of the kinds.
       __builtin_amdgcn_sched_barrier(0);
       const uint32_t drop = ((own_rows >> r) & 1u) ? 0u : kDrop;
-      if (L >= 2 || DIFF) R::st(rC, (vst + r * rstep) | drop, raw_c);
-      R::st(rD, (vst + r * rstep) | drop, raw_d);
+      if (L >= 2 || DIFF) R::st(rC, sl.at(r * rstep, drop), raw_c);
+      R::st(rD, sl.at(r * rstep, drop), raw_d);
       if (odd_edge) {
-        if (L >= 2 || DIFF) R::st1(rC, (vst1 + r * rstep) | drop, raw_c, 0);
-        R::st1(rD, (vst1 + r * rstep) | drop, raw_d, 0);
+        if (L >= 2 || DIFF) R::st1(rC, sl.at1(r * rstep, drop), raw_c, 0);
+        R::st1(rD, sl.at1(r * rstep, drop), raw_d, 0);
       }
       pl[r] = R::ld(ra, vcol + r * rstep);
       pq[r] = R::ld(rb, vcol + r * rstep);
