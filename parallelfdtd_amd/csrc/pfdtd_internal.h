@@ -233,7 +233,7 @@ template <typename S, typename CT, typename C>
 struct SweepArgs {
   const uint16_t *pm;  // coefficient entry per voxel, rows of `pitch` elements
   int pitch;
-  const uint32_t *row_bits;  // a word per wave tile and slice: rows of plain air, solid, unchanged
+  const uint32_t *row_bits;  // a word per wave tile and slice: rows of plain air, never updated, unchanged
   const int32_t *ev_ptr;     // per (slot, wave tile): first event, then one past the last
   const int32_t *events;     // {z, x, y, source index or receiver index | 1 << 31}, by z
   const S *A;

@@ -52,8 +52,8 @@ hipError_t launch_pack_entry(const uint8_t *pos, const uint8_t *mat, uint16_t *p
 }
 
 // A word per (wave tile, slice): bit r of the first byte is set when the tile's row r is plain air over
-// its whole window (and inside the grid), of the second when no voxel of it is updated (outside voxels,
-// past the grid, slices 0 and Z-1), of the third when its entries are those of the slice below (never on
+// its whole window (and inside the grid), of the second when it is never updated (rows 0 and Y-1, past
+// the grid, slices 0 and Z-1), of the third when its entries are those of the slice below (never on
 // slices 0, 1 and Z-1). Bits past the tile's rows are set in all. A wave per tile and run of slices, each
 // lane's columns of the slice below kept in registers, so every entry is loaded once per tile. On
 // 2048x1536x768 3.90 ms, a wave per slice with its slice below loaded again 9.26.
@@ -76,7 +76,6 @@ __global__ __launch_bounds__(64) void row_bits_kernel(const uint16_t *__restrict
     const uint16_t *q = pm + ((size_t)z * Y + y) * pitch + x;  // x and pitch even with two columns
     return (NC == 2 ? *(const uint32_t *)q : (uint32_t)*q) & use;
   };
-  auto is_out = [&](unsigned v) { return centred ? !(v & 0x80u) : v >= kStageRows * ncol; };
   auto is_air = [&](unsigned v) {
     return centred ? (v & 0xFFu) == 0x80u : v >= 6u * ncol && v < kStageRows * ncol;
   };
@@ -93,12 +92,11 @@ __global__ __launch_bounds__(64) void row_bits_kernel(const uint16_t *__restrict
         const int y = ys + r;
         const uint32_t v = entry(z, y);
         const bool not_air = !x_in || y < 0 || y >= Y || !is_air(v & 0xFFFFu) || (NC == 2 && !is_air(v >> 16));
-        const bool not_solid = y >= 0 && y < Y && ((in0 && !is_out(v & 0xFFFFu)) || (in1 && !is_out(v >> 16)));
         const bool changed = z < 2 || v != below[r];
         below[r] = v;
         if (!shell) {
           if (__ballot(not_air) == 0) ma |= 1u << r;
-          if (__ballot(not_solid) == 0) ms |= 1u << r;
+          if (y <= 0 || y >= Y - 1) ms |= 1u << r;
           if (__ballot(changed) == 0) mu |= 1u << r;
         }
       }
