@@ -782,7 +782,7 @@ hipError_t build_sweep_events(pfdtd_ctx *c, const SweepPlan &p) {
   std::vector<int32_t> ptr, data;
   sweep_events(p, batch_slots(c), rec, src, ptr, data);
   hipError_t e = grow(c->d_ev_ptr, c->ev_ptr_cap, ptr.size());
-  if (e == hipSuccess) e = grow(c->d_events, c->ev_cap, std::max<size_t>(data.size(), 4));
+  if (e == hipSuccess) e = grow(c->d_events, c->ev_cap, std::max<size_t>(data.size(), kEvInts));
   if (e == hipSuccess) e = hipStreamSynchronize(c->stream);
   if (e == hipSuccess)
     e = hipMemcpy(c->d_ev_ptr, ptr.data(), sizeof(int32_t) * ptr.size(), hipMemcpyHostToDevice);

@@ -235,7 +235,7 @@ struct SweepArgs {
   int pitch;
   const uint32_t *row_bits;  // a word per wave tile and slice: rows of plain air, never updated, unchanged
   const int32_t *ev_ptr;     // per (slot, wave tile): first event, then one past the last
-  const int32_t *events;     // {z, x, y, source index or receiver index | 1 << 31}, by z
+  const int32_t *events;     // by wave tile, slice and row: kEvInts ints each
   const S *A;
   const S *B;
   S *Cn;
@@ -292,14 +292,19 @@ struct SweepRate {
 };
 int sweep_zchunk(int n, const int64_t *bxy, const int *zi, int levels,
                  const SweepRate &rate = SweepRate{0, 1, 0, 1});
+// An event: slice, row of its wave tile, the first event of the tile's next row with events (or slice) and
+// of its next slice, column, and source index or receiver index | 1 << 31. A wave that looks for a row
+// on a slice passes over the others by these: 64 receivers in a patch of 8 x 8 of 256x256x256 FP32 take
+// 39 us per step, 102 with every event of the tile looked at, one receiver 26.
+constexpr int kEvInts = 8, kEvZ = 0, kEvRow = 1, kEvNextRow = 2, kEvNextZ = 3, kEvX = 4, kEvId = 5;
 // A source or receiver as the sweep's event lists take it.
 struct SweepPoint {
   int32_t x, y, z, slot, id;  // id: source index, or receiver index | 1 << 31
 };
-// Events by wave tile (ptr: n_slots * nby * wy * nbx + 1 entries) and slice (data: four ints each):
+// Events by wave tile (ptr: n_slots * nby * wy * nbx + 1 entries), slice and row (data: kEvInts ints each):
 // a source belongs to every tile whose window covers it (the levels below the last are computed
-// there too), a receiver to the tile that owns it; per tile by slice, the receivers of a slice
-// before its sources, each in index order.
+// there too), a receiver to the tile that owns it; the receivers of a row before its sources, each in
+// index order.
 void sweep_events(const SweepPlan &p, int slots, const std::vector<SweepPoint> &rec,
                   const std::vector<SweepPoint> &src, std::vector<int32_t> &ptr,
                   std::vector<int32_t> &data);

@@ -218,7 +218,7 @@ JobLayout layout_job(int X, int Y, int Z, size_t es, int n_src, int n_samples, i
   L.src_idx = take(sizeof(int64_t) * (size_t)n_src);
   // a source lies in the windows of at most two tiles along x and two along y
   L.ev_ptr = fused ? take(sizeof(int32_t) * (wave_tiles + 1)) : 0;
-  L.events = fused ? take(4 * sizeof(int32_t) * ((size_t)n_rec + 4 * (size_t)n_src)) : 0;
+  L.events = fused ? take(kEvInts * sizeof(int32_t) * ((size_t)n_rec + 4 * (size_t)n_src)) : 0;
   L.src_kind = take(sizeof(int32_t) * (size_t)n_src);
   L.sig = take(sizeof(float) * (size_t)n_src * (size_t)n_samples);
   L.rec_idx = take(sizeof(int64_t) * (size_t)n_rec);

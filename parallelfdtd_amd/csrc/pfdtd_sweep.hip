@@ -241,12 +241,12 @@ void sweep_events(const SweepPlan &p, int slots, const std::vector<SweepPoint> &
                   std::vector<int32_t> &data) {
   const int ntile = p.nby * p.wy * p.nbx;
   struct Ev {
-    int tile;
+    int tile, row;
     const SweepPoint *q;
   };
   std::vector<Ev> ev;
   auto add = [&](const SweepPoint &q, int bx, int by, int row) {
-    ev.push_back(Ev{q.slot * ntile + (by * p.wy + row / p.ty) * p.nbx + bx, &q});
+    ev.push_back(Ev{q.slot * ntile + (by * p.wy + row / p.ty) * p.nbx + bx, row % p.ty, &q});
   };
   for (const SweepPoint &q : rec)
     add(q, q.x / p.ox, q.y / p.oy, q.y % p.oy + p.lm);
@@ -262,16 +262,21 @@ void sweep_events(const SweepPlan &p, int slots, const std::vector<SweepPoint> &
       }
     }
   std::stable_sort(ev.begin(), ev.end(), [](const Ev &a, const Ev &b) {
-    return a.tile != b.tile ? a.tile < b.tile : a.q->z < b.q->z;
+    if (a.tile != b.tile) return a.tile < b.tile;
+    return a.q->z != b.q->z ? a.q->z < b.q->z : a.row < b.row;
   });
   ptr.assign((size_t)slots * ntile + 1, 0);
-  data.resize(4 * ev.size());
-  for (size_t i = 0; i < ev.size(); ++i) {
+  data.assign(kEvInts * ev.size(), 0);
+  for (size_t i = ev.size(); i-- > 0;) {
     ++ptr[(size_t)ev[i].tile + 1];
-    data[4 * i] = ev[i].q->z;
-    data[4 * i + 1] = ev[i].q->x;
-    data[4 * i + 2] = ev[i].q->y;
-    data[4 * i + 3] = ev[i].q->id;
+    int32_t *d = &data[kEvInts * i];
+    d[kEvZ] = ev[i].q->z;
+    d[kEvX] = ev[i].q->x;
+    d[kEvRow] = ev[i].row;
+    d[kEvId] = ev[i].q->id;
+    const bool z_goes_on = i + 1 < ev.size() && ev[i + 1].tile == ev[i].tile && ev[i + 1].q->z == ev[i].q->z;
+    d[kEvNextZ] = z_goes_on ? d[kEvInts + kEvNextZ] : (int32_t)(i + 1);
+    d[kEvNextRow] = z_goes_on && ev[i + 1].row == ev[i].row ? d[kEvInts + kEvNextRow] : (int32_t)(i + 1);
   }
   for (size_t i = 1; i < ptr.size(); ++i) ptr[i] += ptr[i - 1];
 }

@@ -349,10 +349,14 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
     ev = ((ConstI32)a.ev_ptr)[et];
     ev_end = ((ConstI32)a.ev_ptr)[et + 1];
   }
-  auto ev_at = [&](int n, int i) -> int {
+  struct EvHead {
+    int z, row, next_row, next_z;
+  };
+  auto ev_head = [&](int n) -> EvHead {  // one load of four words
     ConstArgs ka = args;
     asm volatile("" : "+s"(ka));
-    return ((ConstI32)ka->events)[4 * n + i];
+    const ConstI32 g = (ConstI32)ka->events + kEvInts * (int64_t)n;
+    return EvHead{g[kEvZ], g[kEvRow], g[kEvNextRow], g[kEvNextZ]};
   };
 
   V q[L][2][TY];  // level 0: P^n, level i: P^{n+i}; two slices each
@@ -433,7 +437,7 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
   // first event at or above the first slice of this chunk
   for (int hi = ev_end; ev < hi;) {
     const int mid = (ev + hi) >> 1;
-    if (ev_at(mid, 0) < kb)
+    if (ev_head(mid).z < kb)
       ev = mid + 1;
     else
       hi = mid;
@@ -460,8 +464,16 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
     const int hb = (k - 1) & 1;
     uint32_t ev_rows = 0;  // rows with an event on one of the slices k-L+1 .. k
     if (ev < ev_end) {
-      while (ev < ev_end && ev_at(ev, 0) < k - (L - 1)) ++ev;
-      for (int n = ev; n < ev_end && ev_at(n, 0) <= k; ++n) ev_rows |= 1u << (ev_at(n, 2) - yw);
+      for (int n = ev; n < ev_end;) {
+        const EvHead h = ev_head(n);
+        if (h.z > k) break;
+        if (h.z < k - (L - 1)) {
+          ev = n = h.next_z;
+        } else {
+          ev_rows |= 1u << h.row;
+          n = h.next_row;
+        }
+      }
     }
     // the rows that are air, fixed, of unchanged entries at every level, or have events: a byte each
     const uint32_t kinds = all_of(hist, L) | (all_of(hist_f, L) << 8) |
@@ -628,9 +640,16 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
           ConstArgs ka = args;
           asm volatile("" : "+s"(ka));
           const ConstI32 gev = (ConstI32)ka->events;
-          for (int n = ev; n < ev_end && gev[4 * n] <= k; ++n) {
-            if (gev[4 * n] != s || gev[4 * n + 2] != yw + r) continue;
-            const int xe = gev[4 * n + 1], id = gev[4 * n + 3];
+          for (int n = ev; n < ev_end;) {
+            const ConstI32 g = gev + kEvInts * (int64_t)n;
+            const EvHead h{g[kEvZ], g[kEvRow], g[kEvNextRow], g[kEvNextZ]};
+            if (h.z > s || (h.z == s && h.row > r)) break;
+            if (h.z < s || h.row < r) {
+              n = h.z < s ? h.next_z : h.next_row;
+              continue;
+            }
+            ++n;
+            const int xe = g[kEvX], id = g[kEvId];
             if (id < 0) {  // receiver
               const bool owned = own_x && ((own_rows >> r) & 1u) && s >= z0 && s < z1;
               const auto rr = sw_rsrc(ka->resp + (int64_t)(id & 0x7FFFFFFF) * ka->resp_steps,

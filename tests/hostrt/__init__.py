@@ -15,8 +15,8 @@ HERE = Path(__file__).resolve().parent
 UNDEFINED_IMAGE = re.compile(r"\bU (__hip_fatbin\w*)")
 
 
-def build(out: Path) -> Path:
-    """libpfdtd with the host half of every source only, linked to the stand-in runtime."""
+def _objects(sources: list[Path], out: Path) -> list[str]:
+    """The host half of HIP sources, compiled."""
     flags = [B.HIPCC, "--offload-arch=gfx950", "--cuda-host-only", "-O1", "-std=c++17", "-fPIC",
              "-I", str(B.ROOT / "include"), "-I", str(B.CSRC)]
 
@@ -26,14 +26,34 @@ def build(out: Path) -> Path:
         return str(obj)
 
     with ThreadPoolExecutor(8) as ex:
-        objs = list(ex.map(one, [*(B.CSRC / s for s in B.LIB_SOURCES), HERE / "fake_hip.cpp"]))
-    # no device images: the symbols that would name them are absolute zeros
-    images = sorted(set(UNDEFINED_IMAGE.findall(
-        subprocess.run(["nm", "-u", *objs], check=True, capture_output=True, text=True).stdout)))
+        return list(ex.map(one, sources))
+
+
+def _no_images(objs: list[str]) -> list[str]:
+    """No device images: the symbols that would name them are absolute zeros."""
+    names = subprocess.run(["nm", "-u", *objs], check=True, capture_output=True, text=True).stdout
+    return [f"-Wl,--defsym={s}=0" for s in sorted(set(UNDEFINED_IMAGE.findall(names)))]
+
+
+def build(out: Path) -> Path:
+    """libpfdtd with the host half of every source only, linked to the stand-in runtime."""
+    objs = _objects([*(B.CSRC / s for s in B.LIB_SOURCES), HERE / "fake_hip.cpp"], out)
     lib = out / "libpfdtd_host.so"
-    subprocess.run(["g++", "-shared", "-fPIC", "-Wl,-Bsymbolic", "-o", str(lib), *objs,
-                    *(f"-Wl,--defsym={s}=0" for s in images)], check=True)
+    subprocess.run(["g++", "-shared", "-fPIC", "-Wl,-Bsymbolic", "-o", str(lib), *objs, *_no_images(objs)],
+                   check=True)
     return lib
+
+
+def run_program(source: str, uses: list[str], out: Path) -> subprocess.CompletedProcess:
+    """A program over the library's host functions, with the named sources of it, run to its end."""
+    main = out / "program.hip"
+    main.write_text(source)
+    objs = _objects([main, HERE / "fake_hip.cpp", *(B.CSRC / u for u in uses)], out)
+    exe = out / "program"
+    # launchers of other sources are not called: their symbols may stay unresolved
+    subprocess.run(["g++", "-no-pie", *objs, *_no_images(objs), "-Wl,--unresolved-symbols=ignore-all",
+                    "-o", str(exe)], check=True)
+    return subprocess.run([str(exe)], capture_output=True, text=True)
 
 
 class Runtime:

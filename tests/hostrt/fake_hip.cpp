@@ -70,7 +70,7 @@ std::string sweep_line(const A &a, const std::vector<int> &t, unsigned blocks) {
   need("row_bits", a.row_bits, 4 * tiles * a.Z);
   need("ev_ptr", a.ev_ptr, 4 * (tiles * a.n_slots + 1));
   if (room(a.ev_ptr) >= 4 * (tiles * a.n_slots + 1))
-    need("events", a.events, 16 * (size_t)a.ev_ptr[tiles * a.n_slots]);
+    need("events", a.events, sizeof(int32_t) * kEvInts * (size_t)a.ev_ptr[tiles * a.n_slots]);
   const size_t field = (size_t)a.slot_elems * a.n_slots * sizeof(*a.A);
   for (const void *f : {(const void *)a.A, (const void *)a.B, (const void *)a.Cn, (const void *)a.Dn})
     need("field", f, field);

@@ -1,11 +1,7 @@
 """The byte offsets at which the lanes of the several-level sweep store, on the CPU: a lane that owns its
 columns and row stores at their place in the slice, every other one past the slice, also on grids whose
 rows are a large part of 2^31 bytes."""
-import subprocess
-
-import pytest
-
-from parallelfdtd_amd import build as B
+import hostrt
 
 SOURCE = r"""
 #include "pfdtd_sweep_kernel.h"
@@ -59,11 +55,5 @@ int main() { return sizes<float>() + sizes<double>() + sizes<h16>() ? 1 : 0; }
 
 
 def test_store_offsets(tmp_path):
-    src, exe = tmp_path / "offsets.hip", tmp_path / "offsets"
-    src.write_text(SOURCE)
-    subprocess.run([B.HIPCC, "--offload-arch=gfx950", "--cuda-host-only", "-O1", "-std=c++17",
-                    "-I", str(B.ROOT / "include"), "-I", str(B.CSRC), "-c", str(src), "-o", str(exe) + ".o"],
-                   check=True)
-    subprocess.run([B.HIPCC, str(exe) + ".o", "-o", str(exe)], check=True)
-    out = subprocess.run([str(exe)], capture_output=True, text=True)
+    out = hostrt.run_program(SOURCE, [], tmp_path)
     assert out.returncode == 0, out.stdout
