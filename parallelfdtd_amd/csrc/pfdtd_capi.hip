@@ -806,7 +806,8 @@ bool sweep_eligible(const pfdtd_ctx *c) {
 // by slot, if its four buffers take no more than half of the free memory (the interleaved layout does
 // with two, and what it leaves is other contexts'): 32 sources on 512x384x256 take 1.9 ms per step that way against
 // 4.27 with the single-step kernel of the interleaved layout, which reads and writes every field
-// at every step. Prepared fields have the buffers of a run, but stay interleaved for steps that follow
+// at every step; not where a poll interval of 1 leaves no several levels (32 sources on 256x200x120: 519 us
+// per step interleaved, 778 slot by slot). Prepared fields have the buffers of a run, but stay interleaved for steps that follow
 // (32 sources on 256x200x120: 539 us per step against 799 slot by slot).
 enum class Use { kPrepare, kRun, kSteps };
 int ensure_fields_for(pfdtd_ctx *c, int precision, int scale_exp, Use use) {
@@ -823,7 +824,7 @@ int ensure_fields_for(pfdtd_ctx *c, int precision, int scale_exp, Use use) {
   }
   const bool want4 = (c->lgB == 0 || c->grouped) && levels_for(c, precision) >= 2;
   const bool was = c->planar;
-  c->planar = spare && use == Use::kRun;
+  c->planar = spare && use == Use::kRun && c->poll_interval > 1;
   rc = ensure_fields(c, precision, scale_exp, want4 || spare);
   if (rc == PFDTD_E_NOMEM && spare) {
     c->planar_nomem = bytes;
@@ -939,6 +940,33 @@ hipError_t run_sweep(pfdtd_ctx *c, const SweepPlan &p, int step, int levels, int
     c->d_P2 = spare;
   }
   return e;
+}
+
+// Whether a single step is better taken as one (an update and a gather/injection launch) than as a sweep
+// of one level, whose tiles compute a halo for five and whose chunks are cut for five. Not in rooms of
+// the small tile (130x98x66 FP32: sweep 22.3 us, single step 23.4, FP64 22.6, 28.3) and not in the difference
+// form, which has no single step. us per call of one step, single step against sweep, where the line
+// lies: the centred scheme 448x264x135 69, 101; FP32 by the nodes that the tiles of either cover
+// (256x256x256 57, 68; 384x320x256 119, 100; 640x480x320 285, 262; 1024x768x384 813, 869); FP64 by size (512x384x256
+// 282, 277; 640x480x320 533, 554; 1024x768x384 1617, 1822); 16-bit storage by whether its two fields fit the
+// Infinity Cache (FP16 256x256x256 44, 57; 512x384x256 111, 125; 640x480x320 218, 200; 1600x900x400 1121, 1011).
+bool single_step_better(const pfdtd_ctx *c, const SweepPlan &p) {
+  if (p.tile != 0 || c->precision == PFDTD_F16_DIFF) return false;
+  if (c->scheme == 2) return true;
+  const int64_t fields = 2 * (int64_t)c->field_bytes;
+  if (c->precision == PFDTD_F64) return fields > (int64_t)1 << 30;
+  if (c->precision != PFDTD_F32) return fields <= (int64_t)256 << 20;
+  const UpdateGeom g = plan_single(c);
+  const int64_t single = (int64_t)g.grid.x * g.block.x * g.grid.y * g.ry;
+  return (int64_t)p.nbx * p.ox * p.nby * p.oy > single;
+}
+
+// Whether calls of two steps are better left to the two-column sweep of two levels: large rooms of 16-bit
+// storage. us per step, two-column against several-level sweep: FP16 768x576x288 212, 203; 1024x768x384 385,
+// 439; 1600x900x400 666, 779; BF16 429, 415 and 720, 782.
+bool two_steps_better(const pfdtd_ctx *c, int steps) {
+  return steps == 2 && (c->precision == PFDTD_F16 || c->precision == PFDTD_BF16) && c->scheme == 0 &&
+         c->lgB == 0 && c->X % 2 == 0 && 4 * (int64_t)c->field_bytes > (int64_t)2 << 30;
 }
 
 int ensure_events(pfdtd_ctx *c, size_t n) {
@@ -1487,7 +1515,7 @@ int pfdtd_run(pfdtd_ctx *c, int precision, int n_steps, pfdtd_interrupt_cb inter
     HIP_TRY(launch_inject_gather(p_storage(c->precision), c->d_P, ia, c->stream));
   }
 
-  bool sweep = diff || sweep_eligible(c);
+  bool sweep = diff || (sweep_eligible(c) && !two_steps_better(c, std::min(bundle, n_steps)));
   SweepPlan sp{};
   if (sweep) {
     sp = plan_sweep(c->precision, (int)c->X, (int)c->Y, (int)c->Z, c->fzc, batch_slots(c));
@@ -1496,6 +1524,7 @@ int pfdtd_run(pfdtd_ctx *c, int precision, int n_steps, pfdtd_interrupt_cb inter
     if (diff && !sweep)
       return fail(PFDTD_E_NOMEM, "no room for the entry plane the difference form's sweep reads");
   }
+  const bool single = sweep && single_step_better(c, sp);
   bool fused = !sweep && fused_eligible(c);
   rc = ensure_pm(c, &fused);
   if (rc) return rc;
@@ -1519,7 +1548,7 @@ int pfdtd_run(pfdtd_ctx *c, int precision, int n_steps, pfdtd_interrupt_cb inter
     int nev = 0;
     for (int k = 0; k < nb;) {
       const int step = done + k;
-      if (sweep) {
+      if (sweep && !(single && nb - k == 1)) {
         const int lv = std::min(sp.lm, nb - k);
         if (c->kernel_timing) HIP_TRY(hipEventRecord(c->events[2 * nev], c->stream));
         HIP_TRY(run_sweep(c, sp, step, lv, n_steps));
@@ -1654,13 +1683,14 @@ int pfdtd_steps(pfdtd_ctx *c, int first_step, int n_steps) {
     if (n_steps == 0) return PFDTD_OK;
   }
   const UpdateGeom g = plan_single(c);
-  bool sweep = sweep_eligible(c);
+  bool sweep = sweep_eligible(c) && !two_steps_better(c, n_steps);
   SweepPlan sp{};
   if (sweep) {
     sp = plan_sweep(c->precision, (int)c->X, (int)c->Y, (int)c->Z, c->fzc, batch_slots(c));
     rc = ensure_sweep(c, sp, &sweep);
     if (rc) return rc;
   }
+  const bool single = sweep && single_step_better(c, sp);
   bool fused = !sweep && fused_eligible(c);
   rc = ensure_pm(c, &fused);
   if (rc) return rc;
@@ -1679,7 +1709,7 @@ int pfdtd_steps(pfdtd_ctx *c, int first_step, int n_steps) {
   HIP_TRY(launch_inject_gather(c->precision, c->d_P, inject_args(c, -1, first_step), c->stream));
   for (int k = 0; k < n_steps;) {
     const int step = first_step + k;
-    if (sweep) {
+    if (sweep && !(single && n_steps - k == 1)) {
       const int lv = std::min(sp.lm, n_steps - k);
       HIP_TRY(run_sweep(c, sp, step, lv, first_step + n_steps));
       k += lv;

@@ -151,3 +151,37 @@ def test_fields_of_a_run_are_read_on_a_full_card(rt, prec, raw):
         rt.budget(rt.used())
         P, Pp = s.fields_raw(raw)
         assert P.shape == (20, 40, 60, 8)
+
+
+# rooms of the large tile: whether a call of one step takes the single-step update, and of two steps
+# the two-column sweep
+SHORT_CALLS = [
+    ((256, 256, 256), N.F32, False, True, False), ((384, 320, 256), N.F32, False, False, False),
+    ((130, 98, 66), N.F32, False, False, False), ((448, 264, 135), N.F32, True, True, False),
+    ((384, 320, 256), N.F64, False, False, False), ((640, 480, 320), N.F64, False, True, False),
+    ((256, 256, 256), N.F16, False, True, False), ((640, 480, 320), N.F16, False, False, False),
+    ((1024, 768, 384), N.F16, False, False, True), ((1023, 768, 384), N.F16, False, False, False),
+    ((256, 256, 256), N.BF16, False, True, False), ((640, 480, 320), N.BF16, False, False, False),
+]
+
+
+@pytest.mark.parametrize("dims,prec,centred,single,pair", SHORT_CALLS)
+def test_short_calls_take_the_faster_kernels(rt, dims, prec, centred, single, pair):
+    lab = rooms.box_room(*dims)
+    with Solver() as s:
+        if centred:
+            s.set_update_type(N.SRL)
+        s.set_domain_labels(lab)
+        s.set_materials(np.full((1, 20), 0.1, np.float32))
+        s.begin_steps(20, prec)
+        got = {}
+        for first, n in ((0, 1), (1, 2), (3, 6), (9, 4)):
+            rt.log()
+            s.steps(first, n)
+            got[n] = [l for l in rt.log() if "inject" not in l]
+    is_sweep = lambda l: l.startswith("sweep")
+    assert all("update_kernel" in l if single else is_sweep(l) and "levels=1" in l for l in got[1][-1:])
+    assert all(("update2" in l) if pair else is_sweep(l) for l in got[2][-1:])
+    assert is_sweep(got[4][-1])
+    if not got[6][-1].startswith("sweep") or "levels=1 " in got[6][-1]:  # five levels and a single step
+        assert is_sweep(got[6][-2]) and ("update_kernel" in got[6][-1]) == single
