@@ -148,16 +148,16 @@ int sweep_zchunk(int n, const int64_t *bxy, const int *zi, int levels, const Swe
   int top = 1, best_c = 1;
   for (int i = 0; i < n; ++i) top = std::max(top, zi[i]);
   double best = 0;
-  for (int nz = 1; nz <= top; ++nz) {
-    const int c = (top + nz - 1) / nz;
-    if (nz > 1 && c == (top + nz - 2) / (nz - 1)) continue;
+  // every chunk length that a number of chunks gives, once: some 2 sqrt(top) of them
+  for (int64_t nz = 1, c = top;; nz = ((int64_t)top + c - 2) / (c - 1), c = (top + nz - 1) / nz) {
     int64_t blocks = 0;
     for (int i = 0; i < n; ++i) blocks += bxy[i] * ((zi[i] + c - 1) / c);
-    const double us = sweep_us(rate, blocks, c, levels);
+    const double us = sweep_us(rate, blocks, (int)c, levels);
     if (nz == 1 || us < best) {
       best = us;
-      best_c = c;
+      best_c = (int)c;
     }
+    if (c == 1) break;
   }
   return best_c;
 }
