@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import hostrt
+import large_tile
 from parallelfdtd_amd import native as N
 from parallelfdtd_amd import rooms
 from parallelfdtd_amd.solver import Solver
@@ -185,3 +186,22 @@ def test_short_calls_take_the_faster_kernels(rt, dims, prec, centred, single, pa
     assert is_sweep(got[4][-1])
     if not got[6][-1].startswith("sweep") or "levels=1 " in got[6][-1]:  # five levels and a single step
         assert is_sweep(got[6][-2]) and ("update_kernel" in got[6][-1]) == single
+
+
+@pytest.mark.parametrize("dx,dy,zchunk,n_steps", large_tile.BORDERS)
+@pytest.mark.parametrize("prec,centred", [(p, c) for p in large_tile.ELEM for c in (False, True)
+                                          if not (c and p == N.F16_DIFF)])
+def test_rooms_of_the_large_tile_take_it(rt, prec, centred, dx, dy, zchunk, n_steps):
+    """The rooms of the GPU tests of the large tile."""
+    ox, oy, hx, lm = large_tile.TILE[prec]
+    with Solver() as s:
+        if centred:
+            s.set_update_type(N.SRL)
+        s.set_time_levels(0, zchunk)
+        s.set_domain_labels(rooms.box_room(*large_tile.dims(prec, dx, dy)))
+        s.set_materials(np.full((1, 20), 0.1, np.float32))
+        rt.log()
+        s.run(n_steps, prec)
+        lines = [l for l in rt.log() if l.startswith("sweep")]
+    assert lines and all(f"tile={ox},{hx},{oy}," in l and l.endswith("bad=none") for l in lines), lines
+    assert f"levels={min(lm, n_steps)} " in lines[0]
