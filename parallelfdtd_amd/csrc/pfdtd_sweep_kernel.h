@@ -69,6 +69,7 @@
 #include "pfdtd_device.h"
 
 #include <type_traits>
+#include <utility>
 
 namespace pfdtd {
 
@@ -96,6 +97,11 @@ __device__ __forceinline__ double sw_prev(double v) {
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t sw_rsrc(const void *p, uint32_t nbytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void *>(p), (short)0, (int)nbytes,
                                            0x00020000);
+}
+
+template <int... R, typename F>
+__device__ __forceinline__ void sw_inner_rows(std::integer_sequence<int, R...>, F &f) {
+  (f(R + 1), ...);
 }
 
 // Keeps a value's computation ahead of the select that masks it (a select between it and 0 would
@@ -724,8 +730,8 @@ __device__ __forceinline__ void sweep_block(ConstSweepArgs<S> args, unsigned til
       pl[r] = R::ld(ra, vcol + r * rstep);
       pq[r] = R::ld(rb, vcol + r * rstep);
     };
-#pragma unroll
-    for (int r = 1; r < TY - 1; ++r) rows(r);
+    // not a loop: its body is beyond what the compiler unrolls, and the queue would go to memory
+    sw_inner_rows(std::make_integer_sequence<int, TY - 2>(), rows);
     rows(0);
     rows(TY - 1);
     // publish the edge rows of the new slices
