@@ -8,12 +8,10 @@ slots -- timing a short run of each candidate on the real domain.
 Throughput is per source: voxel-updates/s summed over the B slots,
   per_source_gvox = N_nodes * B * steps / seconds / 1e9,
 with the step loop's own HIP-event time (injection and gather included). B = 1 is timed both
-as the unbatched single-level update (the batched kernel's own baseline), as the explicit
+as the unbatched single-level update (the batched kernel's own baseline) and as the default
 unbatched paths, the two-time-level sweep (z-chunks `TWO_LEVEL_ZCHUNKS`, column and wide blocks)
-and the three-time-level sweep (z-chunks `THREE_LEVEL_ZCHUNKS`, blocks of 2 x 2 wave tiles), and as
-the default (levels 0: the several-level sweep); the best of all candidates is the tuner's choice,
-never slower than the unbatched default. Batches are not timed with the default setting, which
-is the faster one for them too (8 sources on 512x384x256 FP32: 414 us per step, 770 with three levels).
+and the three-time-level sweep (z-chunks `THREE_LEVEL_ZCHUNKS`, blocks of 2 x 2 wave tiles); the
+best of all candidates is the tuner's choice.
 
 Run:  python -m parallelfdtd_amd.autotune --batches 1,8,16,32,64 --out tune_c4.json
 """
@@ -124,10 +122,6 @@ def sweep(scene, batches=(1, 8, 16, 32, 64), rows=(1, 2, 4, 8), zchunks=(4, 8, 1
                     cand = record(B, 3, None, zc, time_config(s, steps, warmup, N.F32), "square")
                     if cand["per_source_gvox"] > best["per_source_gvox"]:
                         best = cand
-                s.set_time_levels(0)
-                cand = record(B, 0, None, 0, time_config(s, steps, warmup, N.F32))
-                if cand["per_source_gvox"] > best["per_source_gvox"]:
-                    best = cand
                 s.set_time_levels(1)
             out["best"][str(B)] = best
     for table in (out["best"], out["best_single_level"]):
