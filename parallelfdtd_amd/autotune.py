@@ -8,10 +8,12 @@ slots -- timing a short run of each candidate on the real domain.
 Throughput is per source: voxel-updates/s summed over the B slots,
   per_source_gvox = N_nodes * B * steps / seconds / 1e9,
 with the step loop's own HIP-event time (injection and gather included). B = 1 is timed both
-as the unbatched single-level update (the batched kernel's own baseline) and as the default
+as the unbatched single-level update (the batched kernel's own baseline) and as the explicit
 unbatched paths, the two-time-level sweep (z-chunks `TWO_LEVEL_ZCHUNKS`, column and wide blocks)
 and the three-time-level sweep (z-chunks `THREE_LEVEL_ZCHUNKS`, blocks of 2 x 2 wave tiles); the
-best of all candidates is the tuner's choice.
+best of all candidates is the tuner's choice. All of these are explicit settings. What an untuned
+solver takes (levels 0, the several-level sweep) is timed unbatched beside them as "default", with
+whether it is faster than the choice: then the choice is better left unapplied.
 
 Run:  python -m parallelfdtd_amd.autotune --batches 1,8,16,32,64 --out tune_c4.json
 """
@@ -122,6 +124,10 @@ def sweep(scene, batches=(1, 8, 16, 32, 64), rows=(1, 2, 4, 8), zchunks=(4, 8, 1
                     cand = record(B, 3, None, zc, time_config(s, steps, warmup, N.F32), "square")
                     if cand["per_source_gvox"] > best["per_source_gvox"]:
                         best = cand
+                s.set_time_levels(0)
+                ms = time_config(s, steps, warmup, N.F32)
+                out["default"] = {"B": 1, "levels": 0, "ms_per_step": float(f"{ms:.6g}"),
+                                  "per_source_gvox": float(f"{nodes / (ms * 1e-3) / 1e9:.6g}")}
                 s.set_time_levels(1)
             out["best"][str(B)] = best
     for table in (out["best"], out["best_single_level"]):
@@ -131,6 +137,8 @@ def sweep(scene, batches=(1, 8, 16, 32, 64), rows=(1, 2, 4, 8), zchunks=(4, 8, 1
                 v["per_source_speedup_vs_B1"] = float(f"{v['per_source_gvox'] / base['per_source_gvox']:.4g}")
     top = max(out["best"].values(), key=lambda c: c["per_source_gvox"])
     out["choice"] = {k: top[k] for k in ("B", "layout", "levels", "rows", "zchunk", "shape")}
+    if "default" in out:
+        out["default"]["faster_than_choice"] = out["default"]["per_source_gvox"] > top["per_source_gvox"]
     return out
 
 
@@ -154,7 +162,8 @@ def main(argv=None) -> int:
         Path(args.out).parent.mkdir(parents=True, exist_ok=True)
         Path(args.out).write_text(text)
     print(json.dumps({"scene": rep["scene"], "best": rep["best"],
-                      "best_single_level": rep["best_single_level"], "choice": rep["choice"]}))
+                      "best_single_level": rep["best_single_level"], "choice": rep["choice"],
+                      "default": rep.get("default")}))
     return 0
 
 
