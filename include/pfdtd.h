@@ -300,7 +300,10 @@ int pfdtd_set_poll_interval(pfdtd_ctx *ctx, int steps);
  * gathered inside the kernel; four field buffers. A remainder of one step takes a single-step
  * update (so does every step while a source sits on slice z = 0 or z = Z-1), four steps left
  * take two pairs. Non-grouped batches advance one level per sweep
- * with an explicit setting and are held slot by slot for the several-level sweep. Results are bit-identical
+ * with an explicit setting and are held slot by slot for the several-level sweep in pfdtd_run (four
+ * fields instead of two, where these take no more than half of the free memory, and unless the poll
+ * interval is 1). A single step left over takes the single-step update, and a call of two steps the
+ * two-column sweep, where that is the faster one. Results are bit-identical
  * to single steps. No reference counterpart: the reference's loop (kernels3d.cu:83-191)
  * launches one update per step. */
 int pfdtd_set_time_levels(pfdtd_ctx *ctx, int levels, int zchunk);

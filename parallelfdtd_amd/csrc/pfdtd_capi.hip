@@ -293,7 +293,8 @@ int64_t lin_idx(const pfdtd_ctx *c, const int32_t *q) {
   return ((int64_t)q[2] * c->Y + q[1]) * c->X + q[0];
 }
 
-// Slots one two-level launch advances (grouped batch), 1 otherwise.
+// Whether a batch's fields lie one slot after another, and the slots one launch of a sweep then advances
+// (1 otherwise).
 bool slot_major(const pfdtd_ctx *c) { return c->grouped || c->planar; }
 int batch_slots(const pfdtd_ctx *c) { return slot_major(c) ? 1 << c->lgB : 1; }
 
@@ -348,12 +349,12 @@ int scan_domain(pfdtd_ctx *c) {
   return PFDTD_OK;
 }
 
-// Time levels per sweep: the explicit setting, else three for FP32 and FP64 (unbatched or in
-// the grouped batch layout) and two otherwise. Same buffers, alternating settings: on the
-// 2048x1536x768 room three levels take FP32 from 4.37 to 3.85 ms per step and FP64 from 8.61
-// to 7.4-7.7, on 1024x768x384 FP32 from 0.71 to 0.55 and FP64 from 1.19 to 1.06; 16-bit
-// storage stays on the two-column two-level sweep (2.67 ms against 3.46 for three levels of one
-// column). Two levels were faster than single steps for every precision (FP32 7.35 vs 7.74 ms
+// Time levels of the sweeps of independent waves, which runs take where the several-level sweep cannot: the
+// explicit setting, else three for FP32 and FP64 (unbatched or held slot by slot) and two otherwise. Same
+// buffers, alternating settings: on the 2048x1536x768 room three levels take FP32 from 4.37 to 3.85
+// ms per step and FP64 from 8.61 to 7.4-7.7, on 1024x768x384 FP32 from 0.71 to 0.55 and FP64 from
+// 1.19 to 1.06; 16-bit storage takes the two-column two-level sweep (2.67 ms against 3.46 for three
+// levels of one column). Two levels were faster than single steps for every precision (FP32 7.35 vs 7.74 ms
 // per step on the large room).
 int levels_for(const pfdtd_ctx *c, int precision) {
   if (c->levels) return c->levels;
@@ -855,7 +856,7 @@ int ensure_sweep(pfdtd_ctx *c, const SweepPlan &p, bool *ok) {
   if (e == hipSuccess && !std::equal(key, key + 4, c->sweep_key)) {
     std::fill(c->sweep_key, c->sweep_key + 4, 0);
     c->events_ok = false;
-    e = grow(c->d_row_bits, c->air_cap, sweep_row_words(p));
+    e = grow(c->d_row_bits, c->air_cap, sweep_row_words(p, c->Z));
     if (e == hipSuccess)
       e = launch_row_bits(p, c->d_entry, c->d_row_bits, (int)c->X, (int)c->Y, (int)c->Z, ncol,
                           c->scheme, c->stream);

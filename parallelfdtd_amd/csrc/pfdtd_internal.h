@@ -268,12 +268,12 @@ struct SweepPlan {
   double us;             // modelled time of a launch
   int nc, ty, wy, lm;    // columns per lane, rows per wave, waves per block, most levels
   int w, hx, ox, oy;     // window columns, halo columns, owned columns and rows of a block
-  int nbx, nby, zc, band, words, pitch;
+  int nbx, nby, zc, band, pitch;
   int64_t blocks;
 };
-// Words of a plan's row bits.
-inline size_t sweep_row_words(const SweepPlan &p) {
-  return (size_t)p.nbx * p.nby * p.wy * p.words;
+// Words of a plan's row bits for a room of Z slices.
+inline size_t sweep_row_words(const SweepPlan &p, int64_t Z) {
+  return (size_t)p.nbx * p.nby * p.wy * (size_t)Z;
 }
 SweepPlan plan_sweep(int precision, int X, int Y, int Z, int zc, int slots, bool pool = false);
 // Fills the tile geometry of a sweep's arguments.

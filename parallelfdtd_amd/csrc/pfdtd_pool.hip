@@ -5,7 +5,7 @@
 // receivers), a state (step, current buffer, past buffer) and, for the several-level sweep, the
 // sweep's arguments in device memory, indexed by the job's slot. Jobs are advanced in rounds of
 // kPoolLevels steps. A job whose sources avoid the never-updated first and last z slices owns four
-// field buffers and is advanced by the sweep (srl_sweep_pool_kernel, pfdtd_sweep.hip): ONE launch
+// field buffers and is advanced by the sweep (srl_sweep_pool_kernel, pfdtd_sweep_kernel.h): ONE launch
 // per storage type and round enumerates the tiles of every such job (a block finds its job by a
 // binary search over the launch table's tile prefix), gathers and injections included; the steps
 // that do not fill a round are taken when the job is admitted. After the rounds of a bundle one
@@ -212,7 +212,7 @@ JobLayout layout_job(int X, int Y, int Z, size_t es, int n_src, int n_samples, i
   L.pos = take((size_t)N);
   L.mat = take((size_t)N);
   L.entry = fused ? take(sizeof(uint16_t) * (size_t)sp.pitch * Y * Z) : 0;
-  L.row_bits = fused ? take(sizeof(uint32_t) * sweep_row_words(sp)) : 0;
+  L.row_bits = fused ? take(sizeof(uint32_t) * sweep_row_words(sp, Z)) : 0;
   L.labels = take((size_t)N);
   L.coef = take(sizeof(CoefF) * kCoefEntries);
   L.src_idx = take(sizeof(int64_t) * (size_t)n_src);

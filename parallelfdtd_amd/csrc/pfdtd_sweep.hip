@@ -179,7 +179,6 @@ SweepPlan plan_of(int X, int Y, int Z, int zc, int slots) {
   p.oy = T::TY * T::WY - 2 * T::LM;
   p.nbx = (int)(((int64_t)X + p.ox - 1) / p.ox);
   p.nby = (int)(((int64_t)Y + p.oy - 1) / p.oy);
-  p.words = Z;
   p.pitch = (int)((int64_t)X + (X & 1));
   p.band = 2;
   const int zi = std::max(Z - 2, 1);  // a size query may ask for a room without an inner slice

@@ -17,8 +17,8 @@
 // three-level sweep computes 1.8 nodes and loads 4.5 rows per node-update it keeps, this one 1.5 (L =
 // 5) and 2.2.
 //
-// What bounds it (2048x1536x768 FP32, L = 5): 2.06-2.33 ms per step against 3.73-3.83 for the
-// three-level sweep of independent waves, 19.4 GB written and 30.4 read per launch at 4.8 TB/s of a
+// What bounds it (2048x1536x768 FP32, L = 5): 2.04-2.33 ms per step against 3.73-3.83 for the
+// three-level sweep of independent waves, 19.4 GB written and 30.2 read per launch at 4.85 TB/s of a
 // copy's 5.5: the traffic. FP64 (L = 4): 1024x768x384 0.64 ms against 1.03. Rooms in the Infinity Cache
 // are bound by issue (below). Tiles measured before the last steps (ms per step, 2048x1536x768 FP32, same card): L = 4
 // 8 rows 2.95, 6 rows 2.96; L = 5 6 rows 2.52, 7 rows (spills) 2.55; L = 6 does not fit LDS. Windows: stores of
@@ -51,8 +51,8 @@
 //
 // The difference form (A holds P^n, B holds D^n = P^n - P^{n-1}; P^{n+L} to Dn and D^{n+L} to Cn, both
 // from the last level) also keeps every level's rounded differences of one slice; the past value of a
-// node is P - D in FP32, and a sample keeps it. 249 VGPRs. 640x480x320 hall, 400 steps: 66.7 ms with
-// the two-level sweep of independent waves -> 52.7.
+// node is P - D in FP32, and a sample keeps it. 256 VGPRs, two spilled. 640x480x320 hall, 400 steps: 66.7 ms
+// with the two-level sweep of independent waves -> 49.
 //
 // The centred boundaries take the same tiles: the entry plane holds position and material bytes, and the
 // DIR and SIGN bits pick the neighbour that stands in for a missing one (15 VALU operations per air node,
@@ -808,13 +808,20 @@ __global__ __launch_bounds__(64 * WY, (WY + 3) / 4) void srl_sweep_pool_kernel(
 // columns; and the cost model of a launch in us: T0 + slices marched (chunk + 2 (levels - 1) + 2) times
 // A + B n, n <= CAP the blocks that share a CU.
 //
-// V = 0: eight waves at 229 (FP32) and 233 (FP64) VGPRs, two waves per SIMD and one block per CU (160 KB
+// V = 0: eight waves at 238 (FP32) and 236 (FP64) VGPRs, two waves per SIMD and one block per CU (160 KB
 // of LDS with 255 materials). V = 1: for rooms that give the large tile too few blocks or too short
 // chunks. It computes 1.5 times the nodes and launches more often per step, but fills the chip with a
 // third of the rows and half the columns per block, three blocks (FP64 two) to a CU. us per step, large ->
 // small: 130x98x66 FP32 11.3 -> 6.9, FP16 12.1 -> 6.9, FP64 10.5 -> 8.1; 157x111x75 FP32 11.2 -> 7.9, FP64
 // 11.4 -> 8.9; 200x150x120 FP32 13.2 -> 11.3, FP64 15.0 -> 12.8; 256x256x256 FP32 26.9 -> 32.9, FP64 41.5
 // -> 50.0. Other small tiles, FP32 on 130x98x66: two columns and 2 rows 7.5, 3 rows 7.7.
+//
+// The rates are those of forward runs in FP32 and FP64. 16-bit storage, the difference form and the centred
+// boundaries take them too, without rates of their own. Large -> small, us per step: FP16 256x256x256 27.5 ->
+// 29.3, 448x264x135 21.6 -> 26.0, 200x150x120 12.4 -> 10.6, BF16 256x256x256 26.3 -> 29.5; difference form
+// 256x256x256 34.2 -> 30.2, 320x240x200 29.0 -> 25.5, 640x480x320 124 -> 136; centred FP32 256x256x256 54.7
+// -> 45.6, 448x264x135 46.4 -> 41.8, 640x480x320 201 -> 240, centred FP64 256x200x160 33.7 -> 37.6,
+// 256x256x256 51.9 -> 63.4: for the last two modes the line lies up to 17 % off in the rooms between.
 template <typename S, int V>
 struct SweepTile {
   static constexpr int NC = 2, TY = 6, WY = 8, LM = 5, HX = 8, CAP = 1;
