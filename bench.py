@@ -240,7 +240,7 @@ def main() -> int:
     ap.add_argument("--fp16-only", action="store_true",
                     help="only the FP16-storage run (profiling); prints no bench line")
     ap.add_argument("--fp64-only", action="store_true",
-                    help="only the FP64 run (three-level sweep; profiling); prints no bench line")
+                    help="only the FP64 run (several-level sweep; profiling); prints no bench line")
     ap.add_argument("--f16diff-only", action="store_true",
                     help="only the FP16 difference-form run (profiling); prints no bench line")
     ap.add_argument("--copy-calibration", action="store_true",

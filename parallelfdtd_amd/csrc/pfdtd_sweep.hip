@@ -56,7 +56,7 @@ hipError_t launch_pack_entry(const uint8_t *pos, const uint8_t *mat, uint16_t *p
 // the grid, slices 0 and Z-1), of the third when its entries are those of the slice below (never on
 // slices 0, 1 and Z-1). Bits past the tile's rows are set in all. A wave per tile and run of slices, each
 // lane's columns of the slice below kept in registers, so every entry is loaded once per tile. On
-// 2048x1536x768 3.90 ms, a wave per slice with its slice below loaded again 9.26.
+// 2048x1536x768 3.16 ms, a wave per slice with its slice below loaded again 9.26.
 constexpr int kRowRun = 32;
 template <int NC>
 __global__ __launch_bounds__(64) void row_bits_kernel(const uint16_t *__restrict__ pm, int pitch,

@@ -3,7 +3,7 @@ run lengths and storage precisions) served by one device-resident job pool with 
 batching.
 
 The pool (``pfdtd_pool_*`` in libpfdtd.so) keeps every admitted job's fields resident in one HBM
-arena and advances all resident jobs together, one multi-job kernel launch per step and storage
+arena and advances all resident jobs together, one multi-job kernel launch per five steps and storage
 type, in hipGraph-captured bundles of steps. This module supplies the request side: it admits
 jobs first-come-first-served as they arrive, whenever the pool has arena space and a slot free
 (a job that does not fit waits at the head of the queue), keeps bundles flowing while jobs are
